@@ -18,8 +18,8 @@
 //                    with on-the-fly dequantisation.
 //   qdense_gemv (qdense_gemv.hip) — up to 64 rows of the reference's own layout, f32 x, zero
 //                    points, NF4: HBM-bound decode GEMV.
-//   qdense_refgemm_f32_mfma (qdense_refgemm.hip) — the same variants past the GEMV: f32 MFMA
-//                    GEMM with each K block of weights dequantised into LDS.
+//   qdense_refgemm_f32_mfma (qdense_refgemm.hip) — the same variants past the GEMV: f32
+//                    operands in three exact bf16 parts on the bf16 matrix cores (split_gemm.h).
 //   qdense_exact   — one output column per thread, k in order, each term rounded exactly as the
 //                    reference loop rounds it: bit-identical to the reference's f32 result.
 //                    Used for f32 activations and every shape/layout without a fast path.
@@ -357,8 +357,8 @@ static int exact_rows(const QDenseDesc& d) {
 
 // =============================================================================================
 // Reference layout and variants at prefill size (scale [K, ceil(N/B)] with BlockAxis = 1, f32 x,
-// zero points, NF4): the fused dequantise-and-contract kernel of qdense_refgemm.hip (f32 matrix
-// cores, the weights dequantised per K block into LDS).  Problems of at most 2^24 multiply-adds
+// zero points, NF4): the fused dequantise-and-contract kernel of qdense_refgemm.hip (f32 operands
+// in exact bf16 parts, the weights dequantised per K block into LDS).  Problems of at most 2^24 multiply-adds
 // keep the exact kernel (the reference's own BenchmarkQuantizedDense shapes, up to
 // 32 x 512 x 1024, stay bit-identical to it).
 // =============================================================================================

@@ -1,0 +1,483 @@
+// f32 contraction on the bf16 matrix cores, for products whose operands carry more than bf16's
+// 8 significant bits: every f32 operand is split exactly into three bf16 values (24 bits = 3 x 8),
+//   v = h + m + l,   h = bf16(v), m = bf16(v - h), l = v - h - m,
+// and the products of the parts are summed in one f32 accumulator by v_mfma_f32_16x16x32_bf16.
+// A bf16 x and an integer weight code (|code| <= 255) are one part and exact.  Split x against one
+// part takes 3 products per term, against three parts 6 (m*l, l*m and l*l, at most 2^-25 of the
+// term each, are left out).  The bf16 MFMAs have 16 times the rate of v_mfma_f32_16x16x4_f32, so 3
+// products have 5.3 times and 6 products 2.7 times the f32 matrix cores' peak.
+//
+// What bounds it: matrix-core issue, with the conversions (about 7 VALU instructions per x value
+// and part set) beside it.  Measured, f32 x [2048,4096] x Int4 [4096,11008], against the f32-MFMA
+// kernel this replaced (which ran at 0.63 of the f32 peak): scales per row and 128 columns (3
+// products) 1868 -> 607 us, 0.91 PFLOP/s of products; per row and 64 columns (6 products) 1868 ->
+// 1291 us; with 100 rows 363 -> 91 us (K in 2 slices).  The error against 64 bits fell from 1.1e-6
+// to 5.8e-7 (3 products) and 9.9e-7 (6): a step sums 32 terms where the f32 MFMA summed 4.
+//
+// Tiling: a workgroup of 4 waves owns a 128 x 128 output tile (2 x 2 waves of 64 x 64), K in
+// blocks of 32 (one MFMA step).  An operand's part lies in LDS as 128 rows of 32 bf16 (64 bytes,
+// four 16-byte chunks XOR-swizzled by (row >> 1) & 3: every 16-row operand read and every staging
+// write covers all banks).  Block kb + 1 is requested into registers before block kb is
+// multiplied, then split and written to the other LDS buffer (one buffer and a second barrier
+// where both operands have three parts).  Two workgroups share a CU, so one's conversions run
+// under the other's MFMAs.
+//
+// Column n of the tile lies in LDS row (n & 3) * 32 + (n >> 2): MFMA column set c of wave half wn
+// holds columns 64 wn + 4 cg + c, so a lane ends with four consecutive columns of each of its rows.
+//
+// Infinite operands (and finite ones that a product with the scale takes past f32) cannot be split
+// (the parts would meet as inf * 0): staging a value past kSplitMax sets a flag, and a flagged tile
+// is summed again by f32 FMAs over its K range before the epilogue.  NaN passes through the parts.
+#pragma once
+
+#include "device_common.h"
+#include "mxrt_internal.h"
+
+namespace mx {
+namespace sg {
+
+typedef __attribute__((__vector_size__(8 * sizeof(__bf16)))) __bf16 bf16x8_t;
+typedef __attribute__((__vector_size__(2 * sizeof(__bf16)))) __bf16 bf16x2_t;
+typedef __attribute__((__vector_size__(2 * sizeof(float)))) float f32x2_t;
+typedef float f32x4_t __attribute__((ext_vector_type(4)));
+typedef uint32_t u32x4_v __attribute__((ext_vector_type(4)));
+typedef uint32_t u32x2_v __attribute__((ext_vector_type(2)));
+
+constexpr int kBM = 128, kBN = 128, kBK = 32, kThreads = 256;
+constexpr int kPlane = kBM * kBK * 2;  // LDS bytes of one part of an operand
+constexpr size_t kCounterBytes = 64 * 1024;
+constexpr int kPartBytes = kBM * kBN * 4;  // one partial tile
+// Partial tiles of a split K: the most that the allocation-free entry point's static scratch holds
+// (the split is the same for both entry points, so their results are the same bits).
+constexpr int kMaxParts = (int)((MX_QDENSE_NOALLOC_SCRATCH_BYTES - kCounterBytes) / kPartBytes);
+
+// The largest magnitude that rounds to a finite bf16.
+#define MX_SPLIT_MAX __uint_as_float(0x7F7F7FFFu)
+
+struct Args {
+  const void* x;      // [M, K] f32 or bf16
+  const uint8_t* w;   // weight storage
+  const void* scale;
+  const void* zp;     // same layout as scale, or null
+  const void* bias;   // [N] or null
+  void* out;          // [M, N], x's dtype
+  int M, K, N;
+  int s_dt, zp_dt, b_dt, act, nf4;
+  int B;              // block size along the scale's blocked axis
+  int nb;             // scale row length of the reference layout: ceil(N / B)
+  int64_t bpr;        // GGML: bytes per weight row
+  int tiles_n, items, per_xcd;
+  int vec;            // out is aligned for stores of 4 values
+  int S, kpb;         // K slices per tile, 32-row blocks per slice
+  float* part;        // [tile][S] partial tiles (S > 1)
+  uint32_t* ctr;      // [tile] arrivals, zero between launches
+};
+
+__device__ __forceinline__ f32x4_t mfma(const u32x4_v& a, const u32x4_v& b, f32x4_t c) {
+  return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, a), __builtin_bit_cast(bf16x8_t, b), c, 0, 0, 0);
+}
+
+__device__ __forceinline__ uint32_t pack_bf16(float a, float b) {
+  const f32x2_t v = {a, b};
+  return __builtin_bit_cast(uint32_t, __builtin_convertvector(v, bf16x2_t));
+}
+
+// The three bf16 parts of a pair of values, one packed word per part.
+__device__ __forceinline__ void split2(float a, float b, uint32_t& h, uint32_t& m, uint32_t& l) {
+  h = pack_bf16(a, b);
+  const float ra = a - __uint_as_float(h << 16), rb = b - __uint_as_float(h & 0xFFFF0000u);
+  m = pack_bf16(ra, rb);
+  l = pack_bf16(ra - __uint_as_float(m << 16), rb - __uint_as_float(m & 0xFFFF0000u));
+}
+
+// LDS offset of 16-byte chunk `chunk` of LDS row p of a part.
+__device__ __forceinline__ uint32_t chunk_at(int p, int chunk) {
+  return (uint32_t)(p * 64 + ((chunk ^ ((p >> 1) & 3)) << 4));
+}
+
+// Element i of an f32 or bf16 array as f32.
+__device__ __forceinline__ float elem(const void* p, int64_t i, int dt) {
+  return dt == MX_DTYPE_BFLOAT16 ? bf16_to_f32(((const uint16_t*)p)[i]) : ((const float*)p)[i];
+}
+
+// P: the operand policy.  P::kXbf bf16 x (else f32); P::kPA, P::kPB parts of x and of the weights;
+// P::kRow each x value multiplied by its row's scale of the tile's column block before the split
+// (reference layout, one block per tile), zero points summed beside it; P::kCol one scale per
+// column, applied to the sums; P::Regs, load, stage: the weights' registers for a block, their
+// loads, and their parts into LDS; P::value: the f32 weight factor of one (k, n).
+template <class P>
+__global__ __launch_bounds__(kThreads, 2) void split_gemm_kernel(Args a) {
+  constexpr int PA = P::kPA, PB = P::kPB;
+  constexpr int kBufBytes = (PA + PB) * kPlane;
+  constexpr int NBUF = PA + PB <= 4 ? 2 : 1;
+  static_assert(!P::kRow || (PA == 3 && PB == 1), "row scales: split x, exact weight codes");
+  __shared__ __attribute__((aligned(16))) char sm[NBUF][kBufBytes];
+  __shared__ __attribute__((aligned(16))) float ring[P::kRow ? 2 : 1][2][kBK];  // scales, zero points of a block's rows
+  __shared__ float zrow[P::kRow ? kBM : 1];
+  __shared__ float table[16];
+  __shared__ int odd;  // a value that cannot be split was staged
+
+  // XCD-contiguous order, slices of a tile next to each other, tiles M-major.
+  const int item = (blockIdx.x & 7) * a.per_xcd + (blockIdx.x >> 3);
+  if ((int)(blockIdx.x >> 3) >= a.per_xcd || item >= a.items) return;
+  const int tile = item / a.S, slice = item - tile * a.S;
+  const int m0 = (tile / a.tiles_n) * kBM, n0 = (tile % a.tiles_n) * kBN;
+  const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
+  const int wm = wave >> 1, wn = wave & 1, cg = lane & 15, kq = lane >> 4;
+  const int M = a.M, K = a.K, N = a.N;
+  if (t < 16) table[t] = kNF4Table[t];
+  if (t == 16) odd = 0;
+
+  const int kb0 = slice * a.kpb, kb1 = min(kb0 + a.kpb, (K + kBK - 1) / kBK);
+
+  // ---- x: thread t stages k chunk t & 3 (8 values) of rows t / 4 and t / 4 + 64.  Rows past M
+  // read row M - 1 (their outputs are not stored).
+  const int xr = t >> 2, xc = t & 3;
+  const char* xp[2];
+#pragma unroll
+  for (int i = 0; i < 2; ++i) xp[i] = (const char*)a.x + (int64_t)min(m0 + xr + 64 * i, M - 1) * K * (P::kXbf ? 2 : 4);
+  struct XRegs {
+    u32x4_v v[2][P::kXbf ? 1 : 2];
+  };
+  auto load_x = [&](int kb, XRegs& R) __attribute__((always_inline)) {
+    const int k = kb * kBK + 8 * xc;
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      if constexpr (P::kXbf) {
+        R.v[i][0] = *(const u32x4_v*)(xp[i] + (int64_t)min(k, K - 8) * 2);
+      } else {
+        R.v[i][0] = *(const u32x4_v*)(xp[i] + (int64_t)min(k, K - 4) * 4);
+        R.v[i][1] = *(const u32x4_v*)(xp[i] + (int64_t)min(k + 4, K - 4) * 4);
+      }
+    }
+  };
+  float zacc[2] = {0.f, 0.f};
+  // Values of k past K are zero (K % 8 == 0 for bf16 x, K % 4 == 0 for f32).
+  auto stage_x = [&](int kb, const XRegs& R, char* As) __attribute__((always_inline)) {
+    const int k = kb * kBK + 8 * xc;
+    const bool lo = k < K, hi = P::kXbf ? lo : k + 4 < K;
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      char* dst = As + chunk_at(xr + 64 * i, xc);
+      if constexpr (PA == 1) {
+        u32x4_v v = R.v[i][0];
+        if (!lo) v = u32x4_v{0u, 0u, 0u, 0u};
+        *(u32x4_v*)dst = v;
+      } else {
+        float v[8];
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+          if constexpr (P::kXbf)
+            v[e] = __uint_as_float(e & 1 ? R.v[i][0][e >> 1] & 0xFFFF0000u : R.v[i][0][e >> 1] << 16);
+          else
+            v[e] = __uint_as_float(R.v[i][e >> 2][e & 3]);
+          v[e] = (e < 4 ? lo : hi) ? v[e] : 0.0f;
+        }
+        if constexpr (P::kRow) {
+          const float* s = &ring[kb & 1][0][8 * xc];
+          if (a.zp) {
+            const float* z = &ring[kb & 1][1][8 * xc];
+#pragma unroll
+            for (int e = 0; e < 8; ++e) zacc[i] = __builtin_fmaf(v[e], z[e], zacc[i]);
+          }
+#pragma unroll
+          for (int e = 0; e < 8; ++e) v[e] = mul_rn(v[e], s[e]);
+        }
+        float big = fabsf(v[0]);
+#pragma unroll
+        for (int e = 1; e < 8; ++e) big = fmaxf(big, fabsf(v[e]));
+        if (big > MX_SPLIT_MAX) odd = 1;
+        u32x4_v h, m, l;
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          uint32_t hh, mm, ll;
+          split2(v[2 * q], v[2 * q + 1], hh, mm, ll);
+          h[q] = hh;
+          m[q] = mm;
+          l[q] = ll;
+        }
+        *(u32x4_v*)dst = h;
+        *(u32x4_v*)(dst + kPlane) = m;
+        *(u32x4_v*)(dst + 2 * kPlane) = l;
+      }
+    }
+  };
+  // Row scales and zero points of block kb, one row per thread of the first 32, into their slot
+  // two blocks ahead of their use.
+  float rs = 0.f, rz = 0.f;
+  auto load_row_scale = [&](int kb) __attribute__((always_inline)) {
+    if constexpr (P::kRow) {
+      if (t < kBK) {
+        const int64_t i = (int64_t)min(kb * kBK + t, K - 1) * a.nb + n0 / a.B;
+        rs = elem(a.scale, i, a.s_dt);
+        if (a.zp) rz = elem(a.zp, i, a.zp_dt);
+      }
+    }
+  };
+  auto store_row_scale = [&](int kb) __attribute__((always_inline)) {
+    if constexpr (P::kRow) {
+      if (t < kBK) {
+        ring[kb & 1][0][t] = rs;
+        ring[kb & 1][1][t] = rz;
+      }
+    }
+  };
+
+  f32x4_t acc[4][4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i)
+#pragma unroll
+    for (int c = 0; c < 4; ++c) acc[i][c] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+  // One block: small products first.
+  auto compute = [&](const char* buf) __attribute__((always_inline)) {
+    const char* As = buf;
+    const char* Bs = buf + PA * kPlane;
+    u32x4_v B[PB][4];
+#pragma unroll
+    for (int p = 0; p < PB; ++p)
+#pragma unroll
+      for (int c = 0; c < 4; ++c) B[p][c] = *(const u32x4_v*)(Bs + p * kPlane + chunk_at(c * 32 + 16 * wn + cg, kq));
+#pragma unroll
+    for (int rb = 0; rb < 4; ++rb) {
+      u32x4_v A[PA];
+#pragma unroll
+      for (int p = 0; p < PA; ++p) A[p] = *(const u32x4_v*)(As + p * kPlane + chunk_at(64 * wm + 16 * rb + cg, kq));
+#pragma unroll
+      for (int order = PA + PB - 2; order >= 0; --order) {
+        if (order > 2) continue;
+#pragma unroll
+        for (int pa = 0; pa < PA; ++pa) {
+          const int pb = order - pa;
+          if (pb < 0 || pb >= PB) continue;
+#pragma unroll
+          for (int c = 0; c < 4; ++c) acc[rb][c] = mfma(A[pa], B[pb][c], acc[rb][c]);
+        }
+      }
+    }
+  };
+
+  P src(a, t, n0);
+  XRegs X;
+  typename P::Regs W;
+  load_row_scale(kb0);
+  load_x(kb0, X);
+  src.load(a, kb0, W);
+  store_row_scale(kb0);
+  load_row_scale(kb0 + 1);
+  __syncthreads();  // the table, the flag and block kb0's row scales are written
+  if constexpr (NBUF == 2) {
+    store_row_scale(kb0 + 1);
+    stage_x(kb0, X, sm[0]);
+    src.stage(a, kb0, W, table, sm[0] + PA * kPlane, odd);
+    __syncthreads();
+#pragma unroll 1
+    for (int kb = kb0; kb < kb1; ++kb) {
+      const int cur = (kb - kb0) & 1;
+      const bool more = kb + 1 < kb1;
+      if (more) {
+        load_x(kb + 1, X);
+        src.load(a, kb + 1, W);
+        load_row_scale(kb + 2);
+      }
+      compute(sm[cur]);
+      if (more) {
+        char* nxt = sm[NBUF == 2 ? cur ^ 1 : 0];
+        stage_x(kb + 1, X, nxt);
+        src.stage(a, kb + 1, W, table, nxt + PA * kPlane, odd);
+        store_row_scale(kb + 2);
+      }
+      __syncthreads();
+    }
+  } else {
+#pragma unroll 1
+    for (int kb = kb0; kb < kb1; ++kb) {
+      stage_x(kb, X, sm[0]);
+      src.stage(a, kb, W, table, sm[0] + PA * kPlane, odd);
+      __syncthreads();
+      if (kb + 1 < kb1) {
+        load_x(kb + 1, X);
+        src.load(a, kb + 1, W);
+      }
+      compute(sm[0]);
+      __syncthreads();
+    }
+  }
+
+  if constexpr (P::kRow) {
+    if (a.zp) {  // x . zp of each row, added to all of its columns
+#pragma unroll
+      for (int i = 0; i < 2; ++i) {
+        float z = zacc[i];
+        z += __shfl_xor(z, 1);
+        z += __shfl_xor(z, 2);
+        if (xc == 0) zrow[xr + 64 * i] = z;
+      }
+      __syncthreads();
+#pragma unroll
+      for (int rb = 0; rb < 4; ++rb)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const float z = zrow[64 * wm + 16 * rb + 4 * kq + r];
+#pragma unroll
+          for (int c = 0; c < 4; ++c) acc[rb][c][r] += z;
+        }
+    }
+  }
+  const int ncol = n0 + 64 * wn + 4 * cg;
+  if (odd) {  // uniform over the workgroup
+#pragma unroll
+    for (int rb = 0; rb < 4; ++rb)
+#pragma unroll
+      for (int c = 0; c < 4; ++c) acc[rb][c] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+#pragma unroll 1
+    for (int k = kb0 * kBK; k < min(K, kb1 * kBK); ++k) {
+      float wv[4];
+#pragma unroll
+      for (int c = 0; c < 4; ++c) wv[c] = src.value(a, k, min(ncol + c, N - 1), table);
+#pragma unroll
+      for (int rb = 0; rb < 4; ++rb)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const int m = min(m0 + 64 * wm + 16 * rb + 4 * kq + r, M - 1);
+          const float xv = elem(a.x, (int64_t)m * K + k, P::kXbf ? MX_DTYPE_BFLOAT16 : MX_DTYPE_FLOAT32);
+#pragma unroll
+          for (int c = 0; c < 4; ++c) acc[rb][c][r] = __builtin_fmaf(xv, wv[c], acc[rb][c][r]);
+        }
+    }
+  }
+
+  if (a.S > 1) {
+    // Every slice stores its sums; the last to arrive at the tile adds them in slice order and goes
+    // on to the epilogue.  Agent-scope coherent accesses (sc1): the slices may run on other XCDs.
+    const __amdgpu_buffer_rsrc_t prs =
+        __builtin_amdgcn_make_buffer_rsrc(a.part + (size_t)tile * a.S * kBM * kBN, (short)0, a.S * kPartBytes, 0x00020000);
+    constexpr int kSc1 = 16;
+#pragma unroll
+    for (int rb = 0; rb < 4; ++rb)
+#pragma unroll
+      for (int c = 0; c < 4; ++c)
+        __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4_v, acc[rb][c]), prs,
+                                              (unsigned)(slice * kPartBytes + ((4 * rb + c) * kThreads + t) * 16), 0, kSc1);
+    __builtin_amdgcn_s_waitcnt(0);
+    __syncthreads();
+    if (t == 0) {
+      const uint32_t prev = __hip_atomic_fetch_add(&a.ctr[tile], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      if (prev + 1u == (uint32_t)a.S) __hip_atomic_store(&a.ctr[tile], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      odd = prev + 1u == (uint32_t)a.S;
+    }
+    __syncthreads();
+    if (!odd) return;
+#pragma unroll
+    for (int rb = 0; rb < 4; ++rb)
+#pragma unroll
+      for (int c = 0; c < 4; ++c) acc[rb][c] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+#pragma unroll 1
+    for (int s = 0; s < a.S; ++s) {
+#pragma unroll
+      for (int rb = 0; rb < 4; ++rb)
+#pragma unroll
+        for (int c = 0; c < 4; ++c)
+          acc[rb][c] += __builtin_bit_cast(f32x4_t, __builtin_amdgcn_raw_buffer_load_b128(
+                                                        prs, (unsigned)(s * kPartBytes + ((4 * rb + c) * kThreads + t) * 16), 0, kSc1));
+    }
+  }
+
+  // Epilogue: column scales, bias (added after the sum), the reference activation, x's dtype.  The
+  // activation's code is there once: each half of the tile goes through LDS (free after the loop's
+  // last barrier) to a rolled loop over four consecutive columns of a row.
+  float cs[4] = {1.f, 1.f, 1.f, 1.f}, bi[4] = {0.f, 0.f, 0.f, 0.f};
+  if (ncol < N) {
+#pragma unroll
+    for (int c = 0; c < 4; ++c) {
+      if constexpr (P::kCol) cs[c] = elem(a.scale, ncol + c, a.s_dt);
+      if (a.bias) bi[c] = elem(a.bias, ncol + c, a.b_dt);
+    }
+  }
+  auto store4 = [&](int m, int n, const float (&y)[4]) __attribute__((always_inline)) {
+    const int64_t o = (int64_t)m * N + n;
+    if (!a.vec) {
+#pragma unroll
+      for (int c = 0; c < 4; ++c) store_f(a.out, o + c, P::kXbf ? MX_DTYPE_BFLOAT16 : MX_DTYPE_FLOAT32, y[c]);
+    } else if constexpr (P::kXbf) {
+      *(u32x2_v*)((uint16_t*)a.out + o) = u32x2_v{(uint32_t)f32_to_bf16(y[0]) | (uint32_t)f32_to_bf16(y[1]) << 16,
+                                                  (uint32_t)f32_to_bf16(y[2]) | (uint32_t)f32_to_bf16(y[3]) << 16};
+    } else {
+      *(f32x4_t*)((float*)a.out + o) = f32x4_t{y[0], y[1], y[2], y[3]};
+    }
+  };
+  auto finish = [&](float v, int c) __attribute__((always_inline)) {
+    if constexpr (P::kCol) v = mul_rn(v, cs[c]);
+    return a.bias ? add_rn(bi[c], v) : v;
+  };
+  if (a.act == MX_ACT_NONE) {
+    if (ncol >= N) return;
+#pragma unroll
+    for (int rb = 0; rb < 4; ++rb)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int m = m0 + 64 * wm + 16 * rb + 4 * kq + r;
+        float y[4];
+#pragma unroll
+        for (int c = 0; c < 4; ++c) y[c] = finish(acc[rb][c][r], c);
+        if (m < M) store4(m, ncol, y);
+      }
+    return;
+  }
+  constexpr int kCS = kBN * 4;  // LDS bytes per row of a half tile
+  static_assert(64 * kCS <= NBUF * kBufBytes, "half a tile fits the LDS buffers");
+  char* Cs = sm[0];
+#pragma unroll 1
+  for (int half = 0; half < 2; ++half) {
+    __syncthreads();
+    if (wm == half) {
+#pragma unroll
+      for (int rb = 0; rb < 4; ++rb)
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+          *(f32x4_t*)(Cs + (16 * rb + 4 * kq + r) * kCS + (64 * wn + 4 * cg) * 4) =
+              f32x4_t{finish(acc[rb][0][r], 0), finish(acc[rb][1][r], 1), finish(acc[rb][2][r], 2), finish(acc[rb][3][r], 3)};
+    }
+    __syncthreads();
+#pragma unroll 1
+    for (int idx = t; idx < 64 * (kBN / 4); idx += kThreads) {
+      const int row = idx >> 5, col = (idx & 31) * 4;
+      const int m = m0 + 64 * half + row, n = n0 + col;
+      if (m >= M || n >= N) continue;
+      float* v = (float*)(Cs + row * kCS + col * 4);
+#pragma unroll 1
+      for (int c = 0; c < 4; ++c) v[c] = act_ref(v[c], a.act);
+      const float y[4] = {v[0], v[1], v[2], v[3]};
+      store4(m, n, y);
+    }
+  }
+}
+
+// Tiles, K slices and grid of a problem.  Tiles that leave CUs idle are split along K: as many
+// slices of at least eight blocks as fill the 256 CUs (planned whatever the device reports, so the
+// summation order depends on the shape alone) within kMaxParts partial tiles.
+inline int plan(mx_backend* b, Args& a, int64_t M, int* grid) {
+  const int64_t tiles_n = (a.N + kBN - 1) / kBN, tiles = ((M + kBM - 1) / kBM) * tiles_n;
+  if (tiles >= (int64_t)1 << 28) return set_error(MX_ERR_INVALID, "FusedQuantizedDense: M=%lld too large", (long long)M);
+  const int blocks = (a.K + kBK - 1) / kBK;
+  int S = 1;
+  if (tiles <= kMaxParts / 2) S = (int)std::max<int64_t>(1, std::min<int64_t>(kMaxParts / tiles, blocks / 8));
+  a.kpb = (blocks + S - 1) / S;
+  a.S = (blocks + a.kpb - 1) / a.kpb;
+  a.tiles_n = (int)tiles_n;
+  a.items = (int)tiles * a.S;
+  a.per_xcd = (a.items + 7) / 8;
+  *grid = 8 * a.per_xcd;
+  a.vec = (uintptr_t)a.out % 16 == 0;
+  a.part = nullptr;
+  a.ctr = nullptr;
+  if (a.S > 1) {
+    void* scratch = nullptr;
+    MX_TRY(ensure_scratch(b, kCounterBytes + (size_t)a.items * kPartBytes, &scratch));
+    a.ctr = (uint32_t*)scratch;
+    a.part = (float*)((char*)scratch + kCounterBytes);
+  }
+  return MX_OK;
+}
+
+}  // namespace sg
+}  // namespace mx

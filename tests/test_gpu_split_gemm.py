@@ -1,0 +1,117 @@
+"""f32 contraction on the bf16 matrix cores (split_gemm.h): f32 operands in three exact bf16 parts.
+
+The parts reproduce every f32 operand exactly and at most three products of parts (2^-25 of a term
+each) are left out, so the outputs keep the f32 accumulation bound the other paths are held to:
+2^-22 |y| + 1e-5 * sum_k |term_k| of the f64 value (bf16 outputs: one bf16 ulp, 2^-8 |y|, for the
+relative part).  Shapes sit on the edges: rows, columns and k past the last whole tile, K of one
+slice and of many, operands at the ends of f32's range."""
+import dataclasses
+
+import numpy as np
+import pytest
+
+import compute_amd as ca
+from oracle import oracle as O
+from tests.qd_helpers import QDenseRun
+
+pytestmark = pytest.mark.gpu
+
+F32, BF16 = O.DT_FLOAT32, O.DT_BFLOAT16
+
+
+def check(p, y):
+    truth, scale = O.qdense_f64(p), O.qdense_f64(p, absolute=True)
+    got = (O.bf16_to_f32(y) if p.x_dtype == BF16 else y).astype(np.float64)
+    rel = 2.0 ** -8 if p.x_dtype == BF16 else 2.0 ** -22
+    bad = np.abs(got - truth) > rel * np.abs(truth) + 1e-5 * scale
+    assert not bad.any(), f"{bad.sum()} outputs outside the bound; worst at {np.argwhere(bad)[0]}"
+
+
+# (x, axis, B, zero point, NF4): the row form (B a multiple of 128, or one block), the column form
+# (one scale per column) and the weight form (everything else).
+FORMS = [(F32, 1, 128, False, False), (F32, 1, 128, True, False), (BF16, 1, 4096, True, False), (F32, 0, None, False, False),
+         (F32, 0, 96, True, False), (BF16, 0, 96, False, False), (F32, 1, 4, True, False), (BF16, 1, 7, True, False),
+         (F32, 1, 7, False, False), (F32, 1, 128, False, True)]
+
+
+@pytest.mark.parametrize("form", FORMS)
+@pytest.mark.parametrize("w_dtype", [O.DT_INT8, O.DT_UINT4])
+@pytest.mark.parametrize("M,K,N", [(131, 1048, 144), (257, 2088, 400)])
+def test_forms_at_ragged_edges(backend, form, w_dtype, M, K, N):
+    x_dtype, axis, B, zp, nf4 = form
+    p = O.make_problem(M, K, N, w_dtype=w_dtype, x_dtype=x_dtype, scale_dtype=x_dtype, block_axis=axis,
+                       block_size=K if B is None else B, zp=zp, scheme=O.QUANT_NF4 if nf4 else O.QUANT_LINEAR, bias=True,
+                       seed=M + K + w_dtype)
+    r = QDenseRun(backend, p)
+    assert r.plan() == "qdense_refgemm_f32_mfma"
+    y = r.run()
+    check(p, y)
+    assert np.array_equal(y, r.run()), "not deterministic"
+
+
+@pytest.mark.parametrize("form", [FORMS[0], FORMS[6]])
+@pytest.mark.parametrize("M,K,N", [(65, 16388, 16), (129, 8196, 1040), (640, 1028, 2064)])
+def test_k_slices_with_and_without_allocation(backend, form, M, K, N):
+    """One tile in many K slices, tiles in a few, and (85 tiles) none; the allocation-free entry
+    point takes the same slices, so its result is the same bits."""
+    x_dtype, axis, B, zp, _ = form
+    p = O.make_problem(M, K, N, w_dtype=O.DT_INT4, x_dtype=x_dtype, scale_dtype=F32, block_axis=axis, block_size=B, zp=zp,
+                       bias=False, seed=K)
+    r = QDenseRun(backend, p)
+    assert r.plan() == "qdense_refgemm_f32_mfma"
+    y = r.run()
+    check(p, y)
+    out = backend.BufferFromFlatData(0, np.zeros(M * N, np.float32), ca.Shape(ca.Float32, M, N))
+    backend.QDenseNoAlloc(r.args(out))
+    assert np.array_equal(out.ToFlatData().reshape(M, N).view(np.uint32), y.view(np.uint32))
+
+
+@pytest.mark.parametrize("B", [128, 32])
+@pytest.mark.parametrize("magnitude", [1e-36, 1e30])
+def test_operands_at_the_ends_of_the_range(backend, B, magnitude):
+    """x near f32's smallest normals (its lower parts are subnormal) and large."""
+    p = O.make_problem(96, 1024, 256, w_dtype=O.DT_INT4, x_dtype=F32, scale_dtype=F32, block_axis=1, block_size=B, bias=False,
+                       scale_range=(0.5, 2.0), seed=3)
+    p = dataclasses.replace(p, x=(p.x * np.float32(magnitude)).astype(np.float32))
+    check(p, QDenseRun(backend, p).run())
+
+
+@pytest.mark.parametrize("B,K", [(128, 1024), (32, 1024), (128, 16384)])
+def test_infinite_and_nan_operands(backend, B, K):
+    """A tile that holds an operand with no split (infinite, or past the largest bf16) is summed by
+    f32 FMAs: infinities keep their sign, NaN stays in its row or column, the rest is as close as
+    ever.  Codes are positive, so that no infinities of both signs meet."""
+    p = O.make_problem(260, K, 256, w_dtype=O.DT_UINT8, x_dtype=F32, scale_dtype=F32, block_axis=1, block_size=B, bias=True,
+                       scale_range=(0.001, 0.0039), seed=4)  # codes * scales < 1: no finite x makes an infinite term
+    w = np.maximum(p.w, 1)
+    x, s = p.x.copy(), p.scale.copy()
+    x[3, 17], x[140, 5], x[141, 9] = np.inf, -np.inf, np.nan
+    x[200, 1023] = 3.4e38  # rounds past bf16's largest value
+    s[33, 0] = np.inf      # the first block's columns, every row
+    x[:, 33] = np.abs(x[:, 33]) + 0.5
+    p = dataclasses.replace(p, w=w, x=x, scale=s)
+    y = QDenseRun(backend, p).run().astype(np.float64)
+    with np.errstate(invalid="ignore", over="ignore"):
+        truth, scale = O.qdense_f64(p), O.qdense_f64(p, absolute=True)
+    assert np.array_equal(np.isnan(y), np.isnan(truth))
+    inf = np.isinf(truth)
+    assert np.array_equal(y[inf], truth[inf])
+    fin = np.isfinite(truth)
+    assert fin.any() and inf.any()
+    assert np.all(np.abs(y[fin] - truth[fin]) <= 2.0 ** -22 * np.abs(truth[fin]) + 1e-5 * scale[fin])
+
+
+@pytest.mark.parametrize("x_dtype,act", [(F32, O.ACT_NONE), (BF16, O.ACT_RELU)])
+def test_output_aligned_to_its_elements_only(backend, x_dtype, act):
+    """An output array that starts one element past a 16-byte boundary."""
+    p = O.make_problem(70, 1024, 272, w_dtype=O.DT_INT8, x_dtype=x_dtype, scale_dtype=F32, block_axis=1, block_size=64, bias=True,
+                       act=act, seed=9)
+    r = QDenseRun(backend, p)
+    want = r.run()
+    dt, st = (ca.Float32, np.float32) if x_dtype == F32 else (ca.BFloat16, np.uint16)
+    out = backend.BufferFromFlatData(0, np.zeros(p.M * p.N + 1, st), ca.Shape(dt, p.M * p.N + 1))
+    a = r.args(out)
+    a.out = out.DevicePtr() + np.dtype(st).itemsize
+    backend.QDense(a)
+    got = out.ToFlatData()
+    assert got[0] == 0 and np.array_equal(got[1:].reshape(p.M, p.N), want)
