@@ -20,22 +20,20 @@
 //                      once, then the wave adds its lanes in a fixed tree.  f32 FMAs on the VALU:
 //                      x is f32 by contract, and bf16 matrix-core operands would not keep the
 //                      f32 accumulation bound.
-//   ggml_dequant_f32 — past 20 rows: a workgroup per row dequantises it (staged in LDS) to f32,
-//                      eight values per thread, for the f32 DotGeneral; ggml_epilogue then adds
-//                      the bias and applies the activation in place.
+//   split_gemm<GgmlSource> — past 16 rows: each K block of rows dequantised as the reference forms
+//                      each value and contracted in exact bf16 parts (split_gemm.h), bias and
+//                      activation in its epilogue.
 //   ggml_embed       — one thread per output value (the reference's arithmetic, bit-identical);
 //                      indices of any integer dtype, bad indices reported after the launch.
-// Plans: up to 4 rows the GEMV; problems of at most 2^24 multiply-adds the exact kernel; up to 20
-// rows the GEMV once per group of four rows; past that the rows dequantised once to f32 [N, K]
-// (each value exactly as the reference forms it), contracted on the f32 matrix cores (DotGeneral
-// with a transposed right-hand side) and the bias and activation applied in place, within the f32
-// accumulation bound of the reference's sum.  The exact backend option selects the exact kernel;
-// the allocation-free entry point never takes the dequantised path.
+// Plans: up to 4 rows the GEMV; problems of at most 2^24 multiply-adds the exact kernel; up to 16
+// rows the GEMV once per group of four rows; past that the split contraction, within the f32
+// accumulation bound of the reference's sum.  The exact backend option selects the exact kernel.
 #include <algorithm>
 #include <cstring>
 
 #include "device_common.h"
 #include "mxrt_internal.h"
+#include "split_gemm.h"
 
 namespace mx {
 
@@ -453,88 +451,116 @@ static void launch_gemv_t(const GgmlDesc& d, int grid, size_t lds, int ch, int w
 }
 
 
-// Prefill: the rows dequantised to f32 [N, K], each value as the reference forms it (the
-// arithmetic of ggml_value, the type fixed at compile time).  A workgroup per row at a
-// time: the row's bytes staged in LDS with coalesced 2-byte loads (every block size is even),
-// then eight consecutive values (one block's) per thread decoded from LDS and written as two
-// 16-byte stores.  Rows of up to kDqRowBytes bytes (dynamic LDS of the row's size).
-constexpr int kDqRowBytes = 64 * 1024;
+// Prefill: split_gemm.h's contraction over weights dequantised per K block as the reference forms
+// each value (f32 in three exact bf16 parts, 6 products per term).  Thread t takes NC = 8 / NW
+// 8-value chunks of one row of a block of 32 values; rows' blocks are 2-byte aligned.
+template <int T, int NW>
+struct GgmlSource {
+  static constexpr bool kXbf = false, kRow = false, kCol = false, kZp = false;
+  static constexpr int kPA = 3, kPB = 3;
+  static constexpr int vpb = ggml_vpb(T), bpb = ggml_bpb(T), NC = 8 / NW;
+  static constexpr bool kNib32 = T == MX_GGML_Q4_0 || T == MX_GGML_IQ4_NL;
+  struct Regs {
+    uint32_t q[2 * NC];                           // code bytes (4-bit formats: both nibbles)
+    uint32_t h[T == MX_GGML_Q4_K ? 4 : 2 * NC];   // Q4_K: the block's header (d, dmin, scales); Q6_K: upper bits
+    uint32_t d;                                   // block scale bits; Q6_K: and the run's int8 scale above them
+  };
+  int p, chunk;
+  const uint8_t* row;
 
-// Values i .. i+7 of a block (i a multiple of 8), as ggml_value forms each one, with what the
-// eight share (the block scale, a K-quant sub-block's scale and minimum) formed once.
-template <int T>
-__device__ __forceinline__ void ggml_values8(const uint8_t* blk, int i, float* v) {
-  if constexpr (T == MX_GGML_Q8_0) {
-    const float d = f16_at(blk);
-#pragma unroll
-    for (int e = 0; e < 8; ++e) v[e] = mul_rn(d, (float)(int8_t)blk[2 + i + e]);
-  } else if constexpr (T == MX_GGML_Q4_0 || T == MX_GGML_IQ4_NL) {
-    const float d = f16_at(blk);
-    const uint8_t* q = blk + 2 + (i & 15);
-#pragma unroll
-    for (int e = 0; e < 8; ++e) {
-      const uint32_t nib = i < 16 ? q[e] & 15u : (uint32_t)q[e] >> 4;
-      v[e] = T == MX_GGML_Q4_0 ? mul_rn(d, (float)((int)nib - 8)) : mul_rn(d, kIQ4NL[nib]);
-    }
-  } else if constexpr (T == MX_GGML_Q4_K) {
-    const int chunk = i >> 6, w = i & 63, j = 2 * chunk + (w >> 5);
-    uint32_t sc, m;
-    scale_min_k4(j, blk + 4, &sc, &m);
-    const float d1 = mul_rn(f16_at(blk), (float)sc), min1 = mul_rn(f16_at(blk + 2), (float)m);
-    const uint8_t* q = blk + 16 + 32 * chunk + (w & 31);
-#pragma unroll
-    for (int e = 0; e < 8; ++e) v[e] = add_rn(mul_rn(d1, (float)(w < 32 ? q[e] & 15u : (uint32_t)q[e] >> 4)), -min1);
-  } else {  // MX_GGML_Q6_K
-    const int h = i >> 7, r = i & 127, j = r >> 5, l = r & 31;
-    const float ds = mul_rn(f16_at(blk + 208), (float)(int)(int8_t)blk[192 + 8 * h + 2 * j + (l >> 4)]);
-    const uint8_t* ql = blk + 64 * h + 32 * (j & 1) + l;
-    const uint8_t* qh = blk + 128 + 32 * h + l;
-#pragma unroll
-    for (int e = 0; e < 8; ++e) {
-      const uint32_t nib = (j >> 1) ? (uint32_t)ql[e] >> 4 : ql[e] & 15u;
-      const uint32_t hi2 = ((uint32_t)qh[e] >> (2 * j)) & 3u;
-      v[e] = mul_rn(ds, (float)((int)(nib | (hi2 << 4)) - 32));
+  static __device__ __forceinline__ float table_value(int i) { return kIQ4NL[i]; }
+  // N words at 2-byte alignment.
+  template <int N>
+  static __device__ __forceinline__ void words(const uint8_t* a, uint32_t* v) {
+    __builtin_memcpy(v, __builtin_assume_aligned(a, 2), 4 * N);
+  }
+  static __device__ __forceinline__ uint32_t load2(const uint8_t* a) { return *(const uint16_t*)a; }
+
+  __device__ __forceinline__ GgmlSource(const sg::Args& a, int t, int n0) {
+    p = NC == 2 ? t >> 1 : t >> 2;
+    chunk = NC == 2 ? 2 * (t & 1) : t & 3;
+    row = a.w + (int64_t)min(n0 + sg::col_of_row(p), a.N - 1) * a.bpr;
+  }
+  __device__ __forceinline__ void load(const sg::Args& a, sg::Block b, Regs& R) const {
+    const int k = b.k;  // a multiple of 32
+    const uint8_t* blk = row + (int64_t)(k / vpb) * bpb;
+    const int s = (k % vpb) >> 5;  // 32-value run of the block
+    if constexpr (T == MX_GGML_Q8_0) {
+      R.d = load2(blk);
+      words<2 * NC>(blk + 2 + 8 * chunk, R.q);
+    } else if constexpr (kNib32) {
+      R.d = load2(blk);
+      words<2 * NC>(blk + 2 + 8 * (chunk & 1), R.q);
+    } else if constexpr (T == MX_GGML_Q4_K) {
+      words<4>(blk, R.h);
+      words<2 * NC>(blk + 16 + 32 * (s >> 1) + 8 * chunk, R.q);
+    } else {
+      const int h = s >> 2, j = s & 3;
+      words<2 * NC>(blk + 64 * h + 32 * (j & 1) + 8 * chunk, R.q);
+      words<2 * NC>(blk + 128 + 32 * h + 8 * chunk, R.h);
+      R.d = load2(blk + 208) | (uint32_t)blk[192 + 8 * h + 2 * j + (chunk >> 1)] << 24;
     }
   }
-}
-
-template <int T>
-__global__ __launch_bounds__(256) void ggml_dequant_f32_kernel(GgmlDesc d, float* __restrict__ wt) {
-  constexpr int vpb = T == MX_GGML_Q4_K || T == MX_GGML_Q6_K ? 256 : 32;
-  constexpr int vsh = vpb == 256 ? 8 : 5;
-  extern __shared__ __align__(16) uint16_t rs[];
-  const uint8_t* rb = reinterpret_cast<const uint8_t*>(rs);
-  const int bpb = ggml_bpb(T);
-  const int K8 = (int)(d.K / 8), H = (int)(d.bpr / 2);
-  for (int64_t n = blockIdx.x; n < d.N; n += gridDim.x) {
-    const uint16_t* row = reinterpret_cast<const uint16_t*>(d.w + n * d.bpr);
-    for (int h = threadIdx.x; h < H; h += blockDim.x) rs[h] = row[h];
-    __syncthreads();
-    float4* out = reinterpret_cast<float4*>(wt + n * d.K);
-    for (int j = threadIdx.x; j < K8; j += blockDim.x) {
-      const int k = 8 * j;
-      const uint8_t* blk = rb + (k >> vsh) * bpb;
-      const int i = k & (vpb - 1);
-      float v[8];
-      ggml_values8<T>(blk, i, v);
-      out[2 * j] = make_float4(v[0], v[1], v[2], v[3]);
-      out[2 * j + 1] = make_float4(v[4], v[5], v[6], v[7]);
+  // Block scales are used as the reference uses them: every product and difference of a value
+  // rounded to f32 (most are exact).
+  template <class TailT>
+  __device__ __forceinline__ void stage(const sg::Args& a, sg::Block b, const Regs& R, const float* table, char* Bs, float& big, TailT) const {
+    const int s = (b.k % vpb) >> 5;
+    float d, m = 0.0f;
+    if constexpr (T == MX_GGML_Q4_K) {
+      // Scale and minimum s of the 12 packed bytes h[1..3] (scale_min_k4 on registers).
+      const int at = 8 * (s & 3);
+      const uint32_t s0 = R.h[1] >> at & 255u, s1 = R.h[2] >> at & 255u, s2 = R.h[3] >> at & 255u;
+      const uint32_t sc = s < 4 ? s0 & 63u : (s2 & 15u) | (s0 >> 6) << 4;
+      const uint32_t mn = s < 4 ? s1 & 63u : (s2 >> 4) | (s1 >> 6) << 4;
+      d = mul_rn(f16_to_f32((uint16_t)R.h[0]), (float)sc);
+      m = mul_rn(f16_to_f32((uint16_t)(R.h[0] >> 16)), (float)mn);
+    } else if constexpr (T == MX_GGML_Q6_K) {
+      d = mul_rn(f16_to_f32((uint16_t)R.d), (float)((int32_t)R.d >> 24));
+    } else {
+      d = f16_to_f32((uint16_t)R.d);
     }
-    __syncthreads();
+    // The thread's codes as bytes (4-bit formats: which nibble holds them).
+    const int sh4 = 4 * (kNib32 ? chunk >> 1 : T == MX_GGML_Q4_K ? s & 1 : (s & 3) >> 1);
+#pragma unroll
+    for (int c = 0; c < NC; ++c) {
+      sg::u32x4_v h, mid, l;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        uint32_t w = R.q[2 * c + (i >> 1)];
+        if constexpr (T != MX_GGML_Q8_0) w = (w >> sh4) & 0x0F0F0F0Fu;
+        if constexpr (T == MX_GGML_Q6_K) w |= ((R.h[2 * c + (i >> 1)] >> (2 * (s & 3))) & 0x03030303u) << 4;
+        float v[2];
+#pragma unroll
+        for (int e = 0; e < 2; ++e) {
+          const uint32_t sh = 8 * (2 * (i & 1) + e);
+          float f;
+          if constexpr (T == MX_GGML_Q8_0)
+            f = (float)(int8_t)(w >> sh);
+          else if constexpr (T == MX_GGML_IQ4_NL)
+            f = table[(w >> sh) & 15u];
+          else
+            f = (float)(uint8_t)(w >> sh) - (T == MX_GGML_Q4_0 ? 8.0f : T == MX_GGML_Q6_K ? 32.0f : 0.0f);
+          v[e] = mul_rn(d, f);
+          if constexpr (T == MX_GGML_Q4_K) v[e] = add_rn(v[e], -m);
+        }
+        big = fmaxf(fmaxf(fabsf(v[0]), fabsf(v[1])), big);  // past the limit only for an infinite block scale
+        uint32_t hh, mm, ll;
+        sg::split2(v[0], v[1], hh, mm, ll);
+        h[i] = hh;
+        mid[i] = mm;
+        l[i] = ll;
+      }
+      char* dst = Bs + sg::chunk_at(p, chunk + c);
+      *(sg::u32x4_v*)dst = h;
+      *(sg::u32x4_v*)(dst + sg::kPlane) = mid;
+      *(sg::u32x4_v*)(dst + 2 * sg::kPlane) = l;
+    }
   }
-}
-
-// In place on the f32 sums: the bias added after the sum (the reference's order), then the
-// reference activation.
-__global__ void ggml_epilogue_kernel(float* __restrict__ y, const float* __restrict__ bias, int act, int64_t M,
-                                     int64_t N) {
-  const int64_t total = M * N;
-  for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < total; i += (int64_t)gridDim.x * blockDim.x) {
-    float v = y[i];
-    if (bias) v = add_rn(v, bias[i % N]);
-    y[i] = act_ref(v, act);
+  __device__ __forceinline__ float value(const sg::Args& a, int k, int n, const float*) const {
+    return ggml_value(T, a.w + (int64_t)n * a.bpr + (int64_t)(k / vpb) * bpb, k % vpb);
   }
-}
+};
 
 // The K segment of the decode GEMV for these rows: the whole row where it fits (row bytes up to
 // 8 chunks per lane, the rows of x within the LDS), else the longest of ceil(blocks / s) blocks,
@@ -562,7 +588,7 @@ static int64_t ggml_gemv_kseg(const GgmlDesc& d) {
   return 0;
 }
 
-enum class GPlan { kEmpty, kGemv, kDequant, kExact };
+enum class GPlan { kEmpty, kGemv, kSplit, kExact };
 
 static GPlan ggml_plan(const mx_backend* b, const GgmlDesc& d) {
   if (d.M == 0 || d.N == 0) return GPlan::kEmpty;
@@ -576,14 +602,13 @@ static GPlan ggml_plan(const mx_backend* b, const GgmlDesc& d) {
   GgmlDesc g4 = d;
   g4.M = 4;
   const bool gemv4 = ggml_gemv_kseg(g4) != 0;
-  // The weights read once per group of four rows (about 27 us a group at [4096] x 11008 rows),
-  // until one dequantisation and a matrix-core contraction (about 143 us there past 16 rows)
-  // cost less; both scale with the weight bytes, so the crossover holds across shapes.
-  if (d.M <= 20 && gemv4) return GPlan::kGemv;
-  // The dequantised matrix is a device allocation: not for the allocation-free entry point.
-  if (!b->noalloc_active && d.N * d.K * 4 <= ((int64_t)8 << 30) && d.bpr <= kDqRowBytes && d.bpr % 2 == 0 && (uintptr_t)d.w % 2 == 0 &&
-      (uintptr_t)d.x % 16 == 0)
-    return GPlan::kDequant;
+  // The weights read once per group of four rows (22 us a group at [4096] x 11008 Q4_K rows), until
+  // the matrix-core contraction, 90 us there for any count up to 128 rows (333 rows: Q6_K 438 -> 214
+  // us, Q4_K 434 -> 204, Q8_0 443 -> 183 against an f32 copy of the weights and f32 MFMAs), costs
+  // less; both scale with the weights, so the crossover holds across shapes.
+  if (d.M <= 16 && gemv4) return GPlan::kGemv;
+  if (d.M < (int64_t)1 << 30 && d.K <= (int64_t)1 << 22 && d.N < (int64_t)1 << 30 && (uintptr_t)d.w % 2 == 0 && (uintptr_t)d.x % 16 == 0)
+    return GPlan::kSplit;
   return gemv4 ? GPlan::kGemv : GPlan::kExact;
 }
 
@@ -591,7 +616,7 @@ const char* ggml_plan_name(const mx_backend* b, const GgmlDesc& d) {
   switch (ggml_plan(b, d)) {
     case GPlan::kEmpty: return "empty";
     case GPlan::kGemv: return "ggml_gemv";
-    case GPlan::kDequant: return "ggml_dequant_f32_mfma";
+    case GPlan::kSplit: return "ggml_dequant_f32_mfma";
     default: return "ggml_dense_exact";
   }
 }
@@ -646,38 +671,30 @@ int ggml_dense_run(mx_backend* b, const GgmlDesc& d) {
       }
       return MX_OK;
     }
-    case GPlan::kDequant: {
-      void* wt = nullptr;
-      MX_TRY(dev_alloc(b, (size_t)(d.N * d.K) * 4, &wt));
-      const int rows = (int)std::min<int64_t>(d.N, 8 * (int64_t)std::max(b->num_cus, 1));
-      const size_t lds = (size_t)(d.bpr + 15) / 16 * 16;
-      int rc = launch(b, "ggml_dequant_f32", [&] {
+    case GPlan::kSplit: {
+      sg::Args a{};
+      a.x = d.x;
+      a.w = d.w;
+      a.bias = d.bias;
+      a.out = d.out;
+      a.M = (int)d.M;
+      a.K = (int)d.K;
+      a.N = (int)d.N;
+      a.b_dt = MX_DTYPE_FLOAT32;
+      a.act = d.act;
+      a.bpr = d.bpr;
+      int nw = 0, grid = 0;
+      MX_TRY(sg::plan(b, a, d.M, 6, &nw, &grid));
+      return launch(b, "ggml_dequant_f32_mfma", [&] {
+        auto go = [&](auto type) { dispatch(sg::split_gemm_kernel<GgmlSource<decltype(type)::value, 8>, 8>, grid, 512, 0, st, a); };
         switch (d.type) {
-          case MX_GGML_Q4_0: dispatch(ggml_dequant_f32_kernel<MX_GGML_Q4_0>, rows, 256, lds, st, d, (float*)wt); break;
-          case MX_GGML_Q8_0: dispatch(ggml_dequant_f32_kernel<MX_GGML_Q8_0>, rows, 256, lds, st, d, (float*)wt); break;
-          case MX_GGML_IQ4_NL: dispatch(ggml_dequant_f32_kernel<MX_GGML_IQ4_NL>, rows, 256, lds, st, d, (float*)wt); break;
-          case MX_GGML_Q4_K: dispatch(ggml_dequant_f32_kernel<MX_GGML_Q4_K>, rows, 256, lds, st, d, (float*)wt); break;
-          default: dispatch(ggml_dequant_f32_kernel<MX_GGML_Q6_K>, rows, 256, lds, st, d, (float*)wt); break;
+          case MX_GGML_Q4_0: go(std::integral_constant<int, MX_GGML_Q4_0>{}); break;
+          case MX_GGML_Q8_0: go(std::integral_constant<int, MX_GGML_Q8_0>{}); break;
+          case MX_GGML_IQ4_NL: go(std::integral_constant<int, MX_GGML_IQ4_NL>{}); break;
+          case MX_GGML_Q4_K: go(std::integral_constant<int, MX_GGML_Q4_K>{}); break;
+          default: go(std::integral_constant<int, MX_GGML_Q6_K>{}); break;
         }
       });
-      if (rc == MX_OK) {
-        DotDesc dd{};
-        dd.lhs = d.x;
-        dd.rhs = wt;
-        dd.out = d.out;
-        dd.B = 1;
-        dd.M = d.M;
-        dd.K = d.K;
-        dd.N = d.N;
-        dd.rhs_transposed = true;
-        dd.in_dt = MX_DTYPE_FLOAT32;
-        dd.out_dt = MX_DTYPE_FLOAT32;
-        rc = dot_run(b, dd);
-      }
-      if (rc == MX_OK)
-        rc = launch(b, "ggml_epilogue", [&] { dispatch(ggml_epilogue_kernel, 1024, 256, 0, st, d.out, d.bias, d.act, d.M, d.N); });
-      dev_free(b, wt);  // stream-ordered pool: later users run after these kernels
-      return rc;
     }
     default: {
       dim3 grid((unsigned)((d.N + kGxThreads - 1) / kGxThreads), (unsigned)((d.M + kGxRows - 1) / kGxRows));

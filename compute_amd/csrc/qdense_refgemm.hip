@@ -31,48 +31,57 @@ enum RgScales {
   kRgAny = 2    // [K, ceil(N/B)], any B: one per column
 };
 
-// Weights [K, N]: thread t converts columns 4 cq .. 4 cq + 3 of rows 4 j .. 4 j + 3 of a block, with
-// j's low bit in the thread's (so that lane pairs write whole 16-byte chunks).
-template <int WDT, int FORM, int SM, bool XBF>
+// What the weight factor holds beside the code times the scale.
+enum RgKind { kLinear = 0, kZeroPoint, kNf4 };
+
+// Weights [K, N]: thread t converts CT = 16 / NW columns of rows 4 j .. 4 j + 3 of a block, with j's
+// low bit in the thread's (so that lane pairs write whole 16-byte chunks): columns 4 cq + c0 ..
+// 4 cq + c0 + CT - 1 of the tile.
+template <int WDT, int FORM, int SM, int KIND, bool XBF, int NW>
 struct RgSource {
   static constexpr bool kXbf = XBF;
-  static constexpr bool kRow = FORM == RgForm::kRow, kCol = FORM == kColumn;
+  static constexpr bool kRow = FORM == RgForm::kRow, kCol = FORM == kColumn, kZp = KIND == kZeroPoint;
   static constexpr int kPA = XBF && FORM != RgForm::kRow ? 1 : 3;
   static constexpr int kPB = FORM == kWeight ? 3 : 1;
   static constexpr bool kI4 = WDT == MX_DTYPE_INT4 || WDT == MX_DTYPE_UINT4;
   static constexpr bool kSigned = WDT == MX_DTYPE_INT4 || WDT == MX_DTYPE_INT8;
-  static constexpr int kScales = FORM != kWeight ? 1 : SM == kRgBlk ? 1 : 4;  // per row
+  static constexpr int CT = 16 / NW;
+  static constexpr int kScales = FORM != kWeight ? 1 : SM == kRgBlk ? 1 : CT;  // per row
 
   struct Regs {
     uint32_t w[4];
-    uint32_t s[4][kScales], z[4][kScales];  // raw words (kRgCols with bf16: two pairs)
+    uint32_t s[4][kScales], z[4][kScales];  // raw words (kRgCols with bf16: pairs)
     uint32_t ssh[4][kScales], zsh[4][kScales];
   };
-  int cq, j, ncl;
-  const char* wp;
+  int cq, c0, j, ncl;
+  uint32_t woff[4];  // from a block's first row
+  static __device__ __forceinline__ float table_value(int i) { return kNF4Table[i]; }
 
   __device__ __forceinline__ RgSource(const Args& a, int t, int n0) {
     cq = (t >> 1) & 31;
-    j = (t & 1) | (t >> 6) << 1;
-    // N % 16 == 0: the 4 columns are all in range or all past N (then column 0 is read and the
+    c0 = NW == 8 ? 2 * ((t >> 6) & 1) : 0;
+    j = (t & 1) | (t >> (NW == 8 ? 7 : 6)) << 1;
+    // N % 16 == 0: the columns are all in range or all past N (then the first are read and the
     // outputs are not stored).
-    ncl = n0 + 4 * cq < a.N ? n0 + 4 * cq : 0;
-    wp = (const char*)a.w + (kI4 ? ncl / 2 : ncl);
+    ncl = n0 + 4 * cq < a.N ? n0 + 4 * cq + c0 : 0;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) woff[e] = ((uint32_t)(4 * j + e) * (uint32_t)a.N + (uint32_t)ncl) / (kI4 ? 2 : 1);
   }
-  // The aligned word holding element i of an f32 or bf16 array, and the shift that moves a bf16
-  // element to its high half.
-  static __device__ __forceinline__ void word(const void* p, int64_t i, bool bf, uint32_t& w, uint32_t& sh) {
-    const uintptr_t ad = (uintptr_t)p + (uintptr_t)i * (bf ? 2 : 4);
-    w = *(const uint32_t*)(ad & ~(uintptr_t)3);
-    sh = bf && (ad & 2) == 0 ? 16u : 0u;
+  // CT consecutive elements from i on: f32 CT words; bf16 CT / 2 words, repeated (one form for both).
+  static __device__ __forceinline__ void words(const void* p, int64_t i, bool bf, uint32_t (&w)[kScales]) {
+    const uint32_t* q = (const uint32_t*)((const char*)p + i * (bf ? 2 : 4));
+#pragma unroll
+    for (int c = 0; c < kScales; ++c) w[c] = q[bf ? c / 2 : c];
   }
-  __device__ __forceinline__ void load(const Args& a, int kb, Regs& R) const {
-    const int k0 = kb * kBK + 4 * j;
+  __device__ __forceinline__ void load(const Args& a, Block b, Regs& R) const {
+    const char* base = (const char*)a.w + (int64_t)b.k * (kI4 ? a.N / 2 : a.N);
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
-      const int k = min(k0 + e, a.K - 1);
-      const char* p = wp + (int64_t)k * (kI4 ? a.N / 2 : a.N);
-      if constexpr (kI4)
+      const int k = b.k + 4 * j + e;
+      const char* p = base + woff[e];
+      if constexpr (kI4 && CT == 2)
+        R.w[e] = *(const uint8_t*)p;
+      else if constexpr (kI4 || CT == 2)
         R.w[e] = *(const uint16_t*)p;
       else
         R.w[e] = *(const uint32_t*)p;
@@ -80,21 +89,14 @@ struct RgSource {
         const bool sbf = a.s_dt == MX_DTYPE_BFLOAT16, zbf = a.zp_dt == MX_DTYPE_BFLOAT16;
         if constexpr (SM == kRgCols) {
           const int64_t i = (int64_t)(k / a.B) * a.N + ncl;
-          // bf16: 8 bytes are the 4 scales; f32: 16 (two loads, so that the form is one).
-          const char* sp = (const char*)a.scale + i * (sbf ? 2 : 4);
-          const u32x2_v lo = *(const u32x2_v*)sp, hi = *(const u32x2_v*)(sp + (sbf ? 0 : 8));
-          R.s[e][0] = lo[0], R.s[e][1] = lo[1], R.s[e][2] = hi[0], R.s[e][3] = hi[1];
-          if (a.zp) {
-            const char* zq = (const char*)a.zp + i * (zbf ? 2 : 4);
-            const u32x2_v zl = *(const u32x2_v*)zq, zh = *(const u32x2_v*)(zq + (zbf ? 0 : 8));
-            R.z[e][0] = zl[0], R.z[e][1] = zl[1], R.z[e][2] = zh[0], R.z[e][3] = zh[1];
-          }
+          words(a.scale, i, sbf, R.s[e]);
+          if constexpr (kZp) words(a.zp, i, zbf, R.z[e]);
         } else {
 #pragma unroll
           for (int c = 0; c < kScales; ++c) {
             const int64_t i = (int64_t)k * a.nb + (ncl + c) / a.B;
             word(a.scale, i, sbf, R.s[e][c], R.ssh[e][c]);
-            if (a.zp) word(a.zp, i, zbf, R.z[e][c], R.zsh[e][c]);
+            if constexpr (kZp) word(a.zp, i, zbf, R.z[e][c], R.zsh[e][c]);
           }
         }
       }
@@ -108,31 +110,32 @@ struct RgSource {
   }
   static __device__ __forceinline__ float scale_of(const uint32_t (&s)[kScales], const uint32_t (&sh)[kScales], int c, bool bf) {
     if constexpr (SM == kRgCols)
-      return bf ? __uint_as_float(c & 1 ? s[(c >> 1) % kScales] & 0xFFFF0000u : s[(c >> 1) % kScales] << 16)
-                : __uint_as_float(s[c % kScales]);
+      return __uint_as_float(bf ? (c & 1 ? s[c % kScales] & 0xFFFF0000u : s[c % kScales] << 16) : s[c % kScales]);
     else
-      return __uint_as_float((s[c % kScales] << sh[c % kScales]) & (bf ? 0xFFFF0000u : ~0u));
+      return word_f32(s[c % kScales], sh[c % kScales], bf);
   }
-  __device__ __forceinline__ void stage(const Args& a, int kb, const Regs& R, const float* table, char* Bs, int& odd) const {
+  template <class TailT>
+  __device__ __forceinline__ void stage(const Args& a, Block b, const Regs& R, const float* table, char* Bs, float& big, TailT) const {
+    const bool sbf = a.s_dt == MX_DTYPE_BFLOAT16, zbf = a.zp_dt == MX_DTYPE_BFLOAT16;
 #pragma unroll
-    for (int c = 0; c < 4; ++c) {
-      char* dst = Bs + chunk_at(c * 32 + cq, j >> 1) + 8 * (j & 1);
+    for (int c = 0; c < CT; ++c) {
+      char* dst = Bs + chunk_at(row_of_col(4 * cq + c0 + c), j >> 1) + 8 * (j & 1);
       float v[4];
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
         const int q = code(R.w[e], c);
         if constexpr (FORM == kWeight) {
-          const bool sbf = a.s_dt == MX_DTYPE_BFLOAT16, zbf = a.zp_dt == MX_DTYPE_BFLOAT16;
-          const float wf = a.nf4 ? table[(uint32_t)q & 15u] : (float)q;
-          const float ws = mul_rn(wf, scale_of(R.s[e], R.ssh[e], c, sbf));
-          v[e] = a.zp ? add_rn(ws, scale_of(R.z[e], R.zsh[e], c, zbf)) : ws;
-          if (kb * kBK + 4 * j + e >= a.K) v[e] = 0.0f;  // x is zero there, but 0 * inf is not
+          const float wf = KIND == kNf4 ? table[(uint32_t)q & 15u] : (float)q;
+          v[e] = mul_rn(wf, scale_of(R.s[e], R.ssh[e], c, sbf));
+          if constexpr (kZp) v[e] = add_rn(v[e], scale_of(R.z[e], R.zsh[e], c, zbf));
+          if (TailT::value && 4 * j < b.skip) v[e] = 0.0f;  // x is zero there, but 0 * inf is not
         } else {
           v[e] = (float)q;
         }
       }
       if constexpr (FORM == kWeight) {
-        if (fmaxf(fmaxf(fabsf(v[0]), fabsf(v[1])), fmaxf(fabsf(v[2]), fabsf(v[3]))) > MX_SPLIT_MAX) odd = 1;
+        big = fmaxf(fmaxf(fabsf(v[0]), fabsf(v[1])), big);
+        big = fmaxf(fmaxf(fabsf(v[2]), fabsf(v[3])), big);
         uint32_t h0, m0, l0, h1, m1, l1;
         split2(v[0], v[1], h0, m0, l0);
         split2(v[2], v[3], h1, m1, l1);
@@ -149,29 +152,54 @@ struct RgSource {
   // The weight factor of (k, n) as the reference forms it (column form: without its scale).
   __device__ __forceinline__ float value(const Args& a, int k, int n, const float* table) const {
     const int q = decode_weight(a.w, (int64_t)k * a.N + n, WDT);
-    const float wf = a.nf4 ? table[(uint32_t)q & 15u] : (float)q;
+    const float wf = KIND == kNf4 ? table[(uint32_t)q & 15u] : (float)q;
     if constexpr (FORM == kColumn) return wf;
     const int64_t i = SM == kRgCols ? (int64_t)(k / a.B) * a.N + n : (int64_t)k * a.nb + n / a.B;
     const float ws = mul_rn(wf, elem(a.scale, i, a.s_dt));
-    return a.zp ? add_rn(ws, elem(a.zp, i, a.zp_dt)) : ws;
+    return kZp ? add_rn(ws, elem(a.zp, i, a.zp_dt)) : ws;
   }
 };
 
-template <int WDT, bool XBF>
-void rg_dispatch(const QDenseDesc& d, const Args& a, int grid, hipStream_t st) {
-  const bool linear = d.scheme == MX_QUANT_LINEAR;
-  if (d.block_axis == 0) {
-    if (linear && !d.zp && d.block_size >= d.K)
-      dispatch(split_gemm_kernel<RgSource<WDT, kColumn, kRgCols, XBF>>, grid, kThreads, 0, st, a);
-    else
-      dispatch(split_gemm_kernel<RgSource<WDT, kWeight, kRgCols, XBF>>, grid, kThreads, 0, st, a);
-  } else if (linear && (a.nb == 1 || a.B % kBN == 0)) {
-    dispatch(split_gemm_kernel<RgSource<WDT, RgForm::kRow, kRgBlk, XBF>>, grid, kThreads, 0, st, a);
-  } else if (a.B % 4 == 0) {
-    dispatch(split_gemm_kernel<RgSource<WDT, kWeight, kRgBlk, XBF>>, grid, kThreads, 0, st, a);
-  } else {
-    dispatch(split_gemm_kernel<RgSource<WDT, kWeight, kRgAny, XBF>>, grid, kThreads, 0, st, a);
+template <int WDT, int FORM, int SM, int KIND, bool XBF>
+int rg_launch(mx_backend* b, const char* name, Args& a) {
+  using S8 = RgSource<WDT, FORM, SM, KIND, XBF, 8>;
+  int nw = 0, grid = 0;
+  MX_TRY(plan(b, a, a.M, S8::kPA + S8::kPB, &nw, &grid));
+  return launch(b, name, [&] {
+    if constexpr (S8::kPA + S8::kPB <= 4) {
+      if (nw == 4) {
+        dispatch(split_gemm_kernel<RgSource<WDT, FORM, SM, KIND, XBF, 4>, 4>, grid, 256, 0, b->stream, a);
+        return;
+      }
+    }
+    dispatch(split_gemm_kernel<S8, 8>, grid, 512, 0, b->stream, a);
+  });
+}
+
+template <int WDT, int SM, int KIND, bool XBF>
+int rg_forms(mx_backend* b, const char* name, const QDenseDesc& d, Args& a) {
+  if constexpr (KIND == kLinear && SM == kRgCols) {
+    if (d.block_size >= d.K) return rg_launch<WDT, kColumn, kRgCols, KIND, XBF>(b, name, a);
   }
+  if constexpr (KIND != kNf4 && SM == kRgBlk) {
+    if (a.nb == 1 || a.B % kBN == 0) return rg_launch<WDT, RgForm::kRow, kRgBlk, KIND, XBF>(b, name, a);
+  }
+  return rg_launch<WDT, kWeight, SM, KIND, XBF>(b, name, a);
+}
+
+template <int WDT, int KIND, bool XBF>
+int rg_scales(mx_backend* b, const char* name, const QDenseDesc& d, Args& a) {
+  if (d.block_axis == 0) return rg_forms<WDT, kRgCols, KIND, XBF>(b, name, d, a);
+  if (a.B % 4 == 0 || a.nb == 1) return rg_forms<WDT, kRgBlk, KIND, XBF>(b, name, d, a);
+  return rg_forms<WDT, kRgAny, KIND, XBF>(b, name, d, a);
+}
+
+template <int WDT, bool XBF>
+int rg_dispatch(mx_backend* b, const char* name, const QDenseDesc& d, Args& a) {
+  // NF4 codes are taken & 15: signed and unsigned storage are the same.
+  if (d.scheme == MX_QUANT_NF4)
+    return rg_scales<WDT == MX_DTYPE_INT8 ? MX_DTYPE_UINT8 : WDT == MX_DTYPE_INT4 ? MX_DTYPE_UINT4 : WDT, kNf4, XBF>(b, name, d, a);
+  return d.zp ? rg_scales<WDT, kZeroPoint, XBF>(b, name, d, a) : rg_scales<WDT, kLinear, XBF>(b, name, d, a);
 }
 
 }  // namespace
@@ -181,9 +209,10 @@ bool qdense_refgemm_fits(const QDenseDesc& d) {
   const bool xbf = d.x_dt == MX_DTYPE_BFLOAT16;
   const bool packed = dtype_is_packed(d.w_dt);
   if (!(d.scheme == MX_QUANT_LINEAR || d.scheme == MX_QUANT_NF4)) return false;
-  if (!(d.x_dt == MX_DTYPE_FLOAT32 || xbf) || d.M < 1 || d.K < 8 || d.N < 16 || d.N % 16 != 0) return false;
+  if (!(d.x_dt == MX_DTYPE_FLOAT32 || xbf) || d.M < 1 || d.K < kBK || d.N < 16 || d.N % 16 != 0) return false;
   if (d.K % (xbf ? 8 : 4) != 0 || !aligned(d.x, 16) || !aligned(d.w, packed ? 8 : 16)) return false;
-  if (d.M >= (int64_t)1 << 30 || d.K >= (int64_t)1 << 30 || d.N >= (int64_t)1 << 30) return false;
+  // A tile's rows of x and a block's rows of weights are addressed by 32-bit offsets.
+  if (d.M >= (int64_t)1 << 30 || d.K > (int64_t)1 << 22 || d.N > (int64_t)1 << 26) return false;
   if (d.block_axis == 0) {
     // 4 consecutive scales of a row: vector loads.
     if (!aligned(d.scale, 16) || (d.zp && !aligned(d.zp, 16))) return false;
@@ -206,25 +235,19 @@ int qdense_refgemm_run(mx_backend* b, const QDenseDesc& d, const char* name) {
   a.zp_dt = d.zp ? d.zp_dt : MX_DTYPE_FLOAT32;
   a.b_dt = d.b_dt;
   a.act = d.act;
-  a.nf4 = d.scheme == MX_QUANT_NF4 ? 1 : 0;
   a.B = (int)std::min<int64_t>(d.block_size, d.block_axis == 0 ? d.K : d.N);
   a.nb = (int)((d.N + a.B - 1) / a.B);
-  int grid = 0;
-  MX_TRY(plan(b, a, d.M, &grid));
   const bool xbf = d.x_dt == MX_DTYPE_BFLOAT16;
-  hipStream_t st = b->stream;
-  return launch(b, name, [&] {
-    auto go = [&](auto wdt) {
-      constexpr int W = decltype(wdt)::value;
-      xbf ? rg_dispatch<W, true>(d, a, grid, st) : rg_dispatch<W, false>(d, a, grid, st);
-    };
-    switch (d.w_dt) {
-      case MX_DTYPE_INT8: go(std::integral_constant<int, MX_DTYPE_INT8>{}); break;
-      case MX_DTYPE_UINT8: go(std::integral_constant<int, MX_DTYPE_UINT8>{}); break;
-      case MX_DTYPE_INT4: go(std::integral_constant<int, MX_DTYPE_INT4>{}); break;
-      default: go(std::integral_constant<int, MX_DTYPE_UINT4>{}); break;
-    }
-  });
+  auto go = [&](auto wdt) {
+    constexpr int W = decltype(wdt)::value;
+    return xbf ? rg_dispatch<W, true>(b, name, d, a) : rg_dispatch<W, false>(b, name, d, a);
+  };
+  switch (d.w_dt) {
+    case MX_DTYPE_INT8: return go(std::integral_constant<int, MX_DTYPE_INT8>{});
+    case MX_DTYPE_UINT8: return go(std::integral_constant<int, MX_DTYPE_UINT8>{});
+    case MX_DTYPE_INT4: return go(std::integral_constant<int, MX_DTYPE_INT4>{});
+    default: return go(std::integral_constant<int, MX_DTYPE_UINT4>{});
+  }
 }
 
 }  // namespace mx

@@ -7,20 +7,20 @@
 // term each, are left out).  The bf16 MFMAs have 16 times the rate of v_mfma_f32_16x16x4_f32, so 3
 // products have 5.3 times and 6 products 2.7 times the f32 matrix cores' peak.
 //
-// What bounds it: matrix-core issue, with the conversions (about 7 VALU instructions per x value
-// and part set) beside it.  Measured, f32 x [2048,4096] x Int4 [4096,11008], against the f32-MFMA
-// kernel this replaced (which ran at 0.63 of the f32 peak): scales per row and 128 columns (3
-// products) 1868 -> 607 us, 0.91 PFLOP/s of products; per row and 64 columns (6 products) 1868 ->
-// 1291 us; with 100 rows 363 -> 91 us (K in 2 slices).  The error against 64 bits fell from 1.1e-6
-// to 5.8e-7 (3 products) and 9.9e-7 (6): a step sums 32 terms where the f32 MFMA summed 4.
+// What bounds it: matrix-core and VALU issue together (an MFMA keeps the VALU from about 2.5 of its
+// own issue slots; at four VALU instructions per MFMA, the conversions' share with 3 products, the
+// two run 12 ns per MFMA and SIMD where the MFMA alone takes 8).  Measured, f32 x [2048,4096] x Int4
+// [4096,11008], against an f32-MFMA kernel at 0.63 of the f32 peak: scales per row and 128 columns
+// (3 products) 1868 -> 578 us, 0.96 PFLOP/s of products; per row and 64 columns (6 products) 1868 ->
+// 1010 us; with 100 rows 363 -> 60 us (K in 2 slices).  The error against 64 bits fell from 1.1e-6
+// to 5.8e-7 (3 products) and 9.8e-7 (6): a step sums 32 terms where the f32 MFMA summed 4.
 //
-// Tiling: a workgroup of 4 waves owns a 128 x 128 output tile (2 x 2 waves of 64 x 64), K in
-// blocks of 32 (one MFMA step).  An operand's part lies in LDS as 128 rows of 32 bf16 (64 bytes,
-// four 16-byte chunks XOR-swizzled by (row >> 1) & 3: every 16-row operand read and every staging
-// write covers all banks).  Block kb + 1 is requested into registers before block kb is
-// multiplied, then split and written to the other LDS buffer (one buffer and a second barrier
-// where both operands have three parts).  Two workgroups share a CU, so one's conversions run
-// under the other's MFMAs.
+// Tiling: a workgroup of 4 (or 8) waves owns a 128 x 128 output tile, 2 x 2 waves of 64 x 64 (4 x 2
+// of 32 x 64), K in blocks of 32 (one MFMA step).  An operand's part lies in LDS as 128 rows of 32
+// bf16 (64 bytes, four 16-byte chunks XOR-swizzled by (row >> 1) & 3: every operand read and every
+// staging write covers all banks).  Block kb is multiplied while block kb + 1, in registers, is
+// split into the other LDS buffer and block kb + 2 is requested.  K past the last whole block: that
+// block starts 32 before K's end and the values the block before it holds are zeroed.
 //
 // Column n of the tile lies in LDS row (n & 3) * 32 + (n >> 2): MFMA column set c of wave half wn
 // holds columns 64 wn + 4 cg + c, so a lane ends with four consecutive columns of each of its rows.
@@ -43,7 +43,7 @@ typedef float f32x4_t __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x4_v __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x2_v __attribute__((ext_vector_type(2)));
 
-constexpr int kBM = 128, kBN = 128, kBK = 32, kThreads = 256;
+constexpr int kBM = 128, kBN = 128, kBK = 32;
 constexpr int kPlane = kBM * kBK * 2;  // LDS bytes of one part of an operand
 constexpr size_t kCounterBytes = 64 * 1024;
 constexpr int kPartBytes = kBM * kBN * 4;  // one partial tile
@@ -62,19 +62,32 @@ struct Args {
   const void* bias;   // [N] or null
   void* out;          // [M, N], x's dtype
   int M, K, N;
-  int s_dt, zp_dt, b_dt, act, nf4;
+  int s_dt, zp_dt, b_dt, act;
   int B;              // block size along the scale's blocked axis
   int nb;             // scale row length of the reference layout: ceil(N / B)
   int64_t bpr;        // GGML: bytes per weight row
-  int tiles_n, items, per_xcd;
-  int vec;            // out is aligned for stores of 4 values
-  int S, kpb;         // K slices per tile, 32-row blocks per slice
-  float* part;        // [tile][S] partial tiles (S > 1)
-  uint32_t* ctr;      // [tile] arrivals, zero between launches
+  // Work items: `whole` whole tiles (a multiple of 8), then `tail` items, the S slices of each of the
+  // remaining tiles next to each other.
+  int tiles_n, whole, tail, per_xcd;  // per_xcd: tail items per XCD
+  int vec;            // out's rows take stores of 4 values
+  int S, kpb;         // K slices of a tail tile, 32-row blocks per slice
+  float* part;        // [tail tile][S] partial tiles (S > 1)
+  uint32_t* ctr;      // [tail tile] arrivals, zero between launches
 };
 
 __device__ __forceinline__ f32x4_t mfma(const u32x4_v& a, const u32x4_v& b, f32x4_t c) {
   return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, a), __builtin_bit_cast(bf16x8_t, b), c, 0, 0, 0);
+}
+
+// The aligned word holding element i of an f32 or bf16 array, and the shift that moves a bf16
+// element to its high half (no branch on the dtype, and the load never leaves the element's word).
+__device__ __forceinline__ void word(const void* p, int64_t i, bool bf, uint32_t& w, uint32_t& sh) {
+  const uintptr_t ad = (uintptr_t)p + (uintptr_t)i * (bf ? 2 : 4);
+  w = *(const uint32_t*)(ad & ~(uintptr_t)3);
+  sh = bf && (ad & 2) == 0 ? 16u : 0u;
+}
+__device__ __forceinline__ float word_f32(uint32_t w, uint32_t sh, bool bf) {
+  return __uint_as_float((w << sh) & (bf ? 0xFFFF0000u : ~0u));
 }
 
 __device__ __forceinline__ uint32_t pack_bf16(float a, float b) {
@@ -95,6 +108,10 @@ __device__ __forceinline__ uint32_t chunk_at(int p, int chunk) {
   return (uint32_t)(p * 64 + ((chunk ^ ((p >> 1) & 3)) << 4));
 }
 
+// LDS row of column n of the tile, and back.
+__device__ __forceinline__ int row_of_col(int n) { return (n & 3) * 32 + (n >> 2); }
+__device__ __forceinline__ int col_of_row(int p) { return 4 * (p & 31) + (p >> 5); }
+
 // Element i of an f32 or bf16 array as f32.
 __device__ __forceinline__ float elem(const void* p, int64_t i, int dt) {
   return dt == MX_DTYPE_BFLOAT16 ? bf16_to_f32(((const uint16_t*)p)[i]) : ((const float*)p)[i];
@@ -102,66 +119,89 @@ __device__ __forceinline__ float elem(const void* p, int64_t i, int dt) {
 
 // P: the operand policy.  P::kXbf bf16 x (else f32); P::kPA, P::kPB parts of x and of the weights;
 // P::kRow each x value multiplied by its row's scale of the tile's column block before the split
-// (reference layout, one block per tile), zero points summed beside it; P::kCol one scale per
-// column, applied to the sums; P::Regs, load, stage: the weights' registers for a block, their
-// loads, and their parts into LDS; P::value: the f32 weight factor of one (k, n).
-template <class P>
-__global__ __launch_bounds__(kThreads, 2) void split_gemm_kernel(Args a) {
+// (reference layout, one block per tile), P::kZp zero points (row form: summed beside the product);
+// P::kCol one scale per column, applied to the sums; P::Regs, load, stage: a thread's weights of a
+// block, their loads, and their parts into LDS (kTail: zeros past K; `big` takes the largest
+// magnitude); P::value: the f32 weight factor of one (k, n); P::table_value: the 16 entries of the
+// lookup table.
+// NW: waves of the workgroup, 4 (2 x 2 waves of 64 x 64) or 8 (4 x 2 waves of 32 x 64).
+// A block of K: its first row and how many of its rows the block before it holds (the last block of
+// a K that is no multiple of 32).
+struct Block {
+  int k, skip;
+  __device__ __forceinline__ Block(int kb, int K) : k(min(kb * kBK, K - kBK)), skip(kb * kBK - k) {}
+};
+
+template <class P, int NW>
+__global__ __launch_bounds__(64 * NW, 2) void split_gemm_kernel(Args a) {
   constexpr int PA = P::kPA, PB = P::kPB;
+  constexpr int kThreads = 64 * NW, RB = 16 / NW;  // 16-row blocks per wave
   constexpr int kBufBytes = (PA + PB) * kPlane;
-  constexpr int NBUF = PA + PB <= 4 ? 2 : 1;
+  constexpr int XR = 8 / NW;  // rows of x per thread and block
   static_assert(!P::kRow || (PA == 3 && PB == 1), "row scales: split x, exact weight codes");
-  __shared__ __attribute__((aligned(16))) char sm[NBUF][kBufBytes];
+  __shared__ __attribute__((aligned(16))) char sm[2][kBufBytes];
   __shared__ __attribute__((aligned(16))) float ring[P::kRow ? 2 : 1][2][kBK];  // scales, zero points of a block's rows
   __shared__ float zrow[P::kRow ? kBM : 1];
   __shared__ float table[16];
-  __shared__ int odd;  // a value that cannot be split was staged
+  __shared__ int flag;
 
-  // XCD-contiguous order, slices of a tile next to each other, tiles M-major.
-  const int item = (blockIdx.x & 7) * a.per_xcd + (blockIdx.x >> 3);
-  if ((int)(blockIdx.x >> 3) >= a.per_xcd || item >= a.items) return;
-  const int tile = item / a.S, slice = item - tile * a.S;
+  // Workgroups go round-robin over the 8 XCDs: each XCD takes a contiguous run of the whole tiles
+  // (M-major: its tiles share x rows in its L2) and one of the tail items.
+  const int bid = blockIdx.x, xcd = bid & 7;
+  int tile, slice = 0, kpb = 1 << 26;
+  const bool sliced = bid >= a.whole && a.S > 1;
+  if (bid < a.whole) {
+    tile = xcd * (a.whole >> 3) + (bid >> 3);
+  } else {
+    const int j = (bid - a.whole) >> 3, item = xcd * a.per_xcd + j;
+    if (j >= a.per_xcd || item >= a.tail) return;
+    tile = item / a.S;
+    slice = item - tile * a.S;
+    kpb = a.kpb;
+    tile += a.whole;
+  }
   const int m0 = (tile / a.tiles_n) * kBM, n0 = (tile % a.tiles_n) * kBN;
   const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
   const int wm = wave >> 1, wn = wave & 1, cg = lane & 15, kq = lane >> 4;
   const int M = a.M, K = a.K, N = a.N;
-  if (t < 16) table[t] = kNF4Table[t];
-  if (t == 16) odd = 0;
+  const int row0 = 16 * RB * wm;  // the wave's first row in the tile
+  if (t < 16) table[t] = P::table_value(t);
+  if (t == 16) flag = 0;
 
-  const int kb0 = slice * a.kpb, kb1 = min(kb0 + a.kpb, (K + kBK - 1) / kBK);
+  const int kb0 = slice * kpb, kb1 = min(kb0 + kpb, (K + kBK - 1) / kBK);
 
-  // ---- x: thread t stages k chunk t & 3 (8 values) of rows t / 4 and t / 4 + 64.  Rows past M
-  // read row M - 1 (their outputs are not stored).
+  // ---- x: thread t stages k chunk t & 3 (8 values) of rows t / 4 and, with 4 waves, t / 4 + 64.
+  // Rows past M read row M - 1 (their outputs are not stored).
   const int xr = t >> 2, xc = t & 3;
-  const char* xp[2];
+  constexpr int kXe = P::kXbf ? 2 : 4;  // bytes of an element
+  const char* xbase = (const char*)a.x + (int64_t)m0 * K * kXe;
+  uint32_t xoff[XR];  // from the tile's first row (128 K elements stay below 2^31 bytes, checked by the host)
 #pragma unroll
-  for (int i = 0; i < 2; ++i) xp[i] = (const char*)a.x + (int64_t)min(m0 + xr + 64 * i, M - 1) * K * (P::kXbf ? 2 : 4);
+  for (int i = 0; i < XR; ++i) xoff[i] = ((uint32_t)min(xr + 64 * i, M - 1 - m0) * (uint32_t)K + 8u * xc) * kXe;
   struct XRegs {
-    u32x4_v v[2][P::kXbf ? 1 : 2];
+    u32x4_v v[XR][P::kXbf ? 1 : 2];
   };
-  auto load_x = [&](int kb, XRegs& R) __attribute__((always_inline)) {
-    const int k = kb * kBK + 8 * xc;
+  auto load_x = [&](Block b, XRegs& R) __attribute__((always_inline)) {
+    const char* base = xbase + (int64_t)b.k * kXe;
 #pragma unroll
-    for (int i = 0; i < 2; ++i) {
-      if constexpr (P::kXbf) {
-        R.v[i][0] = *(const u32x4_v*)(xp[i] + (int64_t)min(k, K - 8) * 2);
-      } else {
-        R.v[i][0] = *(const u32x4_v*)(xp[i] + (int64_t)min(k, K - 4) * 4);
-        R.v[i][1] = *(const u32x4_v*)(xp[i] + (int64_t)min(k + 4, K - 4) * 4);
-      }
+    for (int i = 0; i < XR; ++i) {
+      R.v[i][0] = *(const u32x4_v*)(base + xoff[i]);
+      if constexpr (!P::kXbf) R.v[i][1] = *(const u32x4_v*)(base + xoff[i] + 16);
     }
   };
-  float zacc[2] = {0.f, 0.f};
-  // Values of k past K are zero (K % 8 == 0 for bf16 x, K % 4 == 0 for f32).
-  auto stage_x = [&](int kb, const XRegs& R, char* As) __attribute__((always_inline)) {
-    const int k = kb * kBK + 8 * xc;
-    const bool lo = k < K, hi = P::kXbf ? lo : k + 4 < K;
+  float zacc[XR], big = 0.0f;
 #pragma unroll
-    for (int i = 0; i < 2; ++i) {
+  for (int i = 0; i < XR; ++i) zacc[i] = 0.0f;
+  // With kTail, the values that the block before holds are zero (whole runs of 8 bf16 or 4 f32).
+  auto stage_x = [&](int slot, Block b, const XRegs& R, char* As, auto tail) __attribute__((always_inline)) {
+    constexpr bool kTail = decltype(tail)::value;
+    const bool lo = !kTail || 8 * xc >= b.skip, hi = !kTail || (P::kXbf ? lo : 8 * xc + 4 >= b.skip);
+#pragma unroll
+    for (int i = 0; i < XR; ++i) {
       char* dst = As + chunk_at(xr + 64 * i, xc);
       if constexpr (PA == 1) {
         u32x4_v v = R.v[i][0];
-        if (!lo) v = u32x4_v{0u, 0u, 0u, 0u};
+        if (kTail && !lo) v = u32x4_v{0u, 0u, 0u, 0u};
         *(u32x4_v*)dst = v;
       } else {
         float v[8];
@@ -171,22 +211,20 @@ __global__ __launch_bounds__(kThreads, 2) void split_gemm_kernel(Args a) {
             v[e] = __uint_as_float(e & 1 ? R.v[i][0][e >> 1] & 0xFFFF0000u : R.v[i][0][e >> 1] << 16);
           else
             v[e] = __uint_as_float(R.v[i][e >> 2][e & 3]);
-          v[e] = (e < 4 ? lo : hi) ? v[e] : 0.0f;
+          if constexpr (kTail) v[e] = (e < 4 ? lo : hi) ? v[e] : 0.0f;
         }
         if constexpr (P::kRow) {
-          const float* s = &ring[kb & 1][0][8 * xc];
-          if (a.zp) {
-            const float* z = &ring[kb & 1][1][8 * xc];
+          const float* s = &ring[slot][0][8 * xc];
+          if constexpr (P::kZp) {
+            const float* z = &ring[slot][1][8 * xc];
 #pragma unroll
             for (int e = 0; e < 8; ++e) zacc[i] = __builtin_fmaf(v[e], z[e], zacc[i]);
           }
 #pragma unroll
           for (int e = 0; e < 8; ++e) v[e] = mul_rn(v[e], s[e]);
         }
-        float big = fabsf(v[0]);
 #pragma unroll
-        for (int e = 1; e < 8; ++e) big = fmaxf(big, fabsf(v[e]));
-        if (big > MX_SPLIT_MAX) odd = 1;
+        for (int e = 0; e < 8; e += 2) big = fmaxf(fmaxf(fabsf(v[e]), fabsf(v[e + 1])), big);
         u32x4_v h, m, l;
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
@@ -202,32 +240,33 @@ __global__ __launch_bounds__(kThreads, 2) void split_gemm_kernel(Args a) {
       }
     }
   };
-  // Row scales and zero points of block kb, one row per thread of the first 32, into their slot
-  // two blocks ahead of their use.
-  float rs = 0.f, rz = 0.f;
-  auto load_row_scale = [&](int kb) __attribute__((always_inline)) {
+  // Row scales and zero points of a block, its row t & 31 by every thread (the copies write the
+  // same words), into their slot two blocks ahead of their use.
+  uint32_t rs = 0, rz = 0, rssh = 0, rzsh = 0;
+  const bool sbf = a.s_dt == MX_DTYPE_BFLOAT16, zbf = a.zp_dt == MX_DTYPE_BFLOAT16;
+  const int scol = P::kRow ? n0 / a.B : 0;
+  auto load_row_scale = [&](Block b) __attribute__((always_inline)) {
     if constexpr (P::kRow) {
-      if (t < kBK) {
-        const int64_t i = (int64_t)min(kb * kBK + t, K - 1) * a.nb + n0 / a.B;
-        rs = elem(a.scale, i, a.s_dt);
-        if (a.zp) rz = elem(a.zp, i, a.zp_dt);
-      }
+      const int64_t i = (int64_t)(b.k + (t & 31)) * a.nb + scol;
+      word(a.scale, i, sbf, rs, rssh);
+      if constexpr (P::kZp) word(a.zp, i, zbf, rz, rzsh);
     }
   };
-  auto store_row_scale = [&](int kb) __attribute__((always_inline)) {
+  auto store_row_scale = [&](int slot) __attribute__((always_inline)) {
     if constexpr (P::kRow) {
-      if (t < kBK) {
-        ring[kb & 1][0][t] = rs;
-        ring[kb & 1][1][t] = rz;
-      }
+      ring[slot][0][t & 31] = word_f32(rs, rssh, sbf);
+      if constexpr (P::kZp) ring[slot][1][t & 31] = word_f32(rz, rzsh, zbf);
     }
   };
 
-  f32x4_t acc[4][4];
+  f32x4_t acc[RB][4];
+  auto clear = [&]() __attribute__((always_inline)) {
 #pragma unroll
-  for (int i = 0; i < 4; ++i)
+    for (int i = 0; i < RB; ++i)
 #pragma unroll
-    for (int c = 0; c < 4; ++c) acc[i][c] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+      for (int c = 0; c < 4; ++c) acc[i][c] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+  };
+  clear();
   // One block: small products first.
   auto compute = [&](const char* buf) __attribute__((always_inline)) {
     const char* As = buf;
@@ -238,10 +277,10 @@ __global__ __launch_bounds__(kThreads, 2) void split_gemm_kernel(Args a) {
 #pragma unroll
       for (int c = 0; c < 4; ++c) B[p][c] = *(const u32x4_v*)(Bs + p * kPlane + chunk_at(c * 32 + 16 * wn + cg, kq));
 #pragma unroll
-    for (int rb = 0; rb < 4; ++rb) {
+    for (int rb = 0; rb < RB; ++rb) {
       u32x4_v A[PA];
 #pragma unroll
-      for (int p = 0; p < PA; ++p) A[p] = *(const u32x4_v*)(As + p * kPlane + chunk_at(64 * wm + 16 * rb + cg, kq));
+      for (int p = 0; p < PA; ++p) A[p] = *(const u32x4_v*)(As + p * kPlane + chunk_at(row0 + 16 * rb + cg, kq));
 #pragma unroll
       for (int order = PA + PB - 2; order >= 0; --order) {
         if (order > 2) continue;
@@ -256,57 +295,53 @@ __global__ __launch_bounds__(kThreads, 2) void split_gemm_kernel(Args a) {
     }
   };
 
+  using Whole = std::integral_constant<bool, false>;
+  using Tail = std::integral_constant<bool, true>;
   P src(a, t, n0);
   XRegs X;
   typename P::Regs W;
-  load_row_scale(kb0);
-  load_x(kb0, X);
-  src.load(a, kb0, W);
-  store_row_scale(kb0);
-  load_row_scale(kb0 + 1);
+  const int last = kb1 - 1;
+  auto block = [&](int kb) { return Block(min(kb, last), K); };  // requests past the slice repeat its last block
+  load_row_scale(block(kb0));
+  load_x(block(kb0), X);
+  src.load(a, block(kb0), W);
+  store_row_scale(0);
+  load_row_scale(block(kb0 + 1));
   __syncthreads();  // the table, the flag and block kb0's row scales are written
-  if constexpr (NBUF == 2) {
-    store_row_scale(kb0 + 1);
-    stage_x(kb0, X, sm[0]);
-    src.stage(a, kb0, W, table, sm[0] + PA * kPlane, odd);
+  store_row_scale(1);
+  stage_x(0, block(kb0), X, sm[0], Tail{});
+  src.stage(a, block(kb0), W, table, sm[0] + PA * kPlane, big, Tail{});
+  load_x(block(kb0 + 1), X);
+  src.load(a, block(kb0 + 1), W);
+  load_row_scale(block(kb0 + 2));
+  __syncthreads();
+  // One basic block per step, so that the conversions run under the MFMAs.
+  auto step = [&](int kb, auto tail) __attribute__((always_inline)) {
+    const int cur = (kb - kb0) & 1;
+    char* nxt = sm[cur ^ 1];
+    compute(sm[cur]);
+    stage_x(cur ^ 1, block(kb + 1), X, nxt, tail);
+    src.stage(a, block(kb + 1), W, table, nxt + PA * kPlane, big, tail);
+    load_x(block(kb + 2), X);
+    src.load(a, block(kb + 2), W);
+    store_row_scale(cur);
+    load_row_scale(block(kb + 3));
     __syncthreads();
+  };
+  const int whole = kb1 * kBK > K ? last - 1 : last;  // steps that stage a whole block
+  int kb = kb0;
 #pragma unroll 1
-    for (int kb = kb0; kb < kb1; ++kb) {
-      const int cur = (kb - kb0) & 1;
-      const bool more = kb + 1 < kb1;
-      if (more) {
-        load_x(kb + 1, X);
-        src.load(a, kb + 1, W);
-        load_row_scale(kb + 2);
-      }
-      compute(sm[cur]);
-      if (more) {
-        char* nxt = sm[NBUF == 2 ? cur ^ 1 : 0];
-        stage_x(kb + 1, X, nxt);
-        src.stage(a, kb + 1, W, table, nxt + PA * kPlane, odd);
-        store_row_scale(kb + 2);
-      }
-      __syncthreads();
-    }
-  } else {
-#pragma unroll 1
-    for (int kb = kb0; kb < kb1; ++kb) {
-      stage_x(kb, X, sm[0]);
-      src.stage(a, kb, W, table, sm[0] + PA * kPlane, odd);
-      __syncthreads();
-      if (kb + 1 < kb1) {
-        load_x(kb + 1, X);
-        src.load(a, kb + 1, W);
-      }
-      compute(sm[0]);
-      __syncthreads();
-    }
-  }
+  for (; kb < whole; ++kb) step(kb, Whole{});
+  if (kb < last) step(kb, Tail{});
+  compute(sm[(last - kb0) & 1]);
+  if (big > MX_SPLIT_MAX) flag = 1;
+  __syncthreads();
 
+  const int ncol = n0 + 64 * wn + 4 * cg;  // this lane's four columns
   if constexpr (P::kRow) {
-    if (a.zp) {  // x . zp of each row, added to all of its columns
+    if constexpr (P::kZp) {  // x . zp of each row, added to all of its columns
 #pragma unroll
-      for (int i = 0; i < 2; ++i) {
+      for (int i = 0; i < XR; ++i) {
         float z = zacc[i];
         z += __shfl_xor(z, 1);
         z += __shfl_xor(z, 2);
@@ -314,19 +349,18 @@ __global__ __launch_bounds__(kThreads, 2) void split_gemm_kernel(Args a) {
       }
       __syncthreads();
 #pragma unroll
-      for (int rb = 0; rb < 4; ++rb)
+      for (int rb = 0; rb < RB; ++rb)
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
-          const float z = zrow[64 * wm + 16 * rb + 4 * kq + r];
+          const float z = zrow[row0 + 16 * rb + 4 * kq + r];
 #pragma unroll
           for (int c = 0; c < 4; ++c) acc[rb][c][r] += z;
         }
     }
   }
-  const int ncol = n0 + 64 * wn + 4 * cg;
-  if (odd) {  // uniform over the workgroup
+  if (flag) {  // uniform over the workgroup
 #pragma unroll
-    for (int rb = 0; rb < 4; ++rb)
+    for (int rb = 0; rb < RB; ++rb)
 #pragma unroll
       for (int c = 0; c < 4; ++c) acc[rb][c] = f32x4_t{0.f, 0.f, 0.f, 0.f};
 #pragma unroll 1
@@ -335,10 +369,10 @@ __global__ __launch_bounds__(kThreads, 2) void split_gemm_kernel(Args a) {
 #pragma unroll
       for (int c = 0; c < 4; ++c) wv[c] = src.value(a, k, min(ncol + c, N - 1), table);
 #pragma unroll
-      for (int rb = 0; rb < 4; ++rb)
+      for (int rb = 0; rb < RB; ++rb)
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
-          const int m = min(m0 + 64 * wm + 16 * rb + 4 * kq + r, M - 1);
+          const int m = min(m0 + row0 + 16 * rb + 4 * kq + r, M - 1);
           const float xv = elem(a.x, (int64_t)m * K + k, P::kXbf ? MX_DTYPE_BFLOAT16 : MX_DTYPE_FLOAT32);
 #pragma unroll
           for (int c = 0; c < 4; ++c) acc[rb][c][r] = __builtin_fmaf(xv, wv[c], acc[rb][c][r]);
@@ -346,14 +380,14 @@ __global__ __launch_bounds__(kThreads, 2) void split_gemm_kernel(Args a) {
     }
   }
 
-  if (a.S > 1) {
+  if (sliced) {
     // Every slice stores its sums; the last to arrive at the tile adds them in slice order and goes
     // on to the epilogue.  Agent-scope coherent accesses (sc1): the slices may run on other XCDs.
     const __amdgpu_buffer_rsrc_t prs =
-        __builtin_amdgcn_make_buffer_rsrc(a.part + (size_t)tile * a.S * kBM * kBN, (short)0, a.S * kPartBytes, 0x00020000);
+        __builtin_amdgcn_make_buffer_rsrc(a.part + (size_t)(tile - a.whole) * a.S * kBM * kBN, (short)0, a.S * kPartBytes, 0x00020000);
     constexpr int kSc1 = 16;
 #pragma unroll
-    for (int rb = 0; rb < 4; ++rb)
+    for (int rb = 0; rb < RB; ++rb)
 #pragma unroll
       for (int c = 0; c < 4; ++c)
         __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4_v, acc[rb][c]), prs,
@@ -361,20 +395,20 @@ __global__ __launch_bounds__(kThreads, 2) void split_gemm_kernel(Args a) {
     __builtin_amdgcn_s_waitcnt(0);
     __syncthreads();
     if (t == 0) {
-      const uint32_t prev = __hip_atomic_fetch_add(&a.ctr[tile], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      if (prev + 1u == (uint32_t)a.S) __hip_atomic_store(&a.ctr[tile], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      odd = prev + 1u == (uint32_t)a.S;
+      const uint32_t prev = __hip_atomic_fetch_add(&a.ctr[tile - a.whole], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      if (prev + 1u == (uint32_t)a.S) __hip_atomic_store(&a.ctr[tile - a.whole], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      flag = prev + 1u == (uint32_t)a.S;
     }
     __syncthreads();
-    if (!odd) return;
+    if (!flag) return;
 #pragma unroll
-    for (int rb = 0; rb < 4; ++rb)
+    for (int rb = 0; rb < RB; ++rb)
 #pragma unroll
       for (int c = 0; c < 4; ++c) acc[rb][c] = f32x4_t{0.f, 0.f, 0.f, 0.f};
 #pragma unroll 1
     for (int s = 0; s < a.S; ++s) {
 #pragma unroll
-      for (int rb = 0; rb < 4; ++rb)
+      for (int rb = 0; rb < RB; ++rb)
 #pragma unroll
         for (int c = 0; c < 4; ++c)
           acc[rb][c] += __builtin_bit_cast(f32x4_t, __builtin_amdgcn_raw_buffer_load_b128(
@@ -389,15 +423,16 @@ __global__ __launch_bounds__(kThreads, 2) void split_gemm_kernel(Args a) {
   if (ncol < N) {
 #pragma unroll
     for (int c = 0; c < 4; ++c) {
-      if constexpr (P::kCol) cs[c] = elem(a.scale, ncol + c, a.s_dt);
-      if (a.bias) bi[c] = elem(a.bias, ncol + c, a.b_dt);
+      if constexpr (P::kCol) cs[c] = elem(a.scale, min(ncol + c, N - 1), a.s_dt);
+      if (a.bias) bi[c] = elem(a.bias, min(ncol + c, N - 1), a.b_dt);
     }
   }
   auto store4 = [&](int m, int n, const float (&y)[4]) __attribute__((always_inline)) {
     const int64_t o = (int64_t)m * N + n;
     if (!a.vec) {
 #pragma unroll
-      for (int c = 0; c < 4; ++c) store_f(a.out, o + c, P::kXbf ? MX_DTYPE_BFLOAT16 : MX_DTYPE_FLOAT32, y[c]);
+      for (int c = 0; c < 4; ++c)
+        if (n + c < N) store_f(a.out, o + c, P::kXbf ? MX_DTYPE_BFLOAT16 : MX_DTYPE_FLOAT32, y[c]);
     } else if constexpr (P::kXbf) {
       *(u32x2_v*)((uint16_t*)a.out + o) = u32x2_v{(uint32_t)f32_to_bf16(y[0]) | (uint32_t)f32_to_bf16(y[1]) << 16,
                                                   (uint32_t)f32_to_bf16(y[2]) | (uint32_t)f32_to_bf16(y[3]) << 16};
@@ -412,10 +447,10 @@ __global__ __launch_bounds__(kThreads, 2) void split_gemm_kernel(Args a) {
   if (a.act == MX_ACT_NONE) {
     if (ncol >= N) return;
 #pragma unroll
-    for (int rb = 0; rb < 4; ++rb)
+    for (int rb = 0; rb < RB; ++rb)
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
-        const int m = m0 + 64 * wm + 16 * rb + 4 * kq + r;
+        const int m = m0 + row0 + 16 * rb + 4 * kq + r;
         float y[4];
 #pragma unroll
         for (int c = 0; c < 4; ++c) y[c] = finish(acc[rb][c][r], c);
@@ -424,17 +459,17 @@ __global__ __launch_bounds__(kThreads, 2) void split_gemm_kernel(Args a) {
     return;
   }
   constexpr int kCS = kBN * 4;  // LDS bytes per row of a half tile
-  static_assert(64 * kCS <= NBUF * kBufBytes, "half a tile fits the LDS buffers");
+  static_assert(64 * kCS <= 2 * kBufBytes, "half a tile fits the LDS buffers");
   char* Cs = sm[0];
 #pragma unroll 1
   for (int half = 0; half < 2; ++half) {
     __syncthreads();
-    if (wm == half) {
+    if (row0 / 64 == half) {
 #pragma unroll
-      for (int rb = 0; rb < 4; ++rb)
+      for (int rb = 0; rb < RB; ++rb)
 #pragma unroll
         for (int r = 0; r < 4; ++r)
-          *(f32x4_t*)(Cs + (16 * rb + 4 * kq + r) * kCS + (64 * wn + 4 * cg) * 4) =
+          *(f32x4_t*)(Cs + (row0 % 64 + 16 * rb + 4 * kq + r) * kCS + (64 * wn + 4 * cg) * 4) =
               f32x4_t{finish(acc[rb][0][r], 0), finish(acc[rb][1][r], 1), finish(acc[rb][2][r], 2), finish(acc[rb][3][r], 3)};
     }
     __syncthreads();
@@ -452,27 +487,41 @@ __global__ __launch_bounds__(kThreads, 2) void split_gemm_kernel(Args a) {
   }
 }
 
-// Tiles, K slices and grid of a problem.  Tiles that leave CUs idle are split along K: as many
-// slices of at least eight blocks as fill the 256 CUs (planned whatever the device reports, so the
-// summation order depends on the shape alone) within kMaxParts partial tiles.
-inline int plan(mx_backend* b, Args& a, int64_t M, int* grid) {
+// Waves per workgroup, tail slices and grid of a problem (planned for 256 CUs whatever the device
+// reports, so the summation order depends on the shape alone).
+//   Below 256 tiles every tile is sliced along K, as many slices of at least eight blocks as fill
+//   the CUs.  One workgroup per CU then has eight waves, two per SIMD: x f32 [100,4096] x Int4
+//   [4096,11008] with 86 tiles in two slices 77 us with four waves, 68 us with eight.
+//   Past that, forms whose operands have at most four parts in all run two workgroups of four waves
+//   per CU (64 KB of LDS each; [2048,4096] x [4096,11008] 603 us, 793 us with eight waves), the
+//   others one of eight waves (96 KB).  Tiles past the last whole round of resident workgroups are
+//   sliced if the slices fit one round: 258 tiles of GGML Q6_K rows (x [333,4096], N = 11008) took
+//   357 us in two rounds, 214 us with the last two tiles in 16 slices each.
+inline int plan(mx_backend* b, Args& a, int64_t M, int parts, int* nw, int* grid) {
   const int64_t tiles_n = (a.N + kBN - 1) / kBN, tiles = ((M + kBM - 1) / kBM) * tiles_n;
   if (tiles >= (int64_t)1 << 28) return set_error(MX_ERR_INVALID, "FusedQuantizedDense: M=%lld too large", (long long)M);
   const int blocks = (a.K + kBK - 1) / kBK;
-  int S = 1;
-  if (tiles <= kMaxParts / 2) S = (int)std::max<int64_t>(1, std::min<int64_t>(kMaxParts / tiles, blocks / 8));
-  a.kpb = (blocks + S - 1) / S;
+  *nw = parts > 4 || tiles < 256 ? 8 : 4;
+  const int64_t round = tiles < 256 || *nw == 8 ? 256 : 512;
+  a.whole = (int)(tiles / round * round);
+  const int64_t tail = tiles - a.whole;
+  int64_t S = 1;
+  if (tail > 0) {
+    S = std::max<int64_t>(1, std::min<int64_t>((a.whole ? round : kMaxParts) / tail, blocks / 8));
+    if (a.whole && b->noalloc_active && tail * S > kMaxParts) S = std::max<int64_t>(1, kMaxParts / tail);
+  }
+  a.kpb = (int)((blocks + S - 1) / S);
   a.S = (blocks + a.kpb - 1) / a.kpb;
   a.tiles_n = (int)tiles_n;
-  a.items = (int)tiles * a.S;
-  a.per_xcd = (a.items + 7) / 8;
-  *grid = 8 * a.per_xcd;
-  a.vec = (uintptr_t)a.out % 16 == 0;
+  a.tail = (int)tail * a.S;
+  a.per_xcd = (a.tail + 7) / 8;
+  *grid = a.whole + 8 * a.per_xcd;
+  a.vec = (uintptr_t)a.out % 16 == 0 && a.N % 4 == 0;
   a.part = nullptr;
   a.ctr = nullptr;
   if (a.S > 1) {
     void* scratch = nullptr;
-    MX_TRY(ensure_scratch(b, kCounterBytes + (size_t)a.items * kPartBytes, &scratch));
+    MX_TRY(ensure_scratch(b, kCounterBytes + (size_t)a.tail * kPartBytes, &scratch));
     a.ctr = (uint32_t*)scratch;
     a.part = (float*)((char*)scratch + kCounterBytes);
   }

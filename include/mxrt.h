@@ -155,7 +155,7 @@ typedef uint64_t mx_value;
  * quantizeddense.go:586-650 at every size).  Without "exact", decode and prefill shapes take the
  * fast kernels.  The bf16-x kernels (skinny, prefill GEMM) and the decode GEMV differ from the
  * reference only in summation order.  The prefill plans of the reference layout, f32 x, zero
- * points and NF4 (past 64 rows), and of GGML rows (past 20 rows), also round each term's weight
+ * points and NF4 (past 64 rows), and of GGML rows (past 16 rows), also round each term's weight
  * factor w*s (or w*s+zp) before the product with x (with at least 128 columns per scale block: the
  * factor x*s before the product with w), where the reference rounds (x*w)*s; they
  * stay within the f32 accumulation bound of the reference's sum.  Below the fast kernels'
@@ -414,11 +414,11 @@ int mx_qdense_plan(mx_backend* b, const mx_qdense_args* args, char* buf, size_t 
  * hipMalloc). The split-K partial sums and arrival counters live in a static device array of
  * MX_QDENSE_NOALLOC_SCRATCH_BYTES per GPU, set up by mx_backend_new and held until the process
  * ends; a problem whose split-K needs more returns MX_ERR_INVALID before anything is launched.
- * Results are bit-identical to mx_qdense's, except for GGML rows past 20 rows, which mx_qdense
- * dequantises into an f32 copy: they run the decode GEMV once per group of four rows, and for
- * prefill GEMMs whose last partial round of tiles mx_qdense splits into two K halves (at most 128
- * tiles past a multiple of 256): those tiles are summed whole here (both within the f32
- * accumulation bound of the reference's sum). Every call on one GPU
+ * Results are bit-identical to mx_qdense's, except where mx_qdense splits the last partial round
+ * of a prefill's tiles along K into more partial tiles than the array holds (bf16 GEMM: at most 128
+ * tiles past a multiple of 256, in two halves; GGML, reference-layout and f32 x prefills: at most
+ * half a round of 256 or 512 tiles past whole rounds): those tiles are summed in fewer slices or
+ * whole here (within the f32 accumulation bound of the reference's sum). Every call on one GPU
  * shares the array, from any backend; the calls are ordered on the device (each call's stream
  * waits for the previous call's completion event), so calls from several streams or backends run
  * one after another.  Under graph capture that wait cannot be recorded: the caller must keep a

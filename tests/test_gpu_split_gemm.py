@@ -115,3 +115,36 @@ def test_output_aligned_to_its_elements_only(backend, x_dtype, act):
     backend.QDense(a)
     got = out.ToFlatData()
     assert got[0] == 0 and np.array_equal(got[1:].reshape(p.M, p.N), want)
+
+
+@pytest.mark.parametrize("M,N", [(300, 11008), (1100, 7296)])
+def test_tail_tiles_in_slices(backend, M, N):
+    """Tiles past whole rounds of resident workgroups: 258 tiles of the weight form (256 + 2), 513 of
+    the row form (512 + 1), the last ones in K slices; rows of the first and of the last tiles."""
+    p = O.make_problem(M, 512, N, w_dtype=O.DT_INT8, x_dtype=F32, scale_dtype=F32, block_axis=1, block_size=64 if M == 300 else 128,
+                       bias=True, seed=M)
+    r = QDenseRun(backend, p)
+    y = r.run()
+    rows = np.r_[0:4, M - 44:M]
+    truth, scale = O.qdense_f64(p, rows), O.qdense_f64(p, rows, absolute=True)
+    assert np.all(np.abs(y[rows].astype(np.float64) - truth) <= 2.0 ** -22 * np.abs(truth) + 1e-5 * scale)
+    assert np.array_equal(y, r.run())
+
+
+@pytest.mark.parametrize("t", [ca.GGMLQ4_0, ca.GGMLQ8_0, ca.GGMLIQ4NL, ca.GGMLQ4_K, ca.GGMLQ6_K])
+@pytest.mark.parametrize("M,K,N", [(17, 1024, 1031), (129, 2048, 130)])
+def test_ggml_rows_at_ragged_edges(backend, t, M, K, N):
+    """GGML rows past 16 rows: odd output widths (scalar stores) and one row past a tile."""
+    rng = np.random.default_rng(M + int(t))
+    w = O.ggml_random_rows(int(t), N, K, rng)
+    x = rng.standard_normal((M, K)).astype(np.float32)
+    up = lambda v, s: backend.BufferFromFlatData(0, np.ascontiguousarray(v).ravel(), s)
+    out = up(np.zeros(M * N, np.float32), ca.Shape(ca.Float32, M, N))
+    bufs = [up(x, ca.Shape(ca.Float32, M, K)), up(w, ca.Shape(ca.Uint8, *w.shape))]
+    a = ca._lib.mx_qdense_args()
+    a.x, a.w, a.out = bufs[0].DevicePtr(), bufs[1].DevicePtr(), out.DevicePtr()
+    a.M, a.K, a.N, a.x_dtype, a.scheme, a.ggml_type = M, K, N, F32, int(ca.QuantGGML), int(t)
+    assert backend.QDensePlan(a) == "ggml_dequant_f32_mfma"
+    backend.QDense(a)
+    exact, ab = O.ggml_dense_f64(x, w, int(t), None)
+    assert np.all(np.abs(out.ToFlatData().reshape(M, N).astype(np.float64) - exact) <= 1e-5 * ab + 1e-30)
