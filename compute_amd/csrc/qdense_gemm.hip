@@ -12,8 +12,8 @@
 // (acc += accg * s[g]): with bf16 scales after every 64-row block (its first MFMAs start from
 // zero, so nothing is cleared), with f32 scales at the group's last block.
 //
-// Tiling.  A workgroup (8 waves, two per SIMD) computes a 256 x 128 output tile; wave w owns
-// rows [64 wr, 64 wr + 64) x columns [64 wc, 64 wc + 64) with wr = w % 4, wc = w / 4.  K advances
+// Tiling.  A workgroup (8 waves, two per SIMD) computes a 256 x 128 output tile (or, RB = 2, 128 x
+// 128 with 32 rows per wave: gemm_plan); wave w owns rows [64 wr, 64 wr + 64) x columns [64 wc, 64 wc + 64) with wr = w % 4, wc = w / 4.  K advances
 // in blocks of 64 (two 32-row steps of v_mfma_f32_16x16x32_bf16).  LDS holds
 //   - x, four buffers (three with f32 group scales): [256 rows][64 k] bf16; 16-byte k-chunks XOR-swizzled within each row by
 //     (row >> 1) & 7 so that an MFMA operand read (16 rows) hits distinct banks;
@@ -54,8 +54,10 @@ typedef __attribute__((__vector_size__(8 * sizeof(_Float16)))) _Float16 f16x8_t;
 typedef __attribute__((__vector_size__(4 * sizeof(float)))) float f32x4_t;
 typedef uint32_t u32x4_v __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x2_v __attribute__((ext_vector_type(2)));
-constexpr int kBM = 256, kBN = 128, kBK = 64, kWaves = 8, kThreads = 64 * kWaves;
-constexpr int kABytes = kBM * kBK * 2;   // 32 KB per x buffer
+constexpr int kBN = 128, kBK = 64, kWaves = 8, kThreads = 64 * kWaves;
+// RB: 16-row blocks per wave; the tile is 64 RB rows (4: 256, 2: 128).
+template <int RB> constexpr int kBM = 64 * RB;
+template <int RB> constexpr int kABytes = kBM<RB> * kBK * 2;  // 32 or 16 KB per x buffer
 constexpr int kBtBytes = kBN * kBK * 2;  // 16 KB per Bt buffer
 // x buffers: a block's rows are requested kXBufs - 1 blocks ahead of its use.  Four (160 KB of
 // LDS with the two Bt buffers) except for f32 group scales, whose run-time group branch leaves no
@@ -63,12 +65,11 @@ constexpr int kBtBytes = kBN * kBK * 2;  // 16 KB per Bt buffer
 // per call with four; C4 unchanged.
 template <int BK, bool GRP, bool FB>
 constexpr int kXBufs = (GRP && !FB) ? 3 : 4;
-constexpr int kXDma = kABytes / (kWaves * 1024);     // 1 KB direct-to-LDS loads per wave per block
+template <int RB> constexpr int kXDmaOf = kABytes<RB> / (kWaves * 1024);  // 1 KB direct-to-LDS loads per wave per block
 constexpr int kWLoads = 4;                           // w loads (one per row) per thread per block
 constexpr int kPf = 4;                               // w blocks loaded ahead into registers
 constexpr int kUnroll = 4;                           // multiple of kPf and of the 2 Bt buffers
 constexpr int64_t kSplitPlanCUs = 256;               // CUs the split tail is planned for (MI355X)
-static_assert(kXDma * kWaves * 1024 == kABytes, "x load split");
 static_assert(kBK * kBN == 16 * kThreads, "conversion: 16 weights per thread");
 
 // B operand kinds: the quantized weights [K, N] (int8 / uint8, converted to bf16), or a
@@ -87,14 +88,14 @@ struct GemmArgs {
   void* out;          // [M, N] bf16 (quantized) or [batch][M, N] f32 / bf16 / f16 (DotGeneral)
   int M, K, N, s_dt, b_dt, act, tiles_n, grouped, tiles, out_dt;
   int gpb;            // blocks of 64 K rows per scale group (grouped scales; scale is [K/G, N])
-  // Split tail (quantized kernels): work items [0, split_from) are whole tiles; the last
-  // (gridDim.x - split_from) / 2 tiles are computed as two halves of K each, by consecutive
-  // workgroups, which exchange f32 partial tiles through `part` (scratch) and count arrivals in
-  // `ctr` (zero between launches); the second to arrive adds the halves (half 0 + half 1) and
+  // Split tiles (quantized kernels): work items [0, split_from) are whole tiles; the remaining tiles
+  // are computed in S slices of K each (kpb blocks of 64 rows, the last may be shorter), by
+  // consecutive workgroups, which exchange f32 partial tiles through `part` (scratch) and count
+  // arrivals in `ctr` (zero between launches); the last to arrive adds the slices in order and
   // stores the tile.  split_from == gridDim.x: no split.
-  int split_from;
-  float* part;        // [tail tiles][2 halves][16][512 threads][4] f32
-  uint32_t* ctr;      // [tail tiles]
+  int split_from, S, kpb;
+  float* part;        // [split tiles][S][4 RB][512 threads][4] f32
+  uint32_t* ctr;      // [split tiles]
 };
 
 template <int BK>
@@ -169,11 +170,11 @@ __device__ __forceinline__ uint32_t scaled_act_bf16x2(float v0, float s0, float 
 // Epilogue of one lane: scale, bias, activation, bf16, 8-byte stores of 4 consecutive columns
 // per row.  The activation is a template parameter so that each variant is straight-line code
 // (no calls, which would save and restore the live accumulators around every one).
-template <int ACT>
-__device__ __forceinline__ void store_tile(const f32x4_t (&acc)[4][4], const float (&sc)[4], const float (&bi)[4],
+template <int ACT, int RB>
+__device__ __forceinline__ void store_tile(const f32x4_t (&acc)[RB][4], const float (&sc)[4], const float (&bi)[4],
                                            uint16_t* out, int row0, int M, size_t N, int ncol) {
 #pragma unroll
-  for (int rb = 0; rb < 4; ++rb) {
+  for (int rb = 0; rb < RB; ++rb) {
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
       const int row = row0 + 16 * rb + r;
@@ -195,14 +196,12 @@ __device__ __forceinline__ void store_tile(const f32x4_t (&acc)[4][4], const flo
 // H (with FB): scale groups of 32 rows, two per 64-row block: each step's sums start from zero and
 // are folded with their own group's scales (after step 0 and at the block's end); HF: those
 // scales in f32 (else bf16).
-template <int BK, bool GRP, bool FB = false, bool H = false, bool HF = false>
+template <int BK, int RB, bool GRP, bool FB = false, bool H = false, bool HF = false>
 __global__ __launch_bounds__(kThreads) void qdense_gemm_kernel(GemmArgs a) {
   static_assert(!H || (GRP && FB), "32-row groups: the fold-every-step form");
   static_assert(!HF || H, "f32 scales for 32-row groups only");
   constexpr int PF = kPf;
-  // With scale groups the tile is 256 x 64: each wave keeps two of the four interleaved MFMA
-  // column sets (columns 4*cg + 2*wc + c, c = 0, 1), which halves both accumulator sets so that
-  // the second one fits beside the operands without spilling.
+  constexpr int kXDma = kXDmaOf<RB>;
   constexpr int BN = kBN;
   constexpr int NC = 4;  // MFMA column sets per wave
   static_assert(kUnroll % PF == 0, "register slots cycle within the unroll");
@@ -211,12 +210,15 @@ __global__ __launch_bounds__(kThreads) void qdense_gemm_kernel(GemmArgs a) {
   // batches are consecutive runs of items.
   const int bid = blockIdx.x;
   const int whole = a.split_from;  // whole-tile work items (dispatched first)
-  int item, half = -1;
+  int item, slice = -1;
   if (bid < whole) {
     item = (whole & 7) == 0 ? (bid & 7) * (whole >> 3) + (bid >> 3) : bid;
   } else {
-    item = whole + ((bid - whole) >> 1);
-    half = (bid - whole) & 1;
+    int j = bid - whole;
+    const int n = (int)gridDim.x - whole;
+    if (whole == 0 && (n & 7) == 0) j = (j & 7) * (n >> 3) + (j >> 3);
+    item = whole + j / a.S;
+    slice = j - (item - whole) * a.S;
   }
   const int batch = item / a.tiles;
   item -= batch * a.tiles;
@@ -234,28 +236,28 @@ __global__ __launch_bounds__(kThreads) void qdense_gemm_kernel(GemmArgs a) {
     tm = item / a.tiles_n;
     tn = item % a.tiles_n;
   }
-  const int m0 = tm * kBM, n0 = tn * BN;
+  const int m0 = tm * kBM<RB>, n0 = tn * BN;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
   const int wr = wave & 3, wc = wave >> 2;
   const int cg = lane & 15, kq = lane >> 4;
   const size_t N = (size_t)a.N;
   const int lda = a.K;  // x row stride
   if constexpr (!kDotB<BK>) {
-    if (half >= 0) {
-      // This workgroup's half of K: the operands start at its first 64-row block (a whole
-      // number of scale groups, checked by the host) and K is the half's extent.
-      const int kbeg = half * (a.K / kBK / 2);
+    if (slice >= 0) {
+      // This workgroup's slice of K: the operands start at its first 64-row block (a whole
+      // number of scale groups, checked by the host) and K is the slice's extent.
+      const int kbeg = slice * a.kpb;
       a.x += (size_t)kbeg * kBK;
       a.w += k4B<BK> ? (size_t)kbeg * kBK * N / 2 : (size_t)kbeg * kBK * N;
       if (a.gpb > 0)
         a.scale = (const char*)a.scale + (size_t)(kbeg / a.gpb) * (H ? 2 : 1) * N * (a.s_dt == MX_DTYPE_FLOAT32 ? 4 : 2);
-      a.K /= 2;
+      a.K = min(a.kpb * kBK, a.K - kbeg * kBK);
     }
   }
   const int KB = a.K / kBK;
 
   constexpr int XB = kXBufs<BK, GRP, FB>;
-  __shared__ __attribute__((aligned(16))) uint8_t xs[XB][kABytes];
+  __shared__ __attribute__((aligned(16))) uint8_t xs[XB][kABytes<RB>];
   __shared__ __attribute__((aligned(16))) uint8_t bt[2][kBtBytes];
 
   // x: each wave moves kXDma 1 KB pieces of a block straight into LDS: piece q = kXDma*wave + i
@@ -271,7 +273,7 @@ __global__ __launch_bounds__(kThreads) void qdense_gemm_kernel(GemmArgs a) {
   }
   const uint32_t xs_lds = lds_addr(&xs[0][0]) + (uint32_t)(kXDma * wave) * 1024u;
   auto dma_x = [&](int kb) {
-    const uint32_t dst = xs_lds + (uint32_t)(kb % XB) * kABytes;
+    const uint32_t dst = xs_lds + (uint32_t)(kb % XB) * kABytes<RB>;
     kb = min(kb, KB - 1);
 #pragma unroll
     for (int i = 0; i < kXDma; ++i) lds_dma_b128(a.x + (size_t)kb * kBK, xoff[i], dst + 1024u * i);
@@ -370,9 +372,9 @@ __global__ __launch_bounds__(kThreads) void qdense_gemm_kernel(GemmArgs a) {
   };
 
   // acc: the total; accg: the current scale group's sums (grouped scales only).
-  f32x4_t acc[4][NC], accg[4][NC];
+  f32x4_t acc[RB][NC], accg[RB][NC];
 #pragma unroll
-  for (int rb = 0; rb < 4; ++rb)
+  for (int rb = 0; rb < RB; ++rb)
 #pragma unroll
     for (int c = 0; c < NC; ++c) acc[rb][c] = accg[rb][c] = f32x4_t{0.f, 0.f, 0.f, 0.f};
   // Grouped scales: this lane's 4 columns' scales of the group being summed, loaded a group ahead.
@@ -407,22 +409,22 @@ __global__ __launch_bounds__(kThreads) void qdense_gemm_kernel(GemmArgs a) {
 
   // MFMA operands of one 32-row step: x row 64*wr + 16*rb + cg, Bt column 64*wc + 4*cg + c (Bt
   // row 64*wc + 4*cg + (c ^ (cg & 1))); with groups, Bt column 4*cg + 2*wc + c.
-  const uint32_t a_row = (uint32_t)((64 * wr + cg) * (kBK * 2));
+  const uint32_t a_row = (uint32_t)((16 * RB * wr + cg) * (kBK * 2));
   const uint32_t b_col = (uint32_t)((64 * wc + 4 * cg) * (kBK * 2));
   const int b_par = cg & 1;
   // Operands of one 32-row step (sub = 0, 1 of a block) from LDS buffer buf, and its 16 MFMAs.
-  auto read_step = [&](int xbuf, int buf, int sub, u32x4_v (&A)[4], u32x4_v (&B)[NC]) {
+  auto read_step = [&](int xbuf, int buf, int sub, u32x4_v (&A)[RB], u32x4_v (&B)[NC]) {
     const int kc = 4 * sub + kq;  // 16-byte k-chunk of this lane
     const uint8_t* ap = &xs[xbuf][a_row + ((kc ^ (cg >> 1)) << 4)];
     const uint8_t* bp = &bt[buf][b_col + ((kc ^ ((cg >> 1) & 7)) << 4)];
 #pragma unroll
-    for (int rb = 0; rb < 4; ++rb) A[rb] = *(const u32x4_v*)(ap + rb * 16 * (kBK * 2));
+    for (int rb = 0; rb < RB; ++rb) A[rb] = *(const u32x4_v*)(ap + rb * 16 * (kBK * 2));
 #pragma unroll
     for (int c = 0; c < NC; ++c) B[c] = *(const u32x4_v*)(bp + (c ^ b_par) * (kBK * 2));
   };
-  auto mma_step = [&](const u32x4_v (&A)[4], const u32x4_v (&B)[NC], auto fresh) __attribute__((always_inline)) {
+  auto mma_step = [&](const u32x4_v (&A)[RB], const u32x4_v (&B)[NC], auto fresh) __attribute__((always_inline)) {
 #pragma unroll
-    for (int rb = 0; rb < 4; ++rb)
+    for (int rb = 0; rb < RB; ++rb)
 #pragma unroll
       for (int c = 0; c < NC; ++c) {
         if constexpr (GRP && decltype(fresh)::value)
@@ -447,7 +449,7 @@ __global__ __launch_bounds__(kThreads) void qdense_gemm_kernel(GemmArgs a) {
       sg[3] = __uint_as_float(w[1] & 0xFFFF0000u);
     }
 #pragma unroll
-    for (int rb = 0; rb < 4; ++rb)
+    for (int rb = 0; rb < RB; ++rb)
 #pragma unroll
       for (int c = 0; c < NC; ++c) {
 #pragma unroll
@@ -477,7 +479,7 @@ __global__ __launch_bounds__(kThreads) void qdense_gemm_kernel(GemmArgs a) {
   constexpr int kWGl = kNKB<BK> ? kNKLoads : kWLoads;
   static_assert(PF >= 3 && kUnroll % PF == 0, "a block's weights are converted two blocks after their load");
   uint32_t wr4[PF][kWWords];
-  u32x4_v A0[4], B0[NC], A1[4], B1[NC];
+  u32x4_v A0[RB], B0[NC], A1[RB], B1[NC];
   int g_left = a.gpb, g_idx = 0;  // scale groups: blocks left in the current group, its index
   auto block = [&](int kb, auto step) __attribute__((always_inline)) {
     constexpr int U = decltype(step)::value;  // kb % kUnroll
@@ -489,7 +491,7 @@ __global__ __launch_bounds__(kThreads) void qdense_gemm_kernel(GemmArgs a) {
     read_step(xb, B, 1, A1, B1);
     mma_step(A0, B0, Fresh{});
 #pragma unroll
-    for (int i = 0; i < 4 + NC; ++i) {
+    for (int i = 0; i < RB + NC; ++i) {
       __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);  // DS read
       __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);  // MFMA
     }
@@ -506,7 +508,7 @@ __global__ __launch_bounds__(kThreads) void qdense_gemm_kernel(GemmArgs a) {
     dma_x(kb + XB);
     mma_step(A1, B1, std::integral_constant<bool, H>{});  // H: the second group starts from zero
 #pragma unroll
-    for (int i = 0; i < 4 + NC; ++i) {
+    for (int i = 0; i < RB + NC; ++i) {
       __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);  // DS read
       __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);  // MFMA
     }
@@ -560,42 +562,54 @@ __global__ __launch_bounds__(kThreads) void qdense_gemm_kernel(GemmArgs a) {
   blocks(kb, KB - kb, I0{}, I1{}, I2{});
 
   if constexpr (!kDotB<BK>) {
-    if (half >= 0) {
-      // Split tail: store this half's sums, count the arrival; the second to arrive adds the
-      // other half's sums in the order half 0 + half 1 and goes on to the epilogue.  The partial
-      // tiles are stored and loaded with the agent-scope coherence bit (sc1); the two halves run
-      // on different XCDs.
+    if (slice >= 0) {
+      // Split tile: store this slice's sums, count the arrival; the last to arrive adds the slices'
+      // sums in order and goes on to the epilogue.  The partial tiles are stored and loaded with the
+      // agent-scope coherence bit (sc1); the slices may run on different XCDs.
       // The arrival flag takes the first word of a Bt buffer: every wave has left the main loop
       // (the barrier below comes first), and four x buffers leave no LDS beyond the two.
       int& s_last = *(int*)&bt[0][0];
-      const int tt = item - whole;  // tail tile
+      const int tt = item - whole;  // split tile
+      constexpr int kSlice = 4 * RB * kThreads * 16;
       const __amdgpu_buffer_rsrc_t prs = __builtin_amdgcn_make_buffer_rsrc(
-          a.part + (size_t)tt * 2 * 16 * kThreads * 4, (short)0, 2 * 16 * kThreads * 16, 0x00020000);
+          (char*)a.part + (size_t)tt * a.S * kSlice, (short)0, a.S * kSlice, 0x00020000);
       constexpr int kSc1 = 16;
 #pragma unroll
-      for (int rb = 0; rb < 4; ++rb)
+      for (int rb = 0; rb < RB; ++rb)
 #pragma unroll
         for (int c = 0; c < NC; ++c)
           __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4_v, acc[rb][c]), prs,
-                                                (unsigned)(((half * 16 + 4 * rb + c) * kThreads + t) * 16), 0, kSc1);
+                                                (unsigned)(slice * kSlice + ((4 * rb + c) * kThreads + t) * 16), 0, kSc1);
       __builtin_amdgcn_s_waitcnt(0);
       __syncthreads();
       if (t == 0) {
         const uint32_t prev = __hip_atomic_fetch_add(&a.ctr[tt], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        if (prev == 1u) __hip_atomic_store(&a.ctr[tt], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        s_last = prev == 1u;
+        const bool last = prev + 1u == (uint32_t)a.S;
+        if (last) __hip_atomic_store(&a.ctr[tt], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        s_last = last;
       }
       __syncthreads();
       if (!s_last) return;
-      const int other = half ^ 1;
+      auto load = [&](int sl, int rb, int c) {
+        return __builtin_bit_cast(f32x4_t, __builtin_amdgcn_raw_buffer_load_b128(
+                                               prs, (unsigned)(sl * kSlice + ((4 * rb + c) * kThreads + t) * 16), 0, kSc1));
+      };
+      if (a.S == 2) {  // a sum of two is the same in either order
 #pragma unroll
-      for (int rb = 0; rb < 4; ++rb)
+        for (int rb = 0; rb < RB; ++rb)
 #pragma unroll
-        for (int c = 0; c < NC; ++c) {
-          const f32x4_t o = __builtin_bit_cast(f32x4_t, __builtin_amdgcn_raw_buffer_load_b128(
-                                                            prs, (unsigned)(((other * 16 + 4 * rb + c) * kThreads + t) * 16), 0, kSc1));
-          acc[rb][c] = half == 0 ? acc[rb][c] + o : o + acc[rb][c];
-        }
+          for (int c = 0; c < NC; ++c) acc[rb][c] += load(slice ^ 1, rb, c);
+      } else {
+#pragma unroll 1
+        for (int sl = 0; sl < a.S; ++sl)
+#pragma unroll
+          for (int rb = 0; rb < RB; ++rb)
+#pragma unroll
+            for (int c = 0; c < NC; ++c) {
+              const f32x4_t o = load(sl, rb, c);
+              acc[rb][c] = sl == 0 ? o : acc[rb][c] + o;
+            }
+      }
     }
   }
 
@@ -604,9 +618,9 @@ __global__ __launch_bounds__(kThreads) void qdense_gemm_kernel(GemmArgs a) {
   const int ncol = lcol;
   if (ncol >= a.N) return;
   if constexpr (kDotB<BK>) {
-    const int r0 = m0 + 64 * wr + 4 * kq;
+    const int r0 = m0 + 16 * RB * wr + 4 * kq;
 #pragma unroll
-    for (int rb = 0; rb < 4; ++rb)
+    for (int rb = 0; rb < RB; ++rb)
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
         const int row = r0 + 16 * rb + r;
@@ -630,15 +644,15 @@ __global__ __launch_bounds__(kThreads) void qdense_gemm_kernel(GemmArgs a) {
       sc[c] = GRP ? 1.0f : load_f(a.scale, ncol + c, a.s_dt);  // grouped: applied by fold()
       bi[c] = a.bias ? load_f(a.bias, ncol + c, a.b_dt) : 0.0f;
     }
-    const int row0 = m0 + 64 * wr + 4 * kq;
+    const int row0 = m0 + 16 * RB * wr + 4 * kq;
     uint16_t* out = (uint16_t*)a.out;
     switch (a.act) {
-      case MX_ACT_GELU: store_tile<MX_ACT_GELU>(acc, sc, bi, out, row0, a.M, N, ncol); break;
-      case MX_ACT_RELU: store_tile<MX_ACT_RELU>(acc, sc, bi, out, row0, a.M, N, ncol); break;
-      case MX_ACT_SILU: store_tile<MX_ACT_SILU>(acc, sc, bi, out, row0, a.M, N, ncol); break;
-      case MX_ACT_HARDSWISH: store_tile<MX_ACT_HARDSWISH>(acc, sc, bi, out, row0, a.M, N, ncol); break;
-      case MX_ACT_TANH: store_tile<MX_ACT_TANH>(acc, sc, bi, out, row0, a.M, N, ncol); break;
-      default: store_tile<MX_ACT_NONE>(acc, sc, bi, out, row0, a.M, N, ncol); break;
+      case MX_ACT_GELU: store_tile<MX_ACT_GELU, RB>(acc, sc, bi, out, row0, a.M, N, ncol); break;
+      case MX_ACT_RELU: store_tile<MX_ACT_RELU, RB>(acc, sc, bi, out, row0, a.M, N, ncol); break;
+      case MX_ACT_SILU: store_tile<MX_ACT_SILU, RB>(acc, sc, bi, out, row0, a.M, N, ncol); break;
+      case MX_ACT_HARDSWISH: store_tile<MX_ACT_HARDSWISH, RB>(acc, sc, bi, out, row0, a.M, N, ncol); break;
+      case MX_ACT_TANH: store_tile<MX_ACT_TANH, RB>(acc, sc, bi, out, row0, a.M, N, ncol); break;
+      default: store_tile<MX_ACT_NONE, RB>(acc, sc, bi, out, row0, a.M, N, ncol); break;
     }
   }
 }
@@ -662,6 +676,53 @@ bool qdense_gemm_fits(const QDenseDesc& d) {
          aligned(d.out, 16);
 }
 
+// Tile rows, whole tiles and K slices of a quantized problem (planned for MI355X's 256 CUs whatever
+// the device reports, so the summation order depends on the shape only).  One workgroup is resident
+// per CU, so a launch takes whole rounds of 256 tiles: tiles past the last whole round are cut into
+// K slices that fill one round, and both tile heights are priced, in tenths of a 256-row tile's
+// 64-row block (1.4 us with scale groups, 0.85 us per channel; a 128-row tile's is 0.8 of it), with
+// what the slices' completion was measured to add.  x [97,4096] x [4096,14336] Int4 g128 89 -> 42 us
+// (112 tiles of 128 rows in two slices, was 112 of 256 rows), [97,14336] x 4096 294 -> 43 (7 slices),
+// [512,4096] x 4096 91 -> 42, [512,14336] x 4096 303 -> 96 (256-row tiles in four slices); int8 per
+// channel [256,4096] x 4096 57 -> 25; shapes that fill the CUs keep the 256-row tiles (1333 rows,
+// N = 14336: 271 us against 345 with 128-row tiles).
+struct GemmPlan {
+  int rb;                    // 4: 256-row tiles, 2: 128-row tiles
+  int64_t tiles_m, tiles_n;
+  int64_t whole, S, kpb;     // whole tiles; slices of the others and their blocks of K
+};
+
+static GemmPlan gemm_plan(int64_t M, int64_t K, int64_t N, int64_t gpb, bool noalloc) {
+  const int64_t KB = K / kBK;
+  auto plan = [&](int rb, int64_t* cost) {
+    GemmPlan p{};
+    p.rb = rb;
+    p.tiles_m = (M + 64 * rb - 1) / (64 * rb);
+    p.tiles_n = (N + kBN - 1) / kBN;
+    const int64_t tiles = p.tiles_m * p.tiles_n, tail = tiles % kSplitPlanCUs;
+    p.whole = tiles;
+    p.S = 1;
+    p.kpb = KB;
+    const int64_t c = rb == 4 ? 10 : 8;
+    *cost = (tiles + kSplitPlanCUs - 1) / kSplitPlanCUs * KB * c;
+    if (tail == 0) return p;
+    const int64_t room = (noalloc ? MX_QDENSE_NOALLOC_SCRATCH_BYTES - 64 * 1024 : 32 << 20) / (tail * 64 * rb * kBN * 4);
+    const int64_t S = std::min({kSplitPlanCUs / tail, room, KB / 4});
+    if (S < 2) return p;
+    const int64_t kpb = ((KB + S - 1) / S + gpb - 1) / gpb * gpb;
+    const int64_t split = tiles / kSplitPlanCUs * KB * c + kpb * c + (rb == 4 ? 160 : 40);
+    if (kpb >= KB || split >= *cost) return p;
+    *cost = split;
+    p.kpb = kpb;
+    p.S = (KB + kpb - 1) / kpb;
+    p.whole = tiles - tail;
+    return p;
+  };
+  int64_t c4, c2;
+  const GemmPlan p4 = plan(4, &c4), p2 = plan(2, &c2);
+  return c2 < c4 ? p2 : p4;
+}
+
 int qdense_gemm_run(mx_backend* b, const QDenseDesc& d, const char* name) {
   GemmArgs ga;
   ga.x = (const uint16_t*)d.x;
@@ -676,67 +737,53 @@ int qdense_gemm_run(mx_backend* b, const QDenseDesc& d, const char* name) {
   ga.b_dt = d.b_dt;
   ga.act = d.act;
   const bool grouped = d.block_size < d.K;
-  // The kernel's tile width: 64 for 4-bit weights with scale groups.
-  const int64_t bn = kBN;
-  const int64_t tiles_m = (d.M + kBM - 1) / kBM, tiles_n = (d.N + bn - 1) / bn;
-  if (tiles_m * tiles_n > (int64_t)1 << 30)
-    return set_error(MX_ERR_INVALID, "FusedQuantizedDense: output too large for the GEMM path");
-  ga.tiles_n = (int)tiles_n;
-  ga.grouped = (tiles_m % 2 == 0 && tiles_n % 16 == 0) ? 1 : 0;
-  ga.tiles = (int)(tiles_m * tiles_n);
-  // Groups of 32 rows (bf16 scales): one block per pair of groups, each step folded on its own.
+  // Groups of 32 rows: one block per pair of groups, each step folded on its own.
   const bool half = grouped && d.block_size == 32;
   ga.gpb = half ? 1 : grouped ? (int)(d.block_size / kBK) : 0;
-  // Split tail: when the tiles leave a last partial round of at most half the CUs (planned for
-  // MI355X's 256 CUs whatever the device reports, so the summation order depends on the shape
-  // only), those tiles are computed as two halves of K by twice as many workgroups.  Not under
-  // mx_qdense_noalloc (its static scratch is smaller than the partial tiles).
-  const int64_t tiles = tiles_m * tiles_n, tail = tiles % kSplitPlanCUs;
-  const int64_t KB = d.K / kBK;
-  const bool split = tiles > kSplitPlanCUs && tail > 0 && 2 * tail <= kSplitPlanCUs && KB % 2 == 0 && KB >= 8 &&
-                     (!grouped || (KB / 2) % ga.gpb == 0) && !b->noalloc_active;
-  ga.split_from = (int)(split ? tiles - tail : tiles);
+  const GemmPlan pl = gemm_plan(d.M, d.K, d.N, std::max(ga.gpb, 1), b->noalloc_active);
+  if (pl.tiles_m * pl.tiles_n > (int64_t)1 << 30)
+    return set_error(MX_ERR_INVALID, "FusedQuantizedDense: output too large for the GEMM path");
+  ga.tiles_n = (int)pl.tiles_n;
+  ga.grouped = (pl.tiles_m % 2 == 0 && pl.tiles_n % 16 == 0) ? 1 : 0;
+  ga.tiles = (int)(pl.tiles_m * pl.tiles_n);
+  ga.split_from = (int)pl.whole;
+  ga.S = (int)pl.S;
+  ga.kpb = (int)pl.kpb;
   ga.part = nullptr;
   ga.ctr = nullptr;
-  if (split) {
+  const int64_t parts = (ga.tiles - pl.whole) * pl.S;
+  if (parts > 0) {
     const size_t counter_bytes = 64 * 1024;  // shared with the decode kernels' counters (zero between launches)
     void* scratch = nullptr;
-    MX_TRY(ensure_scratch(b, counter_bytes + (size_t)tail * 2 * 16 * kThreads * 16, &scratch));
+    MX_TRY(ensure_scratch(b, counter_bytes + (size_t)parts * pl.rb * 4 * kThreads * 16, &scratch));
     ga.ctr = (uint32_t*)scratch;
     ga.part = (float*)((char*)scratch + counter_bytes);
   }
-  const int grid = (int)(split ? tiles + tail : tiles);
+  const int grid = (int)(pl.whole + parts);
   hipStream_t st = b->stream;
   // bf16 group scales: the fold-every-block kernel; f32 group scales count blocks at run time.
-  auto grouped_kernel = [&](auto kind) {
-    constexpr int BK = decltype(kind)::value;
-    if (half && d.s_dt == MX_DTYPE_FLOAT32)
-      dispatch(qdense_gemm_kernel<BK, true, true, true, true>, grid, kThreads, 0, st, ga);
+  auto go = [&](auto kind, auto rbc) {
+    constexpr int BK = decltype(kind)::value, RB = decltype(rbc)::value;
+    if (!grouped)
+      dispatch(qdense_gemm_kernel<BK, RB, false>, grid, kThreads, 0, st, ga);
+    else if (half && d.s_dt == MX_DTYPE_FLOAT32)
+      dispatch(qdense_gemm_kernel<BK, RB, true, true, true, true>, grid, kThreads, 0, st, ga);
     else if (half)
-      dispatch(qdense_gemm_kernel<BK, true, true, true>, grid, kThreads, 0, st, ga);
+      dispatch(qdense_gemm_kernel<BK, RB, true, true, true>, grid, kThreads, 0, st, ga);
     else if (d.s_dt == MX_DTYPE_BFLOAT16)
-      dispatch(qdense_gemm_kernel<BK, true, true>, grid, kThreads, 0, st, ga);
+      dispatch(qdense_gemm_kernel<BK, RB, true, true>, grid, kThreads, 0, st, ga);
     else
-      dispatch(qdense_gemm_kernel<BK, true>, grid, kThreads, 0, st, ga);
+      dispatch(qdense_gemm_kernel<BK, RB, true>, grid, kThreads, 0, st, ga);
+  };
+  auto rows = [&](auto kind) {
+    pl.rb == 2 ? go(kind, std::integral_constant<int, 2>{}) : go(kind, std::integral_constant<int, 4>{});
   };
   return launch(b, name, [&] {
     switch (d.w_dt) {
-      case MX_DTYPE_INT8:
-        grouped ? grouped_kernel(std::integral_constant<int, kBI8>{})
-                : dispatch(qdense_gemm_kernel<kBI8, false>, grid, kThreads, 0, st, ga);
-        break;
-      case MX_DTYPE_UINT8:
-        grouped ? grouped_kernel(std::integral_constant<int, kBU8>{})
-                : dispatch(qdense_gemm_kernel<kBU8, false>, grid, kThreads, 0, st, ga);
-        break;
-      case MX_DTYPE_INT4:
-        grouped ? grouped_kernel(std::integral_constant<int, kBI4>{})
-                : dispatch(qdense_gemm_kernel<kBI4, false>, grid, kThreads, 0, st, ga);
-        break;
-      default:
-        grouped ? grouped_kernel(std::integral_constant<int, kBU4>{})
-                : dispatch(qdense_gemm_kernel<kBU4, false>, grid, kThreads, 0, st, ga);
-        break;
+      case MX_DTYPE_INT8: rows(std::integral_constant<int, kBI8>{}); break;
+      case MX_DTYPE_UINT8: rows(std::integral_constant<int, kBU8>{}); break;
+      case MX_DTYPE_INT4: rows(std::integral_constant<int, kBI4>{}); break;
+      default: rows(std::integral_constant<int, kBU4>{}); break;
     }
   });
 }
@@ -763,7 +810,7 @@ int dot_mfma_run(mx_backend* b, const DotDesc& d, const char* name) {
   ga.M = (int)d.M;
   ga.K = (int)d.K;
   ga.N = (int)d.N;
-  const int64_t tiles_m = (d.M + kBM - 1) / kBM, tiles_n = (d.N + kBN - 1) / kBN;
+  const int64_t tiles_m = (d.M + kBM<4> - 1) / kBM<4>, tiles_n = (d.N + kBN - 1) / kBN;
   if (d.B * tiles_m * tiles_n > (int64_t)1 << 30)
     return set_error(MX_ERR_INVALID, "DotGeneral: output too large for the matrix-core path");
   ga.tiles_n = (int)tiles_n;
@@ -776,14 +823,14 @@ int dot_mfma_run(mx_backend* b, const DotDesc& d, const char* name) {
   return launch(b, name, [&] {
     if (d.rhs_transposed) {
       if (f16)
-        dispatch(qdense_gemm_kernel<kBF16NK, false>, grid, kThreads, 0, st, ga);
+        dispatch(qdense_gemm_kernel<kBF16NK, 4, false>, grid, kThreads, 0, st, ga);
       else
-        dispatch(qdense_gemm_kernel<kBBf16NK, false>, grid, kThreads, 0, st, ga);
+        dispatch(qdense_gemm_kernel<kBBf16NK, 4, false>, grid, kThreads, 0, st, ga);
     } else {
       if (f16)
-        dispatch(qdense_gemm_kernel<kBF16KN, false>, grid, kThreads, 0, st, ga);
+        dispatch(qdense_gemm_kernel<kBF16KN, 4, false>, grid, kThreads, 0, st, ga);
       else
-        dispatch(qdense_gemm_kernel<kBBf16KN, false>, grid, kThreads, 0, st, ga);
+        dispatch(qdense_gemm_kernel<kBBf16KN, 4, false>, grid, kThreads, 0, st, ga);
     }
   });
 }

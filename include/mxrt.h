@@ -414,11 +414,10 @@ int mx_qdense_plan(mx_backend* b, const mx_qdense_args* args, char* buf, size_t 
  * hipMalloc). The split-K partial sums and arrival counters live in a static device array of
  * MX_QDENSE_NOALLOC_SCRATCH_BYTES per GPU, set up by mx_backend_new and held until the process
  * ends; a problem whose split-K needs more returns MX_ERR_INVALID before anything is launched.
- * Results are bit-identical to mx_qdense's, except where mx_qdense splits the last partial round
- * of a prefill's tiles along K into more partial tiles than the array holds (bf16 GEMM: at most 128
- * tiles past a multiple of 256, in two halves; GGML, reference-layout and f32 x prefills: at most
- * half a round of 256 or 512 tiles past whole rounds): those tiles are summed in fewer slices or
- * whole here (within the f32 accumulation bound of the reference's sum). Every call on one GPU
+ * Results are bit-identical to mx_qdense's, except where mx_qdense cuts a prefill's tiles (those
+ * past the last whole round of resident workgroups) into K slices with more partial tiles than the
+ * array holds: those tiles are summed in fewer slices or whole here (within the f32 accumulation
+ * bound of the reference's sum). Every call on one GPU
  * shares the array, from any backend; the calls are ordered on the device (each call's stream
  * waits for the previous call's completion event), so calls from several streams or backends run
  * one after another.  Under graph capture that wait cannot be recorded: the caller must keep a

@@ -11,6 +11,7 @@ oracle computes rows independently).
 import numpy as np
 import pytest
 
+import compute_amd as ca
 from oracle import oracle as O
 from tests.qd_helpers import QDenseRun, assert_bf16_close
 
@@ -142,3 +143,21 @@ def test_gemm_split_tail(backend, w_dtype, G, s_dtype, act):
     rows = np.sort(np.concatenate([np.arange(0, 8), np.arange(256, 264), np.arange(504, 512)]))
     y = check_rows(r, rows=rows, threads=8, what=f"{w_dtype} G={G}")
     assert np.array_equal(y, r.run())
+
+
+@pytest.mark.parametrize("M,K,N", [(65, 1088, 144), (129, 4160, 400), (257, 2176, 272), (600, 1088, 2064)])
+@pytest.mark.parametrize("w_dtype,G,s_dtype", [(O.DT_INT8, None, O.DT_FLOAT32), (O.DT_INT4, 64, O.DT_BFLOAT16),
+                                               (O.DT_UINT4, 64, O.DT_FLOAT32), (O.DT_INT8, 32, O.DT_BFLOAT16),
+                                               (O.DT_UINT8, 32, O.DT_FLOAT32)])
+def test_tiles_in_k_slices(backend, M, K, N, w_dtype, G, s_dtype):
+    """Tiles of 128 and 256 rows in K slices of unequal lengths (17 and 34 blocks of 64 rows, 65 and
+    34 at the other shapes), rows and columns past the last whole tile; the allocation-free entry
+    point runs the same slices (the partial tiles fit its array)."""
+    p = O.make_problem(M, K, N, w_dtype=w_dtype, block_axis=0, block_size=G if G else K, per_channel_1d=G is None,
+                       scale_dtype=s_dtype, bias=True, scale_range=(0.002, 0.02), seed=M + K)
+    r = QDenseRun(backend, p)
+    assert r.plan().startswith("qdense_gemm_mfma")
+    y = check_rows(r, threads=8, what=f"{w_dtype} G={G}")
+    out = backend.BufferFromFlatData(0, np.zeros(M * N, np.uint16), ca.Shape(ca.BFloat16, M, N))
+    backend.QDenseNoAlloc(r.args(out))
+    assert np.array_equal(out.ToFlatData().reshape(M, N), y)
