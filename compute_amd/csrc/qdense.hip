@@ -16,7 +16,7 @@
 //   qdense_gemm_mfma (qdense_gemm.hip) — M > 16 bf16 rows, int8/uint8/int4/uint4 weights, one
 //                    scale per output column or per group of 64k rows (prefill): bf16 MFMA GEMM
 //                    with on-the-fly dequantisation.
-//   qdense_gemv (qdense_gemv.hip) — up to 64 rows of the reference's own layout, f32 x, zero
+//   qdense_gemv (qdense_gemv.hip) — up to 16-64 rows of the reference's own layout, f32 x, zero
 //                    points, NF4: HBM-bound decode GEMV.
 //   qdense_refgemm_f32_mfma (qdense_refgemm.hip) — the same variants past the GEMV: f32
 //                    operands in three exact bf16 parts on the bf16 matrix cores (split_gemm.h).
@@ -368,6 +368,19 @@ static bool qdense_refgemm_plan(const QDenseDesc& d) {
   return d.M > 4 && d.M * d.K * d.N > kRefGemmMinMKN && qdense_refgemm_fits(d);
 }
 
+// Rows past which the contraction, which reads the weights once, is taken where the GEMV would read
+// them for every four rows.  Reference layout with at least 128 columns per scale block (3 products
+// per term): Int4 [4096,11008], f32 x, 79 us (GEMV) against 65 at 16 rows, 94 against 65 at 17, 314
+// against 66 at 64.  Narrower blocks, zero points beside them and NF4 (6 products): int8 with zero
+// points and 64-column blocks 110 against 117 at 20 rows, 138 against 117 at 24, 366 against 117 at
+// 64.  Scales along K: int8 g64 104 against 111 at 24 rows, 138 against 111 at 32, 207 against 111 at
+// 48.  The contraction's error against 64 bits is the smaller one throughout (0.7e-7 to 1.2e-7
+// against 1.4e-7 to 3.2e-7).
+static int64_t refgemm_min_rows(const QDenseDesc& d) {
+  if (d.block_axis == 0) return 32;
+  return d.scheme == MX_QUANT_LINEAR && (d.block_size % 128 == 0 || d.block_size >= d.N) ? 16 : 20;
+}
+
 // =============================================================================================
 // Kernel selection.
 // =============================================================================================
@@ -427,6 +440,7 @@ static QPath choose_path(const mx_backend* b, const QDenseDesc& d) {
   // Past the skinny kernel's 16 rows the GEMM reads every weight once, while the GEMV reads the
   // whole weight matrix again for every 4 rows: the GEMV takes only what the GEMM does not fit.
   if (!b->gemv_over_gemm && qdense_gemm_fits(d)) return QPath::kGemm;
+  if (!b->gemv_over_gemm && d.M > refgemm_min_rows(d) && qdense_refgemm_plan(d)) return QPath::kRefGemm;
   if (qdense_gemv_fits(d)) return QPath::kGemv;
   if (qdense_gemm_fits(d)) return QPath::kGemm;
   // The reference layout, f32 x, zero points and NF4 at prefill size: the fused kernel.

@@ -12,8 +12,9 @@
 // two run 12 ns per MFMA and SIMD where the MFMA alone takes 8).  Measured, f32 x [2048,4096] x Int4
 // [4096,11008], against an f32-MFMA kernel at 0.63 of the f32 peak: scales per row and 128 columns
 // (3 products) 1868 -> 578 us, 0.96 PFLOP/s of products; per row and 64 columns (6 products) 1868 ->
-// 1010 us; with 100 rows 363 -> 60 us (K in 2 slices).  The error against 64 bits fell from 1.1e-6
-// to 5.8e-7 (3 products) and 9.8e-7 (6): a step sums 32 terms where the f32 MFMA summed 4.
+// 1060 us; with 100 rows 363 -> 65 us (K in 2 slices).  The error against 64 bits fell from 1.1e-6
+// to 5.8e-7 (four waves) and 1.1e-7 (eight): a step sums 32 terms where the f32 MFMA summed 4, and
+// eight waves keep the sums in three levels.
 //
 // Tiling: a workgroup of 4 (or 8) waves owns a 128 x 128 output tile, 2 x 2 waves of 64 x 64 (4 x 2
 // of 32 x 64), K in blocks of 32 (one MFMA step).  An operand's part lies in LDS as 128 rows of 32
@@ -259,7 +260,12 @@ __global__ __launch_bounds__(64 * NW, 2) void split_gemm_kernel(Args a) {
     }
   };
 
-  f32x4_t acc[RB][4];
+  // Eight waves leave registers to round less: the products of leading parts and those of the others
+  // have sums of their own (a step then rounds the large sums once instead of 3 or 6 times), and the
+  // large sums go to a total every kFold blocks (chains of kFold and K / 32 kFold additions).
+  constexpr bool kLow = NW == 8 && PA + PB > 2;
+  constexpr int kFold = 8;
+  f32x4_t acc[RB][4], low[RB][4], total[RB][4];
   auto clear = [&]() __attribute__((always_inline)) {
 #pragma unroll
     for (int i = 0; i < RB; ++i)
@@ -267,6 +273,12 @@ __global__ __launch_bounds__(64 * NW, 2) void split_gemm_kernel(Args a) {
       for (int c = 0; c < 4; ++c) acc[i][c] = f32x4_t{0.f, 0.f, 0.f, 0.f};
   };
   clear();
+  if constexpr (kLow) {
+#pragma unroll
+    for (int i = 0; i < RB; ++i)
+#pragma unroll
+      for (int c = 0; c < 4; ++c) low[i][c] = total[i][c] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+  }
   // One block: small products first.
   auto compute = [&](const char* buf) __attribute__((always_inline)) {
     const char* As = buf;
@@ -289,7 +301,12 @@ __global__ __launch_bounds__(64 * NW, 2) void split_gemm_kernel(Args a) {
           const int pb = order - pa;
           if (pb < 0 || pb >= PB) continue;
 #pragma unroll
-          for (int c = 0; c < 4; ++c) acc[rb][c] = mfma(A[pa], B[pb][c], acc[rb][c]);
+          for (int c = 0; c < 4; ++c) {
+            if (kLow && order > 0)
+              low[rb][c] = mfma(A[pa], B[pb][c], low[rb][c]);
+            else
+              acc[rb][c] = mfma(A[pa], B[pb][c], acc[rb][c]);
+          }
         }
       }
     }
@@ -331,9 +348,26 @@ __global__ __launch_bounds__(64 * NW, 2) void split_gemm_kernel(Args a) {
   const int whole = kb1 * kBK > K ? last - 1 : last;  // steps that stage a whole block
   int kb = kb0;
 #pragma unroll 1
-  for (; kb < whole; ++kb) step(kb, Whole{});
+  for (; kb < whole; ++kb) {
+    step(kb, Whole{});
+    if (kLow && (kb - kb0) % kFold == kFold - 1) {
+#pragma unroll
+      for (int i = 0; i < RB; ++i)
+#pragma unroll
+        for (int c = 0; c < 4; ++c) {
+          total[i][c] += acc[i][c];
+          acc[i][c] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+        }
+    }
+  }
   if (kb < last) step(kb, Tail{});
   compute(sm[(last - kb0) & 1]);
+  if constexpr (kLow) {
+#pragma unroll
+    for (int i = 0; i < RB; ++i)
+#pragma unroll
+      for (int c = 0; c < 4; ++c) acc[i][c] = total[i][c] + (acc[i][c] + low[i][c]);
+  }
   if (big > MX_SPLIT_MAX) flag = 1;
   __syncthreads();
 

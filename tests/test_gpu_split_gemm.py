@@ -148,3 +148,15 @@ def test_ggml_rows_at_ragged_edges(backend, t, M, K, N):
     backend.QDense(a)
     exact, ab = O.ggml_dense_f64(x, w, int(t), None)
     assert np.all(np.abs(out.ToFlatData().reshape(M, N).astype(np.float64) - exact) <= 1e-5 * ab + 1e-30)
+
+
+@pytest.mark.parametrize("M,K,N,axis,B,zp", [(17, 2048, 1040, 1, 128, False), (64, 2048, 528, 1, 32, True), (33, 4128, 272, 0, 96, False)])
+def test_few_rows(backend, M, K, N, axis, B, zp):
+    """The fewest rows of the reference layout and of scales along K that leave the GEMV: held to a
+    third of the bound, which the GEMV's sums kept too."""
+    p = O.make_problem(M, K, N, w_dtype=O.DT_INT8, x_dtype=F32, scale_dtype=F32, block_axis=axis, block_size=B, zp=zp, bias=True, seed=M)
+    r = QDenseRun(backend, p)
+    assert r.plan() == "qdense_refgemm_f32_mfma"
+    y = r.run().astype(np.float64)
+    truth, scale = O.qdense_f64(p), O.qdense_f64(p, absolute=True)
+    assert np.all(np.abs(y - truth) <= 2.0 ** -22 * np.abs(truth) + 3e-6 * scale)
