@@ -11,12 +11,14 @@
 // itself (the reference's noSIMD kernels, internal/gobackend/dot/matmul/nosimd.go:66-75), in
 // any summation order.  Larger contractions run on the matrix cores: the
 // small-tile dot_mm_kernel / dot_mm_lds_kernel below (f32, and half problems too small for
-// qdense_gemm.hip's 256x128-tile kernel), or that kernel.
+// qdense_gemm.hip's 256x128-tile kernel), that kernel, or (f32 from 2^30 multiply-adds) the
+// contraction in exact bf16 parts of split_gemm.h.
 
 #include <type_traits>
 
 #include "device_common.h"
 #include "mxrt_internal.h"
+#include "split_gemm.h"
 
 namespace mx {
 
@@ -506,6 +508,124 @@ static int dot_mm_run(mx_backend* b, const DotDesc& d) {
   }
 }
 
+// Large f32 contractions in exact bf16 parts (split_gemm.h, eight waves, 6 products per term): the
+// right-hand side as the kernel's second operand.  [N, K]: thread t takes the 8 values of chunk t & 3
+// of a block's 32 k of one column; [K, N]: rows 4 j .. 4 j + 3 of two columns.
+template <bool BT>
+struct DotSource {
+  static constexpr bool kXbf = false, kRow = false, kCol = false, kZp = false;
+  static constexpr int kPA = 3, kPB = 3;
+  struct Regs {
+    uint32_t v[8];
+  };
+  int p, j, c0, cq;  // [N, K]: LDS row; [K, N]: row group, first column of the quad, quad
+  uint32_t off[BT ? 1 : 4];
+  const char* base;
+
+  static __device__ __forceinline__ float table_value(int) { return 0.0f; }
+  __device__ __forceinline__ DotSource(const sg::Args& a, int t, int n0) {
+    if constexpr (BT) {
+      p = t >> 2;
+      j = t & 3;
+      base = (const char*)a.w + (int64_t)n0 * a.K * 4;
+      off[0] = ((uint32_t)min(sg::col_of_row(p), a.N - 1 - n0) * (uint32_t)a.K + 8u * j) * 4u;
+    } else {
+      cq = (t >> 1) & 31;
+      c0 = 2 * ((t >> 6) & 1);
+      j = (t & 1) | (t >> 7) << 1;
+      base = (const char*)a.w;
+      // N % 4 == 0: the two columns are in range or past N (then the first are read, and not stored).
+      const uint32_t n = n0 + 4 * cq < a.N ? n0 + 4 * cq + c0 : 0;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) off[e] = ((uint32_t)(4 * j + e) * (uint32_t)a.N + n) * 4u;
+    }
+  }
+  __device__ __forceinline__ void load(const sg::Args& a, sg::Block b, Regs& R) const {
+    if constexpr (BT) {
+      const char* q = base + (int64_t)b.k * 4;
+      const sg::u32x4_v lo = *(const sg::u32x4_v*)(q + off[0]), hi = *(const sg::u32x4_v*)(q + off[0] + 16);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        R.v[e] = lo[e];
+        R.v[4 + e] = hi[e];
+      }
+    } else {
+      const char* q = base + (int64_t)b.k * a.N * 4;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const sg::u32x2_v w = *(const sg::u32x2_v*)(q + off[e]);
+        R.v[e] = w[0];
+        R.v[4 + e] = w[1];
+      }
+    }
+  }
+  template <class TailT>
+  __device__ __forceinline__ void stage(const sg::Args& a, sg::Block b, const Regs& R, const float*, char* Bs, float& big, TailT) const {
+    float v[8];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      v[e] = __uint_as_float(R.v[e]);
+      // Values that the block before holds are zero (x is too, but 0 * inf is not).
+      if (TailT::value && (BT ? 8 * j + (e & 4) : 4 * j) < b.skip) v[e] = 0.0f;
+    }
+    uint32_t h[4], m[4], l[4];
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      big = fmaxf(fmaxf(fabsf(v[2 * q]), fabsf(v[2 * q + 1])), big);
+      sg::split2(v[2 * q], v[2 * q + 1], h[q], m[q], l[q]);
+    }
+    if constexpr (BT) {
+      char* dst = Bs + sg::chunk_at(p, j);
+      *(sg::u32x4_v*)dst = sg::u32x4_v{h[0], h[1], h[2], h[3]};
+      *(sg::u32x4_v*)(dst + sg::kPlane) = sg::u32x4_v{m[0], m[1], m[2], m[3]};
+      *(sg::u32x4_v*)(dst + 2 * sg::kPlane) = sg::u32x4_v{l[0], l[1], l[2], l[3]};
+    } else {
+#pragma unroll
+      for (int c = 0; c < 2; ++c) {
+        char* dst = Bs + sg::chunk_at(sg::row_of_col(4 * cq + c0 + c), j >> 1) + 8 * (j & 1);
+        *(sg::u32x2_v*)dst = sg::u32x2_v{h[2 * c], h[2 * c + 1]};
+        *(sg::u32x2_v*)(dst + sg::kPlane) = sg::u32x2_v{m[2 * c], m[2 * c + 1]};
+        *(sg::u32x2_v*)(dst + 2 * sg::kPlane) = sg::u32x2_v{l[2 * c], l[2 * c + 1]};
+      }
+    }
+  }
+  __device__ __forceinline__ float value(const sg::Args& a, int k, int n, const float*) const {
+    return ((const float*)a.w)[BT ? (int64_t)n * a.K + k : (int64_t)k * a.N + n];
+  }
+};
+
+// From 2^30 multiply-adds: below that the small f32 tiles fill the chip sooner (transposed
+// [1920,384] x 384 12 us against 19, [333,704] x 2112 19 against 21).  Above, transposed and not:
+// [2048,1536] x 384 33 and 36 -> 23 us, [1920,384] x 1536 27 and 36 -> 20, [2048,4096] x 4096 586 and
+// 867 -> 362 and 373, [128,4096] x 4096 80 and 55 -> 34; the error against 64 bits 3.5e-7 to 1.2e-6
+// -> 0.8e-7 to 1.2e-7.
+static bool dot_split_fits(const DotDesc& d) {
+  auto aligned = [](const void* p) { return ((uintptr_t)p % 16) == 0; };
+  return d.in_dt == MX_DTYPE_FLOAT32 && d.out_dt == MX_DTYPE_FLOAT32 && d.B == 1 && d.K >= sg::kBK && d.K % 4 == 0 &&
+         (d.rhs_transposed || d.N % 4 == 0) && d.M < (int64_t)1 << 30 && d.N <= (int64_t)1 << 24 && d.K <= (int64_t)1 << 22 &&
+         aligned(d.lhs) && aligned(d.rhs) && d.M >= 96 && d.N >= 96 &&
+         d.M * d.N * d.K >= (int64_t)1 << 30;
+}
+
+static int dot_split_run(mx_backend* b, const DotDesc& d) {
+  sg::Args a{};
+  a.x = d.lhs;
+  a.w = (const uint8_t*)d.rhs;
+  a.out = d.out;
+  a.M = (int)d.M;
+  a.K = (int)d.K;
+  a.N = (int)d.N;
+  a.act = MX_ACT_NONE;
+  int nw = 0, grid = 0;
+  MX_TRY(sg::plan(b, a, d.M, 6, &nw, &grid));
+  return launch(b, "dot_mfma_f32", [&] {
+    if (d.rhs_transposed)
+      dispatch(sg::split_gemm_kernel<DotSource<true>, 8>, grid, 512, 0, b->stream, a);
+    else
+      dispatch(sg::split_gemm_kernel<DotSource<false>, 8>, grid, 512, 0, b->stream, a);
+  });
+}
+
 // qdense_gemm.hip's 256x128-tile kernel takes half contractions with M >= 256 that give it
 // >= 64 workgroups (measured: at 96 it beats the small tiles 12 us to 22 us; at 24 or fewer,
 // or batched with M = 128 / 192, the small tiles win); others go to the small-tile kernels.
@@ -523,6 +643,7 @@ int dot_run(mx_backend* b, const DotDesc& d) {
   }
   if (dot_big_tiles(d))
     return dot_mfma_run(b, d, d.in_dt == MX_DTYPE_BFLOAT16 ? "dot_mfma_bf16" : "dot_mfma_f16");
+  if (dot_split_fits(d)) return dot_split_run(b, d);
   if (dot_mm_fits(d)) return dot_mm_run(b, d);
   if (dot_mfma_fits(d))
     return dot_mfma_run(b, d, d.in_dt == MX_DTYPE_BFLOAT16 ? "dot_mfma_bf16" : "dot_mfma_f16");

@@ -160,3 +160,26 @@ def test_few_rows(backend, M, K, N, axis, B, zp):
     y = r.run().astype(np.float64)
     truth, scale = O.qdense_f64(p), O.qdense_f64(p, absolute=True)
     assert np.all(np.abs(y - truth) <= 2.0 ** -22 * np.abs(truth) + 3e-6 * scale)
+
+
+@pytest.mark.parametrize("transposed", [True, False])
+@pytest.mark.parametrize("M,K,N", [(96, 115004, 100), (1037, 1028, 1036), (2049, 548, 1000)])
+def test_dot_general_f32(backend, transposed, M, K, N):
+    """f32 DotGeneral from 2^30 multiply-adds: one tile in many K slices, ragged tiles, K past the last
+    block of 32; one infinity, in a row (and so a tile) of its own."""
+    assert M * K * N >= 1 << 30
+    rng = np.random.default_rng(K)
+    x, w = rng.standard_normal((M, K)).astype(np.float32), rng.standard_normal((K, N)).astype(np.float32)
+    x[M - 1, K - 1] = np.inf
+    w[K - 1] = np.abs(w[K - 1]) + 0.5
+    bld = backend.Builder("dot")
+    f = bld.Main()
+    shapes = [ca.Shape(ca.Float32, M, K), ca.Shape(ca.Float32, *((N, K) if transposed else (K, N)))]
+    a, b = (f.Parameter(n, s) for n, s in zip("ab", shapes))
+    f.Return([f.DotGeneral(a, [1], [], b, [1 if transposed else 0], [])])
+    bufs = [backend.BufferFromFlatData(0, np.ascontiguousarray(v).ravel(), s) for v, s in zip((x, w.T if transposed else w), shapes)]
+    exe = bld.Compile()
+    y = exe.Execute(bufs)[0].ToFlatData().reshape(M, N)
+    assert np.all(np.isposinf(y[M - 1]))
+    truth, scale = x[:-1].astype(np.float64) @ w.astype(np.float64), np.abs(x[:-1]).astype(np.float64) @ np.abs(w).astype(np.float64)
+    assert np.all(np.abs(y[:-1] - truth) <= 2.0 ** -22 * np.abs(truth) + 3e-6 * scale)
