@@ -348,6 +348,160 @@ __global__ __launch_bounds__(kExactThreads) void qdense_exact_kernel(QDenseDesc 
     if (r < rows) store_f(d.out, (m0 + r) * N + n, d.x_dt, act_ref(acc[r], d.act));
 }
 
+// The same sums for problems of few outputs, whose chains leave most of the chip idle (bounded by
+// the latency of the additions and, before them, of the loads): only the additions are a chain, so eight waves form the terms of 64 columns of one row, kChainK of k at a
+// time, into LDS (each as the reference rounds it), and a ninth adds the chunk before in k order.
+// The bits are the reference-order kernel's.
+constexpr int kChainK = 128, kChainWaves = 8, kChainThreads = 64 * (kChainWaves + 1);
+constexpr int kChainRows = kChainK / kChainWaves;  // k per wave and chunk
+constexpr int kChainStride = kChainK + 4;          // floats per column: 16-byte accesses of 8 lanes cover all banks
+
+template <bool ZP, bool SK>
+__global__ __launch_bounds__(kChainThreads) void qdense_exact_chain_kernel(QDenseDesc d) {
+  __shared__ __attribute__((aligned(16))) float terms[2][64][kChainStride];
+  __shared__ float nf4[16];
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+  const int64_t N = d.N, m = blockIdx.y;
+  const int K = (int)d.K;
+  const uint32_t B = (uint32_t)d.block_size;
+  const int64_t n = (int64_t)blockIdx.x * 64 + lane;
+  const uint32_t nn = (uint32_t)min(n, N - 1);  // lanes past N repeat the last column, unstored
+  const bool packed = d.w_dt == MX_DTYPE_INT4 || d.w_dt == MX_DTYPE_UINT4;
+  const bool sgn = d.w_dt == MX_DTYPE_INT4 || d.w_dt == MX_DTYPE_INT8;
+  const bool xbf = d.x_dt == MX_DTYPE_BFLOAT16, sbf = d.s_dt == MX_DTYPE_BFLOAT16, zbf = d.zp_dt == MX_DTYPE_BFLOAT16;
+  const bool nf = d.scheme == MX_QUANT_NF4;
+  if (threadIdx.x < 16) nf4[threadIdx.x] = kNF4Table[threadIdx.x];
+  const bool ax1 = d.block_axis == 1;
+  const int64_t nb = (N + B - 1) / B;
+  const uint32_t scol = ax1 ? nn / B : nn;
+  // Rows are uniform over a wave: a row's address is scalar, a lane adds its column's offset.
+  // Element `col` of row r (rows `len` elements long) of an f32 or bf16 array.
+  auto at = [](const void* p, int64_t r, int64_t len, uint32_t col, bool bf) __attribute__((always_inline)) {
+    if (bf) return (uint32_t)*(const uint16_t*)((const char*)p + r * len * 2 + 2ull * col) << 16;
+    return *(const uint32_t*)((const char*)p + r * len * 4 + 4ull * col);
+  };
+  float s_col = 0.0f, z_col = 0.0f;  // one scale per column (SK false)
+  if constexpr (!SK) {
+    s_col = __uint_as_float(at(d.scale, 0, 0, scol, sbf));
+    if constexpr (ZP) z_col = __uint_as_float(at(d.zp, 0, 0, scol, zbf));
+  }
+  // A wave's operands of a chunk: k0 + r for r < kChainRows (past K: those of K - 1, never added).
+  struct Ops {
+    uint32_t w[kChainRows], s[SK ? kChainRows : 1], z[SK && ZP ? kChainRows : 1];
+    uint32_t x;  // lane r: x[k0 + r]
+  };
+  // 4-bit rows that start mid-byte (k and N odd) hold column nn in byte (nn + 1) / 2.
+  const uint32_t half[2] = {nn >> 1, (nn + 1) >> 1}, off[2] = {4u * (nn & 1u), 4u * (~nn & 1u)};
+  auto load = [&](int k0, Ops& o) __attribute__((always_inline)) {
+    o.x = at(d.x, m, K, (uint32_t)min(k0 + (lane & (kChainRows - 1)), K - 1), xbf);
+#pragma unroll
+    for (int r = 0; r < kChainRows; ++r) {
+      const int k = min(k0 + r, K - 1);
+      const int64_t row = (int64_t)k * N;
+      const uint8_t* p = (const uint8_t*)d.w + (packed ? row >> 1 : row);
+      o.w[r] = p[packed ? half[row & 1] : nn];
+    }
+    if constexpr (SK) {
+      auto rows = [&](const void* p, bool bf, uint32_t (&v)[kChainRows]) __attribute__((always_inline)) {
+#pragma unroll
+        for (int r = 0; r < kChainRows; ++r) {
+          const uint32_t k = (uint32_t)min(k0 + r, K - 1);
+          v[r] = at(p, ax1 ? k : k / B, ax1 ? nb : N, scol, bf);
+        }
+      };
+      if (sbf)
+        rows(d.scale, true, o.s);
+      else
+        rows(d.scale, false, o.s);
+      if constexpr (ZP) {
+        if (zbf)
+          rows(d.zp, true, o.z);
+        else
+          rows(d.zp, false, o.z);
+      }
+    }
+  };
+  auto form = [&](int k0, const Ops& o, float* out) __attribute__((always_inline)) {
+    float w[kChainRows];
+#pragma unroll
+    for (int r = 0; r < kChainRows; ++r) {
+      uint32_t v = o.w[r];
+      if (packed) v = (v >> off[((int64_t)min(k0 + r, K - 1) * N) & 1]) & 15u;
+      const int sv = packed ? __builtin_amdgcn_sbfe((int)v, 0, 4) : (int)(int8_t)v;
+      w[r] = (float)(sgn ? sv : (int)v);
+    }
+    if (nf) {
+#pragma unroll
+      for (int r = 0; r < kChainRows; ++r) w[r] = nf4[(uint32_t)(int)w[r] & 15u];
+    }
+#pragma unroll
+    for (int r = 0; r < kChainRows; r += 4) {
+      float t[4];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const float x = __uint_as_float(__builtin_amdgcn_readlane(o.x, r + e));
+        const float s = SK ? __uint_as_float(o.s[SK ? r + e : 0]) : s_col;
+        const float z = SK && ZP ? __uint_as_float(o.z[SK && ZP ? r + e : 0]) : z_col;
+        t[e] = ZP ? mul_rn(x, add_rn(mul_rn(w[r + e], s), z)) : mul_rn(mul_rn(x, w[r + e]), s);
+      }
+      *(f32x4_t*)(out + r) = f32x4_t{t[0], t[1], t[2], t[3]};
+    }
+  };
+  const int chunks = (K + kChainK - 1) / kChainK;
+  const bool adds = wave == kChainWaves;
+  float acc = adds && d.bias ? load_f(d.bias, nn, d.b_dt) : 0.0f;
+  const int kw = kChainRows * min(wave, kChainWaves - 1);
+  constexpr int kAhead = SK ? 2 : 4;  // chunks requested ahead of their use
+  Ops o[kAhead];
+  if (!adds) {
+#pragma unroll
+    for (int i = 0; i < kAhead; ++i) load(i * kChainK + kw, o[i]);
+  }
+  __syncthreads();  // the NF4 table is written
+  auto phase = [&](int c, Ops& oc) __attribute__((always_inline)) {
+    if (!adds) {
+      if (c < chunks) {
+        form(c * kChainK + kw, oc, &terms[c & 1][lane][kw]);
+        if (c + kAhead < chunks) load((c + kAhead) * kChainK + kw, oc);
+      }
+    } else if (c > 0) {
+      const float* t = terms[(c - 1) & 1][lane];
+      const int kn = min(kChainK, K - (c - 1) * kChainK);
+      if (kn == kChainK) {
+#pragma unroll
+        for (int k = 0; k < kChainK; k += 4) {
+          const f32x4_t v = *(const f32x4_t*)(t + k);
+#pragma unroll
+          for (int e = 0; e < 4; ++e) acc = add_rn(acc, v[e]);
+        }
+      } else {
+#pragma unroll 1
+        for (int k = 0; k < kn; ++k) acc = add_rn(acc, t[k]);
+      }
+    }
+    __syncthreads();
+  };
+#pragma unroll 1
+  for (int c = 0; c <= chunks; c += kAhead) {
+#pragma unroll
+    for (int i = 0; i < kAhead; ++i) {
+      if (c + i <= chunks) phase(c + i, o[i]);  // uniform over the workgroup
+    }
+  }
+  if (adds && n < N) store_f(d.out, m * N + n, d.x_dt, act_ref(acc, d.act));
+}
+
+// Whether the chain kernel takes a problem: few enough workgroups (64 outputs each) that the other
+// kernel would leave most of the chip idle, and chains long enough to pay for the barriers.  int8 per
+// channel [4,512] x 512 17.2 -> 9.8 us, [16,512] x 1024 17.4 -> 9.9 ([32,512] x 1024, 512 workgroups,
+// 17.4 against 20.9; [4,128] x 4096 6.0 against 7.8); scales along K, whose loads the other kernel
+// makes per output: [8,128] x 256 14.4 -> 7.0, [32,512] x 1024 51 -> 24, [4,2048] x 1000 196 -> 48
+// ([100,256] x 512, 800 workgroups, 27 against 29).
+static bool exact_chain_plan(const QDenseDesc& d) {
+  const bool sk = d.block_axis == 1 || d.block_size < d.K;
+  return d.K >= (sk ? 128 : 256) && d.M * ((d.N + 63) / 64) <= (sk ? 512 : 256);
+}
+
 // Rows per thread of the reference-order kernel: 8 when the grid has two waves per SIMD of a
 // 256-CU part even so, else 1.
 static int exact_rows(const QDenseDesc& d) {
@@ -570,11 +724,21 @@ int qdense_run(mx_backend* b, const QDenseDesc& d) {
     case QPath::kRefGemm:
       return qdense_refgemm_run(b, d, name);
     default: {
+      // The scale varies along K unless there is one per column (block_axis 0, one group).
+      const bool sk = d.block_axis == 1 || d.block_size < d.K;
+      if (exact_chain_plan(d)) {
+        const dim3 grid((unsigned)((d.N + 63) / 64), (unsigned)d.M);
+        return launch(b, name, [&] {
+          auto go = [&](auto kern) { dispatch(kern, grid, kChainThreads, 0, st, d); };
+          if (d.zp)
+            sk ? go(qdense_exact_chain_kernel<true, true>) : go(qdense_exact_chain_kernel<true, false>);
+          else
+            sk ? go(qdense_exact_chain_kernel<false, true>) : go(qdense_exact_chain_kernel<false, false>);
+        });
+      }
       const int R = exact_rows(d);
       dim3 grid((unsigned)((d.N + kExactThreads - 1) / kExactThreads), (unsigned)((d.M + R - 1) / R));
       if (grid.y > 65535u) return set_error(MX_ERR_INVALID, "FusedQuantizedDense: M too large for the exact path");
-      // The scale varies along K unless there is one per column (block_axis 0, one group).
-      const bool sk = d.block_axis == 1 || d.block_size < d.K;
       return launch(b, name, [&] {
         auto go = [&](auto kern) { dispatch(kern, grid, kExactThreads, 0, st, d); };
         if (R == 8) {

@@ -11,6 +11,7 @@ Bars (from the task's north star):
 import numpy as np
 import pytest
 
+import compute_amd as ca
 from oracle import oracle as O
 from tests.qd_helpers import QDenseRun, assert_bf16_close, run_qdense
 
@@ -159,3 +160,26 @@ def test_gemv_accumulation_f32_bound(backend):
     got = O.bf16_to_f32(y).astype(np.float64)
     assert np.all(np.abs(got - truth) <= 2.0 ** -8 * np.abs(truth) + 1e-5 * scale)
     assert_bf16_close(y, ref)
+
+
+@pytest.mark.parametrize("M,K,N", [(1, 128, 1), (3, 257, 65), (2, 511, 63), (5, 640, 130), (4, 1030, 201)])
+@pytest.mark.parametrize("w_dtype,x_dtype,axis,B,zp,nf4", [
+    (O.DT_INT8, O.DT_FLOAT32, 0, None, False, False), (O.DT_UINT4, O.DT_FLOAT32, 0, None, True, False),
+    (O.DT_INT4, O.DT_BFLOAT16, 1, 7, True, False), (O.DT_UINT8, O.DT_FLOAT32, 0, 48, False, False),
+    (O.DT_UINT4, O.DT_FLOAT32, 1, 64, False, True), (O.DT_INT4, O.DT_FLOAT32, 1, 16, True, False)])
+def test_chain_kernel_bit_exact(backend, M, K, N, w_dtype, x_dtype, axis, B, zp, nf4):
+    """Few outputs: terms formed by eight waves a chunk of 128 k at a time, added in k order by a ninth
+    (chunks of one, part of one and several; 4-bit rows that start mid-byte): the reference's bits."""
+    p = O.make_problem(M, K, N, w_dtype=w_dtype, x_dtype=x_dtype, scale_dtype=x_dtype, block_axis=axis, block_size=K if B is None else B,
+                       zp=zp, scheme=O.QUANT_NF4 if nf4 else O.QUANT_LINEAR, bias=True, act=O.ACT_NONE, seed=K + N)
+    b = ca.New("exact")  # bf16 x takes the fast kernels otherwise
+    try:
+        r = QDenseRun(b, p)
+        assert r.plan() == "qdense_exact"
+        y, want = r.run(), O.qdense_f32(p)
+        if x_dtype == O.DT_BFLOAT16:
+            assert np.array_equal(y, O.bf16_round(want))
+        else:
+            assert np.array_equal(y.view(np.uint32), want.view(np.uint32))
+    finally:
+        b.Finalize()
