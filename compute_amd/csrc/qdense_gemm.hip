@@ -9,8 +9,8 @@
 // with one group for per-channel scales; every product x*w is exact in f32 (bf16 x, |w| < 256),
 // so only the summation order differs from the reference.  With groups, the MFMAs accumulate
 // into a second set of registers that is folded into the total with the group's scales
-// (acc += accg * s[g]): with bf16 scales after every 64-row block (its first MFMAs start from
-// zero, so nothing is cleared), with f32 scales at the group's last block.
+// (acc += accg * s[g]) after every 64-row block or pair of blocks, whose first MFMAs start from
+// zero, so nothing is cleared.
 //
 // Tiling.  A workgroup (8 waves, two per SIMD) computes a 256 x 128 output tile (or, RB = 2, 128 x
 // 128 with 32 rows per wave: gemm_plan); wave w owns rows [64 wr, 64 wr + 64) x columns [64 wc, 64 wc + 64) with wr = w % 4, wc = w / 4.  K advances
@@ -189,17 +189,20 @@ __device__ __forceinline__ void store_tile(const f32x4_t (&acc)[RB][4], const fl
   }
 }
 
-// FB (scale groups with bf16 scales): every block's MFMA sums start from zero (C operand 0) and
-// are folded into the total with the scales of the block's group at the block's end, so there is
-// no clearing and no per-block branch (a group of G = 64 j rows is folded j times, once per
-// block).  Otherwise groups are counted at run time and the sums cleared after each fold.
+// FB (scale groups): every block's MFMA sums start from zero (C operand 0) and are folded into the
+// total with the scales of the block's group at the block's end, so there is no clearing and no
+// per-block branch (a group of G = 64 j rows is folded j times, once per block).  Otherwise (f32
+// scales off 16-byte alignment) groups are counted at run time and the sums cleared after each fold.
+// HF: f32 scales (else bf16).
+// F2 (with FB, groups of an even number of blocks): folded after every second block.  A fold waits
+// for the MFMAs in flight and stands between two blocks of every wave: x [1333,4096] x Int4 g128
+// [4096,14336] 275 -> 198 us, [97,4096] 42 -> 31, int8 g128 [2048,4096] 330 -> 252.
 // H (with FB): scale groups of 32 rows, two per 64-row block: each step's sums start from zero and
-// are folded with their own group's scales (after step 0 and at the block's end); HF: those
-// scales in f32 (else bf16).
-template <int BK, int RB, bool GRP, bool FB = false, bool H = false, bool HF = false>
+// are folded with their own group's scales (after step 0 and at the block's end).
+template <int BK, int RB, bool GRP, bool FB = false, bool H = false, bool HF = false, bool F2 = false>
 __global__ __launch_bounds__(kThreads) void qdense_gemm_kernel(GemmArgs a) {
   static_assert(!H || (GRP && FB), "32-row groups: the fold-every-step form");
-  static_assert(!HF || H, "f32 scales for 32-row groups only");
+  static_assert(!HF || FB, "f32 scales of the fold-every-block forms");
   constexpr int PF = kPf;
   constexpr int kXDma = kXDmaOf<RB>;
   constexpr int BN = kBN;
@@ -388,7 +391,9 @@ __global__ __launch_bounds__(kThreads) void qdense_gemm_kernel(GemmArgs a) {
   for (int c = 0; c < NC; ++c) sg[c] = 0.f;
   auto load_sg = [&](int g) __attribute__((always_inline)) {
     g = min(g, a.K / (kBK * max(a.gpb, 1)) - 1);
-    if constexpr (HF) {
+    if constexpr (HF && !H) {
+      sgf = *(const f32x4_t*)((const float*)a.scale + (size_t)g * N + scol);
+    } else if constexpr (HF) {
       // The block's two scale rows (groups 2g and 2g + 1), one 16-byte load each.
       sgf = *(const f32x4_t*)((const float*)a.scale + (size_t)(2 * g) * N + scol);
       sgf2 = *(const f32x4_t*)((const float*)a.scale + (size_t)(2 * g + 1) * N + scol);
@@ -458,7 +463,7 @@ __global__ __launch_bounds__(kThreads) void qdense_gemm_kernel(GemmArgs a) {
       }
   };
   auto fold = [&](int g_next) __attribute__((always_inline)) {
-    fold_sums(H ? sgw2 : sgw, sgf2);  // H: the block's second group (its first was folded after step 0)
+    fold_sums(H ? sgw2 : sgw, H ? sgf2 : sgf);  // H: the block's second group (its first was folded after step 0)
     load_sg(g_next);
   };
 
@@ -486,7 +491,7 @@ __global__ __launch_bounds__(kThreads) void qdense_gemm_kernel(GemmArgs a) {
     constexpr int S = U % PF, S2 = (U + 2) % PF, B = U % 2;
     const int xb = (int)((unsigned)kb % XB), xb1 = xb == XB - 1 ? 0 : xb + 1;
     // FB: the block's first step starts its sums from zero (the C operand 0).
-    using Fresh = std::integral_constant<bool, FB>;
+    using Fresh = std::integral_constant<bool, FB && (!F2 || U % 2 == 0)>;
     using Acc = std::integral_constant<bool, false>;
     read_step(xb, B, 1, A1, B1);
     mma_step(A0, B0, Fresh{});
@@ -524,15 +529,16 @@ __global__ __launch_bounds__(kThreads) void qdense_gemm_kernel(GemmArgs a) {
       __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);  // MFMA
     }
     __builtin_amdgcn_sched_barrier(0);
-    if constexpr (GRP && FB) {
+    if constexpr (GRP && FB && (!F2 || U % 2 == 1)) {
       // Every block's sums are folded with its group's scales; the scale row of the next block
       // advances every a.gpb blocks (scalar countdown, no branch).
-      const int last = --g_left == 0;
+      g_left -= F2 ? 2 : 1;
+      const int last = g_left == 0;
       g_left = last ? a.gpb : g_left;
       g_idx += last;
       fold(g_idx);
       __builtin_amdgcn_sched_barrier(0);
-    } else if constexpr (GRP) {
+    } else if constexpr (GRP && !FB) {
       if (--g_left == 0) {
         g_left = a.gpb;
         fold(++g_idx);
@@ -682,7 +688,7 @@ bool qdense_gemm_fits(const QDenseDesc& d) {
 // K slices that fill one round, and both tile heights are priced, in tenths of a 256-row tile's
 // 64-row block (1.4 us with scale groups, 0.85 us per channel; a 128-row tile's is 0.8 of it), with
 // what the slices' completion was measured to add.  x [97,4096] x [4096,14336] Int4 g128 89 -> 42 us
-// (112 tiles of 128 rows in two slices, was 112 of 256 rows), [97,14336] x 4096 294 -> 43 (7 slices),
+// (before F2; 112 tiles of 128 rows in two slices, was 112 of 256 rows), [97,14336] x 4096 294 -> 43 (7 slices),
 // [512,4096] x 4096 91 -> 42, [512,14336] x 4096 303 -> 96 (256-row tiles in four slices); int8 per
 // channel [256,4096] x 4096 57 -> 25; shapes that fill the CUs keep the 256-row tiles (1333 rows,
 // N = 14336: 271 us against 345 with 128-row tiles).
@@ -761,7 +767,6 @@ int qdense_gemm_run(mx_backend* b, const QDenseDesc& d, const char* name) {
   }
   const int grid = (int)(pl.whole + parts);
   hipStream_t st = b->stream;
-  // bf16 group scales: the fold-every-block kernel; f32 group scales count blocks at run time.
   auto go = [&](auto kind, auto rbc) {
     constexpr int BK = decltype(kind)::value, RB = decltype(rbc)::value;
     if (!grouped)
@@ -770,8 +775,15 @@ int qdense_gemm_run(mx_backend* b, const QDenseDesc& d, const char* name) {
       dispatch(qdense_gemm_kernel<BK, RB, true, true, true, true>, grid, kThreads, 0, st, ga);
     else if (half)
       dispatch(qdense_gemm_kernel<BK, RB, true, true, true>, grid, kThreads, 0, st, ga);
+    else if (d.s_dt == MX_DTYPE_FLOAT32 && (uintptr_t)d.scale % 16 == 0)
+      // Not uint4 in 256-row tiles: the pair form spills 120 bytes a lane there ([512,4096] x 14336
+      // 130 us, 94 with a fold per block).
+      ga.gpb % 2 == 0 && !(BK == kBU4 && RB == 4)
+          ? dispatch(qdense_gemm_kernel<BK, RB, true, true, false, true, !(BK == kBU4 && RB == 4)>, grid, kThreads, 0, st, ga)
+          : dispatch(qdense_gemm_kernel<BK, RB, true, true, false, true>, grid, kThreads, 0, st, ga);
     else if (d.s_dt == MX_DTYPE_BFLOAT16)
-      dispatch(qdense_gemm_kernel<BK, RB, true, true>, grid, kThreads, 0, st, ga);
+      ga.gpb % 2 == 0 ? dispatch(qdense_gemm_kernel<BK, RB, true, true, false, false, true>, grid, kThreads, 0, st, ga)
+                      : dispatch(qdense_gemm_kernel<BK, RB, true, true>, grid, kThreads, 0, st, ga);
     else
       dispatch(qdense_gemm_kernel<BK, RB, true>, grid, kThreads, 0, st, ga);
   };

@@ -161,3 +161,17 @@ def test_tiles_in_k_slices(backend, M, K, N, w_dtype, G, s_dtype):
     out = backend.BufferFromFlatData(0, np.zeros(M * N, np.uint16), ca.Shape(ca.BFloat16, M, N))
     backend.QDenseNoAlloc(r.args(out))
     assert np.array_equal(out.ToFlatData().reshape(M, N), y)
+
+
+@pytest.mark.parametrize("M,N", [(70, 144), (520, 2320)])
+@pytest.mark.parametrize("w_dtype", [O.DT_INT8, O.DT_INT4, O.DT_UINT4])
+@pytest.mark.parametrize("G,s_dtype", [(128, O.DT_BFLOAT16), (384, O.DT_FLOAT32), (128, O.DT_FLOAT32), (192, O.DT_FLOAT32)])
+def test_scale_groups_of_block_pairs(backend, M, N, w_dtype, G, s_dtype):
+    """Groups of 2 and 6 blocks of 64 rows (folded after every second block) and of 3 (every block),
+    with both tile heights; 18 blocks, whole and in slices."""
+    p = O.make_problem(M, 1152, N, w_dtype=w_dtype, block_axis=0, block_size=G, scale_dtype=s_dtype, bias=True,
+                       scale_range=(0.002, 0.02), seed=M + G)
+    r = QDenseRun(backend, p)
+    assert r.plan().startswith("qdense_gemm_mfma")
+    y = check_rows(r, threads=8, what=f"{w_dtype} G={G}")
+    assert np.array_equal(y, r.run())
