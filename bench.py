@@ -46,7 +46,6 @@ sys.path.insert(0, ROOT)
 
 HBM_PEAK_GBS = 8000.0
 BF16_PEAK_TFLOPS = 2500.0
-F32_PEAK_TFLOPS = 157.3
 MALL_BYTES = 256 << 20
 METRIC = "QuantizedDense GB/s & TFLOP/s vs MI355X roofline; µs/call at decode+prefill"
 
@@ -180,11 +179,10 @@ def hbm_roofline(nbytes: float, us: float, traffic):
             "frac": round(achieved / HBM_PEAK_GBS, 4), "traffic": traffic}
 
 
-def mfma_roofline(flops: float, us: float, traffic, peak: float = None):
-    peak = peak or BF16_PEAK_TFLOPS
+def mfma_roofline(flops: float, us: float, traffic):
     achieved = flops / (us * 1e-6) / 1e12
-    return {"bound": "mfma", "achieved": round(achieved, 1), "peak": peak, "unit": "TFLOP/s",
-            "frac": round(achieved / peak, 4), "traffic": traffic}
+    return {"bound": "mfma", "achieved": round(achieved, 1), "peak": BF16_PEAK_TFLOPS, "unit": "TFLOP/s",
+            "frac": round(achieved / BF16_PEAK_TFLOPS, 4), "traffic": traffic}
 
 
 def _cpu_model() -> str:
@@ -297,12 +295,12 @@ def extra_entry(wl, r):
         e["TFLOPs_kernel"] = round(wl.flops() / (r["kernel_us"] * 1e-6) / 1e12, 1)
         e["roofline"] = mfma_roofline(wl.flops(), r["kernel_us"], traffic_for(wl.name))
     elif wl.name.startswith("R3"):
-        # f32 x: the dequantised weights are contracted on the f32 matrix cores; the whole call
-        # (dequantisation, contraction, epilogue) priced against the dense f32 MFMA peak.
+        # f32 x in three exact bf16 parts: three bf16 MFMA products per term, priced against the dense
+        # bf16 MFMA peak.
         e["TFLOPs_call"] = round(wl.flops() / (r["kernel_us_per_step"] * 1e-6) / 1e12, 1)
         e["kernels"] = {k: {"per_call": round(v["launches_per_step"], 2), "avg_us": round(v["avg_us"], 3)}
                         for k, v in r["kernels"].items()}
-        e["roofline"] = mfma_roofline(wl.flops(), r["kernel_us_per_step"], traffic_for(wl.name), F32_PEAK_TFLOPS)
+        e["roofline"] = mfma_roofline(3 * wl.flops(), r["kernel_us_per_step"], traffic_for(wl.name))
     elif wl.name.startswith("C5"):
         # Whole graph per call: the three quantized projections dominate; price one call's device
         # time (the timed region per call, all kernels and the gaps between them) against HBM.
