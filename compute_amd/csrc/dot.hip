@@ -560,7 +560,7 @@ struct DotSource {
     }
   }
   template <class TailT>
-  __device__ __forceinline__ void stage(const sg::Args& a, sg::Block b, const Regs& R, const float*, char* Bs, float& big, TailT) const {
+  __device__ __forceinline__ void stage(const sg::Args& a, sg::Block b, const Regs& R, const float*, char* Bs, TailT) const {
     float v[8];
 #pragma unroll
     for (int e = 0; e < 8; ++e) {
@@ -570,10 +570,7 @@ struct DotSource {
     }
     uint32_t h[4], m[4], l[4];
 #pragma unroll
-    for (int q = 0; q < 4; ++q) {
-      big = fmaxf(fmaxf(fabsf(v[2 * q]), fabsf(v[2 * q + 1])), big);
-      sg::split2(v[2 * q], v[2 * q + 1], h[q], m[q], l[q]);
-    }
+    for (int q = 0; q < 4; ++q) sg::split2(v[2 * q], v[2 * q + 1], h[q], m[q], l[q]);
     if constexpr (BT) {
       char* dst = Bs + sg::chunk_at(p, j);
       *(sg::u32x4_v*)dst = sg::u32x4_v{h[0], h[1], h[2], h[3]};

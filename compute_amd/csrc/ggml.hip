@@ -504,7 +504,7 @@ struct GgmlSource {
   // Block scales are used as the reference uses them: every product and difference of a value
   // rounded to f32 (most are exact).
   template <class TailT>
-  __device__ __forceinline__ void stage(const sg::Args& a, sg::Block b, const Regs& R, const float* table, char* Bs, float& big, TailT) const {
+  __device__ __forceinline__ void stage(const sg::Args& a, sg::Block b, const Regs& R, const float* table, char* Bs, TailT) const {
     const int s = (b.k % vpb) >> 5;
     float d, m = 0.0f;
     if constexpr (T == MX_GGML_Q4_K) {
@@ -544,7 +544,6 @@ struct GgmlSource {
           v[e] = mul_rn(d, f);
           if constexpr (T == MX_GGML_Q4_K) v[e] = add_rn(v[e], -m);
         }
-        big = fmaxf(fmaxf(fabsf(v[0]), fabsf(v[1])), big);  // past the limit only for an infinite block scale
         uint32_t hh, mm, ll;
         sg::split2(v[0], v[1], hh, mm, ll);
         h[i] = hh;

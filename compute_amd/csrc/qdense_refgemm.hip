@@ -115,7 +115,7 @@ struct RgSource {
       return word_f32(s[c % kScales], sh[c % kScales], bf);
   }
   template <class TailT>
-  __device__ __forceinline__ void stage(const Args& a, Block b, const Regs& R, const float* table, char* Bs, float& big, TailT) const {
+  __device__ __forceinline__ void stage(const Args& a, Block b, const Regs& R, const float* table, char* Bs, TailT) const {
     const bool sbf = a.s_dt == MX_DTYPE_BFLOAT16, zbf = a.zp_dt == MX_DTYPE_BFLOAT16;
 #pragma unroll
     for (int c = 0; c < CT; ++c) {
@@ -134,8 +134,6 @@ struct RgSource {
         }
       }
       if constexpr (FORM == kWeight) {
-        big = fmaxf(fmaxf(fabsf(v[0]), fabsf(v[1])), big);
-        big = fmaxf(fmaxf(fabsf(v[2]), fabsf(v[3])), big);
         uint32_t h0, m0, l0, h1, m1, l1;
         split2(v[0], v[1], h0, m0, l0);
         split2(v[2], v[3], h1, m1, l1);
@@ -149,11 +147,10 @@ struct RgSource {
       }
     }
   }
-  // The weight factor of (k, n) as the reference forms it (column form: without its scale).
+  // The weight factor of (k, n) as the reference forms it.
   __device__ __forceinline__ float value(const Args& a, int k, int n, const float* table) const {
     const int q = decode_weight(a.w, (int64_t)k * a.N + n, WDT);
     const float wf = KIND == kNf4 ? table[(uint32_t)q & 15u] : (float)q;
-    if constexpr (FORM == kColumn) return wf;
     const int64_t i = SM == kRgCols ? (int64_t)(k / a.B) * a.N + n : (int64_t)k * a.nb + n / a.B;
     const float ws = mul_rn(wf, elem(a.scale, i, a.s_dt));
     return kZp ? add_rn(ws, elem(a.zp, i, a.zp_dt)) : ws;

@@ -26,9 +26,11 @@
 // Column n of the tile lies in LDS row (n & 3) * 32 + (n >> 2): MFMA column set c of wave half wn
 // holds columns 64 wn + 4 cg + c, so a lane ends with four consecutive columns of each of its rows.
 //
-// Infinite operands (and finite ones that a product with the scale takes past f32) cannot be split
-// (the parts would meet as inf * 0): staging a value past kSplitMax sets a flag, and a flagged tile
-// is summed again by f32 FMAs over its K range before the epilogue.  NaN passes through the parts.
+// Infinities, and finite operands, products or sums past the range of the parts, leave sums that are
+// not finite (the parts of an infinity are inf, NaN, NaN; leading and lower products that overflow meet
+// as inf - inf): a wave that ends with such sums forms those again by f32 FMAs in k order, each term
+// with the weight factor as the reference rounds it, before the epilogue.  Rows with a NaN in x are
+// left as they are.
 #pragma once
 
 #include "device_common.h"
@@ -51,9 +53,6 @@ constexpr int kPartBytes = kBM * kBN * 4;  // one partial tile
 // Partial tiles of a split K: the most that the allocation-free entry point's static scratch holds
 // (the split is the same for both entry points, so their results are the same bits).
 constexpr int kMaxParts = (int)((MX_QDENSE_NOALLOC_SCRATCH_BYTES - kCounterBytes) / kPartBytes);
-
-// The largest magnitude that rounds to a finite bf16.
-#define MX_SPLIT_MAX __uint_as_float(0x7F7F7FFFu)
 
 struct Args {
   const void* x;      // [M, K] f32 or bf16
@@ -121,10 +120,9 @@ __device__ __forceinline__ float elem(const void* p, int64_t i, int dt) {
 // P: the operand policy.  P::kXbf bf16 x (else f32); P::kPA, P::kPB parts of x and of the weights;
 // P::kRow each x value multiplied by its row's scale of the tile's column block before the split
 // (reference layout, one block per tile), P::kZp zero points (row form: summed beside the product);
-// P::kCol one scale per column, applied to the sums; P::Regs, load, stage: a thread's weights of a
-// block, their loads, and their parts into LDS (kTail: zeros past K; `big` takes the largest
-// magnitude); P::value: the f32 weight factor of one (k, n); P::table_value: the 16 entries of the
-// lookup table.
+// P::kCol one scale per column, applied to a slice's sums; P::Regs, load, stage: a thread's weights of a
+// block, their loads, and their parts into LDS (kTail: zeros past K); P::value: the f32 weight
+// factor of one (k, n), its scale included; P::table_value: the 16 entries of the lookup table.
 // NW: waves of the workgroup, 4 (2 x 2 waves of 64 x 64) or 8 (4 x 2 waves of 32 x 64).
 // A block of K: its first row and how many of its rows the block before it holds (the last block of
 // a K that is no multiple of 32).
@@ -144,7 +142,7 @@ __global__ __launch_bounds__(64 * NW, 2) void split_gemm_kernel(Args a) {
   __shared__ __attribute__((aligned(16))) float ring[P::kRow ? 2 : 1][2][kBK];  // scales, zero points of a block's rows
   __shared__ float zrow[P::kRow ? kBM : 1];
   __shared__ float table[16];
-  __shared__ int flag;
+  __shared__ int last_slice;
 
   // Workgroups go round-robin over the 8 XCDs: each XCD takes a contiguous run of the whole tiles
   // (M-major: its tiles share x rows in its L2) and one of the tail items.
@@ -167,7 +165,6 @@ __global__ __launch_bounds__(64 * NW, 2) void split_gemm_kernel(Args a) {
   const int M = a.M, K = a.K, N = a.N;
   const int row0 = 16 * RB * wm;  // the wave's first row in the tile
   if (t < 16) table[t] = P::table_value(t);
-  if (t == 16) flag = 0;
 
   const int kb0 = slice * kpb, kb1 = min(kb0 + kpb, (K + kBK - 1) / kBK);
 
@@ -190,7 +187,7 @@ __global__ __launch_bounds__(64 * NW, 2) void split_gemm_kernel(Args a) {
       if constexpr (!P::kXbf) R.v[i][1] = *(const u32x4_v*)(base + xoff[i] + 16);
     }
   };
-  float zacc[XR], big = 0.0f;
+  float zacc[XR];
 #pragma unroll
   for (int i = 0; i < XR; ++i) zacc[i] = 0.0f;
   // With kTail, the values that the block before holds are zero (whole runs of 8 bf16 or 4 f32).
@@ -224,8 +221,6 @@ __global__ __launch_bounds__(64 * NW, 2) void split_gemm_kernel(Args a) {
 #pragma unroll
           for (int e = 0; e < 8; ++e) v[e] = mul_rn(v[e], s[e]);
         }
-#pragma unroll
-        for (int e = 0; e < 8; e += 2) big = fmaxf(fmaxf(fabsf(v[e]), fabsf(v[e + 1])), big);
         u32x4_v h, m, l;
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
@@ -324,10 +319,10 @@ __global__ __launch_bounds__(64 * NW, 2) void split_gemm_kernel(Args a) {
   src.load(a, block(kb0), W);
   store_row_scale(0);
   load_row_scale(block(kb0 + 1));
-  __syncthreads();  // the table, the flag and block kb0's row scales are written
+  __syncthreads();  // the table and block kb0's row scales are written
   store_row_scale(1);
   stage_x(0, block(kb0), X, sm[0], Tail{});
-  src.stage(a, block(kb0), W, table, sm[0] + PA * kPlane, big, Tail{});
+  src.stage(a, block(kb0), W, table, sm[0] + PA * kPlane, Tail{});
   load_x(block(kb0 + 1), X);
   src.load(a, block(kb0 + 1), W);
   load_row_scale(block(kb0 + 2));
@@ -338,7 +333,7 @@ __global__ __launch_bounds__(64 * NW, 2) void split_gemm_kernel(Args a) {
     char* nxt = sm[cur ^ 1];
     compute(sm[cur]);
     stage_x(cur ^ 1, block(kb + 1), X, nxt, tail);
-    src.stage(a, block(kb + 1), W, table, nxt + PA * kPlane, big, tail);
+    src.stage(a, block(kb + 1), W, table, nxt + PA * kPlane, tail);
     load_x(block(kb + 2), X);
     src.load(a, block(kb + 2), W);
     store_row_scale(cur);
@@ -368,49 +363,84 @@ __global__ __launch_bounds__(64 * NW, 2) void split_gemm_kernel(Args a) {
 #pragma unroll
       for (int c = 0; c < 4; ++c) acc[i][c] = total[i][c] + (acc[i][c] + low[i][c]);
   }
-  if (big > MX_SPLIT_MAX) flag = 1;
-  __syncthreads();
 
   const int ncol = n0 + 64 * wn + 4 * cg;  // this lane's four columns
-  if constexpr (P::kRow) {
-    if constexpr (P::kZp) {  // x . zp of each row, added to all of its columns
+  if constexpr (P::kZp && P::kRow) {  // x . zp of each row, added to all of its columns
 #pragma unroll
-      for (int i = 0; i < XR; ++i) {
-        float z = zacc[i];
-        z += __shfl_xor(z, 1);
-        z += __shfl_xor(z, 2);
-        if (xc == 0) zrow[xr + 64 * i] = z;
-      }
-      __syncthreads();
-#pragma unroll
-      for (int rb = 0; rb < RB; ++rb)
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          const float z = zrow[row0 + 16 * rb + 4 * kq + r];
-#pragma unroll
-          for (int c = 0; c < 4; ++c) acc[rb][c][r] += z;
-        }
+    for (int i = 0; i < XR; ++i) {
+      float z = zacc[i];
+      z += __shfl_xor(z, 1);
+      z += __shfl_xor(z, 2);
+      if (xc == 0) zrow[xr + 64 * i] = z;
     }
-  }
-  if (flag) {  // uniform over the workgroup
+    __syncthreads();
 #pragma unroll
     for (int rb = 0; rb < RB; ++rb)
 #pragma unroll
-      for (int c = 0; c < 4; ++c) acc[rb][c] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-#pragma unroll 1
-    for (int k = kb0 * kBK; k < min(K, kb1 * kBK); ++k) {
-      float wv[4];
+      for (int r = 0; r < 4; ++r) {
+        const float z = zrow[row0 + 16 * rb + 4 * kq + r];
 #pragma unroll
-      for (int c = 0; c < 4; ++c) wv[c] = src.value(a, k, min(ncol + c, N - 1), table);
+        for (int c = 0; c < 4; ++c) acc[rb][c][r] += z;
+      }
+  }
+  if constexpr (P::kCol) {
+#pragma unroll
+    for (int c = 0; c < 4; ++c) {
+      const float s = elem(a.scale, min(ncol + c, N - 1), a.s_dt);
 #pragma unroll
       for (int rb = 0; rb < RB; ++rb)
 #pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          const int m = min(m0 + row0 + 16 * rb + 4 * kq + r, M - 1);
-          const float xv = elem(a.x, (int64_t)m * K + k, P::kXbf ? MX_DTYPE_BFLOAT16 : MX_DTYPE_FLOAT32);
+        for (int r = 0; r < 4; ++r) acc[rb][c][r] = mul_rn(acc[rb][c][r], s);
+    }
+  }
+  auto finite = [](float v) { return fabsf(v) < __builtin_inff(); };
+  uint64_t redo = 0;  // the wave's rows that hold such sums
 #pragma unroll
-          for (int c = 0; c < 4; ++c) acc[rb][c][r] = __builtin_fmaf(xv, wv[c], acc[rb][c][r]);
-        }
+  for (int rb = 0; rb < RB; ++rb)
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      bool bad = false;
+#pragma unroll
+      for (int c = 0; c < 4; ++c) bad |= !finite(acc[rb][c][r]);
+      const uint64_t lanes = __ballot(bad);
+#pragma unroll
+      for (int q = 0; q < 4; ++q)
+        if (lanes >> (16 * q) & 0xFFFFu) redo |= (uint64_t)1 << (16 * rb + 4 * q + r);
+    }
+  // Row by row, a column per lane (0.7 ms a row of a tile at K = 4096, bound by the latency of the loads).
+  const int kbeg = kb0 * kBK, kend = min(K, kb1 * kBK);
+  for (; redo; redo &= redo - 1) {
+    const int i = __builtin_ctzll(redo), m = min(m0 + row0 + i, M - 1);
+    auto xat = [&](int k) { return elem(a.x, (int64_t)m * K + k, P::kXbf ? MX_DTYPE_BFLOAT16 : MX_DTYPE_FLOAT32); };
+    bool nan = false;  // a NaN in the row of x: the sums are NaN, as they should be
+    for (int k = kbeg; k < kend && !nan; k += 256) {
+      float v[4];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) v[e] = xat(min(k + 64 * e + lane, kend - 1));
+      nan = __any(v[0] != v[0] || v[1] != v[1] || v[2] != v[2] || v[3] != v[3]);
+    }
+    if (nan) continue;
+    const int n = min(n0 + 64 * wn + lane, N - 1);
+    float sum = 0.0f;
+#pragma unroll 1
+    for (int k = kbeg; k < kend; k += 4) {  // K is a multiple of 4
+      float xv[4], wv[4];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        xv[e] = xat(k + e);
+        wv[e] = src.value(a, k + e, n, table);
+      }
+#pragma unroll
+      for (int e = 0; e < 4; ++e) sum = __builtin_fmaf(xv[e], wv[e], sum);
+    }
+#pragma unroll
+    for (int c = 0; c < 4; ++c) {
+      const float v = __shfl(sum, 4 * cg + c);
+#pragma unroll
+      for (int rb = 0; rb < RB; ++rb)
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+          if (i == 16 * rb + 4 * kq + r && !finite(acc[rb][c][r])) acc[rb][c][r] = v;
     }
   }
 
@@ -431,10 +461,10 @@ __global__ __launch_bounds__(64 * NW, 2) void split_gemm_kernel(Args a) {
     if (t == 0) {
       const uint32_t prev = __hip_atomic_fetch_add(&a.ctr[tile - a.whole], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
       if (prev + 1u == (uint32_t)a.S) __hip_atomic_store(&a.ctr[tile - a.whole], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      flag = prev + 1u == (uint32_t)a.S;
+      last_slice = prev + 1u == (uint32_t)a.S;
     }
     __syncthreads();
-    if (!flag) return;
+    if (!last_slice) return;
 #pragma unroll
     for (int rb = 0; rb < RB; ++rb)
 #pragma unroll
@@ -450,16 +480,13 @@ __global__ __launch_bounds__(64 * NW, 2) void split_gemm_kernel(Args a) {
     }
   }
 
-  // Epilogue: column scales, bias (added after the sum), the reference activation, x's dtype.  The
+  // Epilogue: bias (added after the sum), the reference activation, x's dtype.  The
   // activation's code is there once: each half of the tile goes through LDS (free after the loop's
   // last barrier) to a rolled loop over four consecutive columns of a row.
-  float cs[4] = {1.f, 1.f, 1.f, 1.f}, bi[4] = {0.f, 0.f, 0.f, 0.f};
-  if (ncol < N) {
+  float bi[4] = {0.f, 0.f, 0.f, 0.f};
+  if (a.bias && ncol < N) {
 #pragma unroll
-    for (int c = 0; c < 4; ++c) {
-      if constexpr (P::kCol) cs[c] = elem(a.scale, min(ncol + c, N - 1), a.s_dt);
-      if (a.bias) bi[c] = elem(a.bias, min(ncol + c, N - 1), a.b_dt);
-    }
+    for (int c = 0; c < 4; ++c) bi[c] = elem(a.bias, min(ncol + c, N - 1), a.b_dt);
   }
   auto store4 = [&](int m, int n, const float (&y)[4]) __attribute__((always_inline)) {
     const int64_t o = (int64_t)m * N + n;
@@ -474,10 +501,7 @@ __global__ __launch_bounds__(64 * NW, 2) void split_gemm_kernel(Args a) {
       *(f32x4_t*)((float*)a.out + o) = f32x4_t{y[0], y[1], y[2], y[3]};
     }
   };
-  auto finish = [&](float v, int c) __attribute__((always_inline)) {
-    if constexpr (P::kCol) v = mul_rn(v, cs[c]);
-    return a.bias ? add_rn(bi[c], v) : v;
-  };
+  auto finish = [&](float v, int c) __attribute__((always_inline)) { return a.bias ? add_rn(bi[c], v) : v; };
   if (a.act == MX_ACT_NONE) {
     if (ncol >= N) return;
 #pragma unroll

@@ -101,6 +101,57 @@ def test_infinite_and_nan_operands(backend, B, K):
     assert np.all(np.abs(y[fin] - truth[fin]) <= 2.0 ** -22 * np.abs(truth[fin]) + 1e-5 * scale[fin])
 
 
+@pytest.mark.parametrize("K", [1024, 1000])
+@pytest.mark.parametrize("axis,B,zp,nf4", [(1, 64, False, False), (1, 128, False, True), (0, 96, True, False), (1, 7, True, False)])
+def test_infinite_and_nan_bf16_x(backend, axis, B, zp, nf4, K):
+    """bf16 x is one part and meets three parts of each weight factor: an infinity keeps its sign."""
+    p = O.make_problem(260, K, 256, w_dtype=O.DT_UINT4, x_dtype=BF16, scale_dtype=BF16, block_axis=axis, block_size=B, zp=zp,
+                       scheme=O.QUANT_NF4 if nf4 else O.QUANT_LINEAR, bias=True, seed=K + B)
+    x = p.x.copy()
+    x[3, 17], x[140, 5], x[141, 9], x[259, K - 1] = 0x7F80, 0xFF80, 0x7FC0, 0x7F80
+    p = dataclasses.replace(p, x=x)
+    r = QDenseRun(backend, p)
+    assert r.plan() == "qdense_refgemm_f32_mfma"
+    y = O.bf16_to_f32(r.run()).astype(np.float64)
+    with np.errstate(invalid="ignore", over="ignore"):
+        truth, scale = O.qdense_f64(p), O.qdense_f64(p, absolute=True)
+    assert np.array_equal(np.isnan(y), np.isnan(truth)) and np.isnan(truth[141]).all()
+    inf = np.isinf(truth)
+    assert inf[3].any() and inf[140].any() and inf[259].any() and np.array_equal(y[inf], truth[inf])
+    fin = np.isfinite(truth)
+    assert np.all(np.abs(y[fin] - truth[fin]) <= 2.0 ** -8 * np.abs(truth[fin]) + 1e-5 * scale[fin])
+
+
+@pytest.mark.parametrize("axis,B,K,s", [(1, 64, 1024, 1e14), (1, 64, 16388, 1e14), (0, 96, 1024, 1e14), (0, None, 1024, 1e14), (1, 128, 1024, 1e14)])
+def test_finite_operands_that_overflow(backend, axis, B, K, s):
+    """Products of finite operands past f32's range are infinities, not NaN; rows beside them are as
+    close as ever.  (The sums of one row have one sign, so that no infinities cancel.)"""
+    p = O.make_problem(130, K, 144, w_dtype=O.DT_UINT8, x_dtype=F32, scale_dtype=F32, block_axis=axis, block_size=K if B is None else B,
+                       bias=True, scale_range=(0.5 * s, s), seed=K)
+    x = np.abs(p.x) + np.float32(0.1)
+    x[1] *= np.float32(1e25)
+    x[2] *= np.float32(-1e25)
+    p = dataclasses.replace(p, x=x, w=np.maximum(p.w, 1))
+    y = QDenseRun(backend, p).run()
+    assert np.all(np.isposinf(y[1])) and np.all(np.isneginf(y[2]))
+    rest = np.r_[0, 3:130]
+    truth, scale = O.qdense_f64(p, rest), O.qdense_f64(p, rest, absolute=True)
+    assert np.all(np.abs(y[rest].astype(np.float64) - truth) <= 2.0 ** -22 * np.abs(truth) + 1e-5 * scale)
+
+
+def test_column_sums_past_the_range_before_their_scale(backend):
+    """One scale per column, applied to the sums: sums of x * w past f32's range whose scaled terms and
+    result are in range."""
+    p = O.make_problem(130, 1024, 144, w_dtype=O.DT_UINT8, x_dtype=F32, scale_dtype=F32, block_axis=0, block_size=1024, bias=True,
+                       scale_range=(1e-6, 1e-5), seed=8)
+    x = np.abs(p.x)
+    x[5] = np.float32(1.2e36)
+    p = dataclasses.replace(p, x=x)
+    r = QDenseRun(backend, p)
+    assert r.plan() == "qdense_refgemm_f32_mfma"
+    check(p, r.run())
+
+
 @pytest.mark.parametrize("x_dtype,act", [(F32, O.ACT_NONE), (BF16, O.ACT_RELU)])
 def test_output_aligned_to_its_elements_only(backend, x_dtype, act):
     """An output array that starts one element past a 16-byte boundary."""
@@ -162,6 +213,18 @@ def test_few_rows(backend, M, K, N, axis, B, zp):
     assert np.all(np.abs(y - truth) <= 2.0 ** -22 * np.abs(truth) + 3e-6 * scale)
 
 
+def dot_general(backend, x, w, transposed):
+    """x [M, K] . w [K, N] through DotGeneral, w passed as it is or transposed."""
+    bld = backend.Builder("dot")
+    f = bld.Main()
+    vals = [x, w.T if transposed else w]
+    shapes = [ca.Shape(ca.Float32, *v.shape) for v in vals]
+    a, b = (f.Parameter(n, s) for n, s in zip("ab", shapes))
+    f.Return([f.DotGeneral(a, [1], [], b, [1 if transposed else 0], [])])
+    bufs = [backend.BufferFromFlatData(0, np.ascontiguousarray(v).ravel(), s) for v, s in zip(vals, shapes)]
+    return bld.Compile().Execute(bufs)[0].ToFlatData().reshape(x.shape[0], w.shape[1])
+
+
 @pytest.mark.parametrize("transposed", [True, False])
 @pytest.mark.parametrize("M,K,N", [(96, 115004, 100), (1037, 1028, 1036), (2049, 548, 1000)])
 def test_dot_general_f32(backend, transposed, M, K, N):
@@ -183,3 +246,18 @@ def test_dot_general_f32(backend, transposed, M, K, N):
     assert np.all(np.isposinf(y[M - 1]))
     truth, scale = x[:-1].astype(np.float64) @ w.astype(np.float64), np.abs(x[:-1]).astype(np.float64) @ np.abs(w).astype(np.float64)
     assert np.all(np.abs(y[:-1] - truth) <= 2.0 ** -22 * np.abs(truth) + 3e-6 * scale)
+
+
+@pytest.mark.parametrize("transposed", [True, False])
+def test_dot_general_f32_overflow(backend, transposed):
+    """Rows of x whose products with the right-hand side pass f32's range: infinities, not NaN."""
+    M, K, N = 1024, 1024, 1024
+    rng = np.random.default_rng(7)
+    x, w = np.abs(rng.standard_normal((2, M, K)).astype(np.float32)) + np.float32(0.1)
+    w *= np.float32(1e25)
+    x[1], x[2] = x[1] * np.float32(1e25), x[2] * np.float32(-1e25)
+    y = dot_general(backend, x, w, transposed)
+    assert np.all(np.isposinf(y[1])) and np.all(np.isneginf(y[2]))
+    truth = x.astype(np.float64) @ w.astype(np.float64)
+    rest = np.r_[0, 3:M]
+    assert np.all(np.abs(y[rest] - truth[rest]) <= (2.0 ** -22 + 3e-6) * truth[rest])
