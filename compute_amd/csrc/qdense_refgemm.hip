@@ -5,8 +5,9 @@
 //
 // Three forms, by where the scale enters:
 //   row      reference layout, one column block per 128-column tile (B % 128 == 0 or one block),
-//            linear scheme: x * s is formed and rounded once per (row, k) of the tile, the codes
-//            stay exact; 3 products per term.  Zero points add x . zp, summed in f32 beside it.
+//            linear scheme, no zero points: x * s is formed and rounded once per (row, k) of the
+//            tile, the codes stay exact; 3 products per term.  (With zero points the sums of x*s*w
+//            and x*zp would cancel, codes near the zero point above all.)
 //   column   one scale per output column, linear scheme, no zero points: the sums of x * w, scaled
 //            once; 3 products (1 with bf16 x).
 //   weight   everything else: the weight factor formed as the reference forms it (w*s, w*s + zp
@@ -41,6 +42,7 @@ template <int WDT, int FORM, int SM, int KIND, bool XBF, int NW>
 struct RgSource {
   static constexpr bool kXbf = XBF;
   static constexpr bool kRow = FORM == RgForm::kRow, kCol = FORM == kColumn, kZp = KIND == kZeroPoint;
+  static_assert(KIND == kLinear || FORM == kWeight, "zero points and NF4 are in the weight factor");
   static constexpr int kPA = XBF && FORM != RgForm::kRow ? 1 : 3;
   static constexpr int kPB = FORM == kWeight ? 3 : 1;
   static constexpr bool kI4 = WDT == MX_DTYPE_INT4 || WDT == MX_DTYPE_UINT4;
@@ -178,7 +180,7 @@ int rg_forms(mx_backend* b, const char* name, const QDenseDesc& d, Args& a) {
   if constexpr (KIND == kLinear && SM == kRgCols) {
     if (d.block_size >= d.K) return rg_launch<WDT, kColumn, kRgCols, KIND, XBF>(b, name, a);
   }
-  if constexpr (KIND != kNf4 && SM == kRgBlk) {
+  if constexpr (KIND == kLinear && SM == kRgBlk) {
     if (a.nb == 1 || a.B % kBN == 0) return rg_launch<WDT, RgForm::kRow, kRgBlk, KIND, XBF>(b, name, a);
   }
   return rg_launch<WDT, kWeight, SM, KIND, XBF>(b, name, a);

@@ -119,7 +119,7 @@ __device__ __forceinline__ float elem(const void* p, int64_t i, int dt) {
 
 // P: the operand policy.  P::kXbf bf16 x (else f32); P::kPA, P::kPB parts of x and of the weights;
 // P::kRow each x value multiplied by its row's scale of the tile's column block before the split
-// (reference layout, one block per tile), P::kZp zero points (row form: summed beside the product);
+// (reference layout, one block per tile);
 // P::kCol one scale per column, applied to a slice's sums; P::Regs, load, stage: a thread's weights of a
 // block, their loads, and their parts into LDS (kTail: zeros past K); P::value: the f32 weight
 // factor of one (k, n), its scale included; P::table_value: the 16 entries of the lookup table.
@@ -139,8 +139,7 @@ __global__ __launch_bounds__(64 * NW, 2) void split_gemm_kernel(Args a) {
   constexpr int XR = 8 / NW;  // rows of x per thread and block
   static_assert(!P::kRow || (PA == 3 && PB == 1), "row scales: split x, exact weight codes");
   __shared__ __attribute__((aligned(16))) char sm[2][kBufBytes];
-  __shared__ __attribute__((aligned(16))) float ring[P::kRow ? 2 : 1][2][kBK];  // scales, zero points of a block's rows
-  __shared__ float zrow[P::kRow ? kBM : 1];
+  __shared__ __attribute__((aligned(16))) float ring[P::kRow ? 2 : 1][kBK];  // scales of a block's rows
   __shared__ float table[16];
   __shared__ int last_slice;
 
@@ -187,9 +186,6 @@ __global__ __launch_bounds__(64 * NW, 2) void split_gemm_kernel(Args a) {
       if constexpr (!P::kXbf) R.v[i][1] = *(const u32x4_v*)(base + xoff[i] + 16);
     }
   };
-  float zacc[XR];
-#pragma unroll
-  for (int i = 0; i < XR; ++i) zacc[i] = 0.0f;
   // With kTail, the values that the block before holds are zero (whole runs of 8 bf16 or 4 f32).
   auto stage_x = [&](int slot, Block b, const XRegs& R, char* As, auto tail) __attribute__((always_inline)) {
     constexpr bool kTail = decltype(tail)::value;
@@ -212,12 +208,7 @@ __global__ __launch_bounds__(64 * NW, 2) void split_gemm_kernel(Args a) {
           if constexpr (kTail) v[e] = (e < 4 ? lo : hi) ? v[e] : 0.0f;
         }
         if constexpr (P::kRow) {
-          const float* s = &ring[slot][0][8 * xc];
-          if constexpr (P::kZp) {
-            const float* z = &ring[slot][1][8 * xc];
-#pragma unroll
-            for (int e = 0; e < 8; ++e) zacc[i] = __builtin_fmaf(v[e], z[e], zacc[i]);
-          }
+          const float* s = &ring[slot][8 * xc];
 #pragma unroll
           for (int e = 0; e < 8; ++e) v[e] = mul_rn(v[e], s[e]);
         }
@@ -236,23 +227,19 @@ __global__ __launch_bounds__(64 * NW, 2) void split_gemm_kernel(Args a) {
       }
     }
   };
-  // Row scales and zero points of a block, its row t & 31 by every thread (the copies write the
+  // Row scales of a block, its row t & 31 by every thread (the copies write the
   // same words), into their slot two blocks ahead of their use.
-  uint32_t rs = 0, rz = 0, rssh = 0, rzsh = 0;
-  const bool sbf = a.s_dt == MX_DTYPE_BFLOAT16, zbf = a.zp_dt == MX_DTYPE_BFLOAT16;
+  uint32_t rs = 0, rssh = 0;
+  const bool sbf = a.s_dt == MX_DTYPE_BFLOAT16;
   const int scol = P::kRow ? n0 / a.B : 0;
   auto load_row_scale = [&](Block b) __attribute__((always_inline)) {
     if constexpr (P::kRow) {
       const int64_t i = (int64_t)(b.k + (t & 31)) * a.nb + scol;
       word(a.scale, i, sbf, rs, rssh);
-      if constexpr (P::kZp) word(a.zp, i, zbf, rz, rzsh);
     }
   };
   auto store_row_scale = [&](int slot) __attribute__((always_inline)) {
-    if constexpr (P::kRow) {
-      ring[slot][0][t & 31] = word_f32(rs, rssh, sbf);
-      if constexpr (P::kZp) ring[slot][1][t & 31] = word_f32(rz, rzsh, zbf);
-    }
+    if constexpr (P::kRow) ring[slot][t & 31] = word_f32(rs, rssh, sbf);
   };
 
   // Eight waves leave registers to round less: the products of leading parts and those of the others
@@ -365,24 +352,6 @@ __global__ __launch_bounds__(64 * NW, 2) void split_gemm_kernel(Args a) {
   }
 
   const int ncol = n0 + 64 * wn + 4 * cg;  // this lane's four columns
-  if constexpr (P::kZp && P::kRow) {  // x . zp of each row, added to all of its columns
-#pragma unroll
-    for (int i = 0; i < XR; ++i) {
-      float z = zacc[i];
-      z += __shfl_xor(z, 1);
-      z += __shfl_xor(z, 2);
-      if (xc == 0) zrow[xr + 64 * i] = z;
-    }
-    __syncthreads();
-#pragma unroll
-    for (int rb = 0; rb < RB; ++rb)
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const float z = zrow[row0 + 16 * rb + 4 * kq + r];
-#pragma unroll
-        for (int c = 0; c < 4; ++c) acc[rb][c][r] += z;
-      }
-  }
   if constexpr (P::kCol) {
 #pragma unroll
     for (int c = 0; c < 4; ++c) {

@@ -156,8 +156,8 @@ typedef uint64_t mx_value;
  * fast kernels.  The bf16-x kernels (skinny, prefill GEMM) and the decode GEMV differ from the
  * reference only in summation order.  The prefill plans of the reference layout, f32 x, zero
  * points and NF4 (past 16 to 32 rows and 2^24 multiply-adds), and of GGML rows (past 16 rows), also round each term's weight
- * factor w*s (or w*s+zp) before the product with x (with at least 128 columns per scale block: the
- * factor x*s before the product with w), where the reference rounds (x*w)*s; they
+ * factor w*s (or w*s+zp) before the product with x (with at least 128 columns per scale block and no
+ * zero points: the factor x*s before the product with w), where the reference rounds (x*w)*s; they
  * stay within the f32 accumulation bound of the reference's sum.  Below the fast kernels'
  * thresholds (the decode GEMV from 2^20 weights, and past 64 rows, for widths whose packed rows
  * start mid-word, from 2^24 weights; the f32 dequantise-and-contract paths and the GGML paths

@@ -27,8 +27,8 @@ def check(p, y):
     assert not bad.any(), f"{bad.sum()} outputs outside the bound; worst at {np.argwhere(bad)[0]}"
 
 
-# (x, axis, B, zero point, NF4): the row form (B a multiple of 128, or one block), the column form
-# (one scale per column) and the weight form (everything else).
+# (x, axis, B, zero point, NF4): the row form (B a multiple of 128, or one block; no zero points), the
+# column form (one scale per column) and the weight form (everything else).
 FORMS = [(F32, 1, 128, False, False), (F32, 1, 128, True, False), (BF16, 1, 4096, True, False), (F32, 0, None, False, False),
          (F32, 0, 96, True, False), (BF16, 0, 96, False, False), (F32, 1, 4, True, False), (BF16, 1, 7, True, False),
          (F32, 1, 7, False, False), (F32, 1, 128, False, True)]
@@ -150,6 +150,26 @@ def test_column_sums_past_the_range_before_their_scale(backend):
     r = QDenseRun(backend, p)
     assert r.plan() == "qdense_refgemm_f32_mfma"
     check(p, r.run())
+
+
+@pytest.mark.parametrize("M,K,N,B", [(130, 1024, 272, 128), (130, 1028, 272, 272), (24, 4096, 256, 128)])
+def test_zero_points_that_cancel_the_codes(backend, M, K, N, B):
+    """Asymmetric weights, zp = -z * s with codes at and next to z: the terms are x * ((w - z) * s), and
+    the bound is of these, not of x * w * s and x * zp.  (64 bits: z = 8, so that z * s is exact; the
+    sums' chains are at most 8 + K / 256 + 2 additions, each 2^-24 of the terms' sum.)  A column whose
+    codes are all z is the bias, to the bit."""
+    for z in (8, 7):
+        p = O.make_problem(M, K, N, w_dtype=O.DT_UINT4, x_dtype=F32, scale_dtype=F32, block_axis=1, block_size=B, zp=True, bias=True, seed=K)
+        codes = np.random.default_rng(K).integers(z - 1, z + 2, (K, N))
+        codes[:, ::5] = z
+        p = dataclasses.replace(p, w=O.pack_int4(codes.ravel()), zp=(-np.float32(z) * p.scale).astype(np.float32))
+        r = QDenseRun(backend, p)
+        assert r.plan() == "qdense_refgemm_f32_mfma"
+        y = r.run()
+        assert np.array_equal(y[:, ::5], np.broadcast_to(p.bias[::5], (M, len(range(0, N, 5)))))
+        if z == 8:
+            truth, scale = O.qdense_f64(p), O.qdense_f64(p, absolute=True)
+            assert np.all(np.abs(y - truth) <= 2.0 ** -22 * np.abs(truth) + (10 + K / 256) * 2.0 ** -24 * scale)
 
 
 @pytest.mark.parametrize("x_dtype,act", [(F32, O.ACT_NONE), (BF16, O.ACT_RELU)])
