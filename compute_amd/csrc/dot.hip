@@ -515,6 +515,7 @@ template <bool BT>
 struct DotSource {
   static constexpr bool kXbf = false, kRow = false, kCol = false, kZp = false;
   static constexpr int kPA = 3, kPB = 3;
+  static constexpr bool kLiftW = true;
   struct Regs {
     uint32_t v[8];
   };
@@ -564,7 +565,7 @@ struct DotSource {
     float v[8];
 #pragma unroll
     for (int e = 0; e < 8; ++e) {
-      v[e] = __uint_as_float(R.v[e]);
+      v[e] = __uint_as_float(R.v[e]) * sg::kLift;
       // Values that the block before holds are zero (x is too, but 0 * inf is not).
       if (TailT::value && (BT ? 8 * j + (e & 4) : 4 * j) < b.skip) v[e] = 0.0f;
     }

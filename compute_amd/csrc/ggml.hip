@@ -458,6 +458,7 @@ template <int T, int NW>
 struct GgmlSource {
   static constexpr bool kXbf = false, kRow = false, kCol = false, kZp = false;
   static constexpr int kPA = 3, kPB = 3;
+  static constexpr bool kLiftW = false;  // steps of f16 scales: values are multiples of 2^-24
   static constexpr int vpb = ggml_vpb(T), bpb = ggml_bpb(T), NC = 8 / NW;
   static constexpr bool kNib32 = T == MX_GGML_Q4_0 || T == MX_GGML_IQ4_NL;
   struct Regs {

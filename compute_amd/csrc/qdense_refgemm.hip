@@ -45,6 +45,7 @@ struct RgSource {
   static_assert(KIND == kLinear || FORM == kWeight, "zero points and NF4 are in the weight factor");
   static constexpr int kPA = XBF && FORM != RgForm::kRow ? 1 : 3;
   static constexpr int kPB = FORM == kWeight ? 3 : 1;
+  static constexpr bool kLiftW = FORM == kWeight;
   static constexpr bool kI4 = WDT == MX_DTYPE_INT4 || WDT == MX_DTYPE_UINT4;
   static constexpr bool kSigned = WDT == MX_DTYPE_INT4 || WDT == MX_DTYPE_INT8;
   static constexpr int CT = 16 / NW;
@@ -128,8 +129,8 @@ struct RgSource {
         const int q = code(R.w[e], c);
         if constexpr (FORM == kWeight) {
           const float wf = KIND == kNf4 ? table[(uint32_t)q & 15u] : (float)q;
-          v[e] = mul_rn(wf, scale_of(R.s[e], R.ssh[e], c, sbf));
-          if constexpr (kZp) v[e] = add_rn(v[e], scale_of(R.z[e], R.zsh[e], c, zbf));
+          v[e] = mul_rn(wf, scale_of(R.s[e], R.ssh[e], c, sbf) * kLift);
+          if constexpr (kZp) v[e] = add_rn(v[e], scale_of(R.z[e], R.zsh[e], c, zbf) * kLift);
           if (TailT::value && 4 * j < b.skip) v[e] = 0.0f;  // x is zero there, but 0 * inf is not
         } else {
           v[e] = (float)q;

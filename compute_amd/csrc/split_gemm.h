@@ -1,11 +1,17 @@
 // f32 contraction on the bf16 matrix cores, for products whose operands carry more than bf16's
 // 8 significant bits: every f32 operand is split exactly into three bf16 values (24 bits = 3 x 8),
-//   v = h + m + l,   h = bf16(v), m = bf16(v - h), l = v - h - m,
+//   v = h + m + l,   h = bf16(v), m = bf16(v - h), l = v - h - m
+// (Henry, Tang and Heinecke, "Leveraging the bfloat16 Artificial Intelligence Datatype For
+// Higher-Precision Computations", 2019),
 // and the products of the parts are summed in one f32 accumulator by v_mfma_f32_16x16x32_bf16.
 // A bf16 x and an integer weight code (|code| <= 255) are one part and exact.  Split x against one
 // part takes 3 products per term, against three parts 6 (m*l, l*m and l*l, at most 2^-25 of the
 // term each, are left out).  The bf16 MFMAs have 16 times the rate of v_mfma_f32_16x16x4_f32, so 3
 // products have 5.3 times and 6 products 2.7 times the f32 matrix cores' peak.
+// The split is exact for every f32: the parts hold 2^16 v, so that f32's smallest step, 2^-149, is
+// bf16's, 2^-133 (the matrix cores keep subnormals); unlifted, operands below 2^-110 lose bits (9e-5 of
+// a value at 1e-36).  x times its row's scale is lifted by 2^24: its bits below 2^-149 count, since a
+// code of up to 8 bits comes after it.  The sums are brought back once.
 //
 // What bounds it: matrix-core and VALU issue together (an MFMA keeps the VALU from about 2.5 of its
 // own issue slots; at four VALU instructions per MFMA, the conversions' share with 3 products, the
@@ -53,6 +59,8 @@ constexpr int kPartBytes = kBM * kBN * 4;  // one partial tile
 // Partial tiles of a split K: the most that the allocation-free entry point's static scratch holds
 // (the split is the same for both entry points, so their results are the same bits).
 constexpr int kMaxParts = (int)((MX_QDENSE_NOALLOC_SCRATCH_BYTES - kCounterBytes) / kPartBytes);
+
+constexpr float kLift = 0x1p16f, kLiftRow = 0x1p24f;
 
 struct Args {
   const void* x;      // [M, K] f32 or bf16
@@ -118,6 +126,7 @@ __device__ __forceinline__ float elem(const void* p, int64_t i, int dt) {
 }
 
 // P: the operand policy.  P::kXbf bf16 x (else f32); P::kPA, P::kPB parts of x and of the weights;
+// P::kLiftW whether the weights' parts are lifted (those of f32 weight factors of any size);
 // P::kRow each x value multiplied by its row's scale of the tile's column block before the split
 // (reference layout, one block per tile);
 // P::kCol one scale per column, applied to a slice's sums; P::Regs, load, stage: a thread's weights of a
@@ -211,6 +220,9 @@ __global__ __launch_bounds__(64 * NW, 2) void split_gemm_kernel(Args a) {
           const float* s = &ring[slot][8 * xc];
 #pragma unroll
           for (int e = 0; e < 8; ++e) v[e] = mul_rn(v[e], s[e]);
+        } else {
+#pragma unroll
+          for (int e = 0; e < 8; ++e) v[e] *= kLift;
         }
         u32x4_v h, m, l;
 #pragma unroll
@@ -239,7 +251,7 @@ __global__ __launch_bounds__(64 * NW, 2) void split_gemm_kernel(Args a) {
     }
   };
   auto store_row_scale = [&](int slot) __attribute__((always_inline)) {
-    if constexpr (P::kRow) ring[slot][t & 31] = word_f32(rs, rssh, sbf);
+    if constexpr (P::kRow) ring[slot][t & 31] = word_f32(rs, rssh, sbf) * kLiftRow;
   };
 
   // Eight waves leave registers to round less: the products of leading parts and those of the others
@@ -349,6 +361,13 @@ __global__ __launch_bounds__(64 * NW, 2) void split_gemm_kernel(Args a) {
     for (int i = 0; i < RB; ++i)
 #pragma unroll
       for (int c = 0; c < 4; ++c) acc[i][c] = total[i][c] + (acc[i][c] + low[i][c]);
+  }
+  constexpr float kBack = (PA == 3 ? 1 / (P::kRow ? kLiftRow : kLift) : 1.0f) * (P::kLiftW ? 1 / kLift : 1.0f);
+  if constexpr (kBack != 1.0f) {
+#pragma unroll
+    for (int i = 0; i < RB; ++i)
+#pragma unroll
+      for (int c = 0; c < 4; ++c) acc[i][c] *= kBack;
   }
 
   const int ncol = n0 + 64 * wn + 4 * cg;  // this lane's four columns

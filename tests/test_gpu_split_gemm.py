@@ -27,6 +27,32 @@ def check(p, y):
     assert not bad.any(), f"{bad.sum()} outputs outside the bound; worst at {np.argwhere(bad)[0]}"
 
 
+def dot_general(backend, x, w, transposed):
+    """x [M, K] . w [K, N] through DotGeneral, w passed as it is or transposed."""
+    bld = backend.Builder("dot")
+    f = bld.Main()
+    vals = [x, w.T if transposed else w]
+    shapes = [ca.Shape(ca.Float32, *v.shape) for v in vals]
+    a, b = (f.Parameter(n, s) for n, s in zip("ab", shapes))
+    f.Return([f.DotGeneral(a, [1], [], b, [1 if transposed else 0], [])])
+    bufs = [backend.BufferFromFlatData(0, np.ascontiguousarray(v).ravel(), s) for v, s in zip(vals, shapes)]
+    return bld.Compile().Execute(bufs)[0].ToFlatData().reshape(x.shape[0], w.shape[1])
+
+
+def ggml_dense(backend, t, x, w):
+    """x [M, K] . GGML rows w, through mx_qdense."""
+    (M, K), N = x.shape, w.shape[0]
+    up = lambda v, s: backend.BufferFromFlatData(0, np.ascontiguousarray(v).ravel(), s)
+    out = up(np.zeros(M * N, np.float32), ca.Shape(ca.Float32, M, N))
+    bufs = [up(x, ca.Shape(ca.Float32, M, K)), up(w, ca.Shape(ca.Uint8, *w.shape))]
+    a = ca._lib.mx_qdense_args()
+    a.x, a.w, a.out = bufs[0].DevicePtr(), bufs[1].DevicePtr(), out.DevicePtr()
+    a.M, a.K, a.N, a.x_dtype, a.scheme, a.ggml_type = M, K, N, F32, int(ca.QuantGGML), int(t)
+    assert backend.QDensePlan(a) == "ggml_dequant_f32_mfma"
+    backend.QDense(a)
+    return out.ToFlatData().reshape(M, N)
+
+
 # (x, axis, B, zero point, NF4): the row form (B a multiple of 128, or one block; no zero points), the
 # column form (one scale per column) and the weight form (everything else).
 FORMS = [(F32, 1, 128, False, False), (F32, 1, 128, True, False), (BF16, 1, 4096, True, False), (F32, 0, None, False, False),
@@ -64,6 +90,60 @@ def test_k_slices_with_and_without_allocation(backend, form, M, K, N):
     out = backend.BufferFromFlatData(0, np.zeros(M * N, np.float32), ca.Shape(ca.Float32, M, N))
     backend.QDenseNoAlloc(r.args(out))
     assert np.array_equal(out.ToFlatData().reshape(M, N).view(np.uint32), y.view(np.uint32))
+
+
+# A product's error without its smallest parts is up to 2^-17 of it; with them it is a few roundings,
+# 2^-24 each: of x * s or w * s, of each of up to four sums, and the three products left out.
+ONE_PRODUCT = 2.0 ** -21
+
+
+def one_term_rows(M, K, magnitude, rng):
+    """x with one value of 24 significant bits in each row, at k from 0 to K - 1."""
+    x = np.zeros((M, K), np.float32)
+    k = np.linspace(0, K - 1, M).round().astype(int)
+    x[np.arange(M), k] = rng.uniform(0.5, 2.0, M).astype(np.float32) * np.float32(magnitude)
+    return x
+
+
+@pytest.mark.parametrize("axis,B,zp,nf4", [(1, 128, False, False), (1, 272, False, False), (0, None, False, False), (1, 64, False, False),
+                                           (1, 7, True, False), (0, 96, True, False), (1, 128, True, False), (1, 128, False, True)])
+@pytest.mark.parametrize("magnitude,s", [(1.0, 0.01), (1e-37, 0.01), (1e-3, 1e-34), (1.0, 1e-37)])
+@pytest.mark.parametrize("M,K", [(131, 1048), (70, 8196)])
+def test_every_part_of_every_product(backend, axis, B, zp, nf4, magnitude, s, M, K):
+    """Outputs of a single product each, over every k (K slices and the last part of a block among
+    them), with operands down to the smallest normals: each holds all of its operands' bits.  Against
+    the reference's own roundings, so that w * s + zp has no error of its own."""
+    N = 272
+    p = O.make_problem(M, K, N, w_dtype=O.DT_INT4 if nf4 or B == 64 else O.DT_INT8, x_dtype=F32, scale_dtype=F32, block_axis=axis,
+                       block_size=K if B is None else B, zp=zp, scheme=O.QUANT_NF4 if nf4 else O.QUANT_LINEAR, bias=False,
+                       scale_range=(0.5 * s, 2 * s), seed=M + K)
+    p = dataclasses.replace(p, x=one_term_rows(M, K, magnitude, np.random.default_rng(K)), zp=p.zp * np.float32(20 * s) if zp else None)
+    r = QDenseRun(backend, p)
+    assert r.plan() == "qdense_refgemm_f32_mfma"
+    y, want = r.run().astype(np.float64), O.qdense_f32(p).astype(np.float64)
+    # Results below the smallest normal keep its step, and (x*w)*s may pass through that range before.
+    assert np.all(np.abs(y - want) <= ONE_PRODUCT * np.abs(want) + 2.0 ** -147)
+    assert np.count_nonzero(y) > 0.8 * y.size
+
+
+@pytest.mark.parametrize("t", [ca.GGMLQ4_0, ca.GGMLQ8_0, ca.GGMLIQ4NL, ca.GGMLQ4_K, ca.GGMLQ6_K])
+@pytest.mark.parametrize("magnitude", [1.0, 1e-34])
+def test_every_part_of_every_ggml_product(backend, t, magnitude):
+    rng = np.random.default_rng(int(t))
+    M, K, N = 70, 2048, 260
+    w, x = O.ggml_random_rows(int(t), N, K, rng), one_term_rows(M, K, magnitude, rng)
+    y, (exact, _) = ggml_dense(backend, t, x, w), O.ggml_dense_f64(x, w, int(t), None)
+    assert np.all(np.abs(y.astype(np.float64) - exact) <= ONE_PRODUCT * np.abs(exact) + 2.0 ** -147)
+
+
+@pytest.mark.parametrize("transposed", [True, False])
+@pytest.mark.parametrize("mx,mw", [(1.0, 1.0), (1e-37, 1.0), (1.0, 1e-37)])
+def test_every_part_of_every_dot_general_product(backend, transposed, mx, mw):
+    M, K, N = 1037, 1028, 1036
+    rng = np.random.default_rng(3)
+    x, w = one_term_rows(M, K, mx, rng), (rng.standard_normal((K, N)) * mw).astype(np.float32)
+    y, want = dot_general(backend, x, w, transposed).astype(np.float64), x.astype(np.float64) @ w.astype(np.float64)
+    assert np.all(np.abs(y - want) <= ONE_PRODUCT * np.abs(want) + 2.0 ** -147)
 
 
 @pytest.mark.parametrize("B", [128, 32])
@@ -231,18 +311,6 @@ def test_few_rows(backend, M, K, N, axis, B, zp):
     y = r.run().astype(np.float64)
     truth, scale = O.qdense_f64(p), O.qdense_f64(p, absolute=True)
     assert np.all(np.abs(y - truth) <= 2.0 ** -22 * np.abs(truth) + 3e-6 * scale)
-
-
-def dot_general(backend, x, w, transposed):
-    """x [M, K] . w [K, N] through DotGeneral, w passed as it is or transposed."""
-    bld = backend.Builder("dot")
-    f = bld.Main()
-    vals = [x, w.T if transposed else w]
-    shapes = [ca.Shape(ca.Float32, *v.shape) for v in vals]
-    a, b = (f.Parameter(n, s) for n, s in zip("ab", shapes))
-    f.Return([f.DotGeneral(a, [1], [], b, [1 if transposed else 0], [])])
-    bufs = [backend.BufferFromFlatData(0, np.ascontiguousarray(v).ravel(), s) for v, s in zip(vals, shapes)]
-    return bld.Compile().Execute(bufs)[0].ToFlatData().reshape(x.shape[0], w.shape[1])
 
 
 @pytest.mark.parametrize("transposed", [True, False])
