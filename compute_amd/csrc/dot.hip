@@ -615,7 +615,7 @@ static int dot_split_run(mx_backend* b, const DotDesc& d) {
   a.N = (int)d.N;
   a.act = MX_ACT_NONE;
   int nw = 0, grid = 0;
-  MX_TRY(sg::plan(b, a, d.M, 6, &nw, &grid));
+  MX_TRY(sg::plan(b, a, d.M, 6, false, &nw, &grid));
   return launch(b, "dot_mfma_f32", [&] {
     if (d.rhs_transposed)
       dispatch(sg::split_gemm_kernel<DotSource<true>, 8>, grid, 512, 0, b->stream, a);

@@ -684,7 +684,7 @@ int ggml_dense_run(mx_backend* b, const GgmlDesc& d) {
       a.act = d.act;
       a.bpr = d.bpr;
       int nw = 0, grid = 0;
-      MX_TRY(sg::plan(b, a, d.M, 6, &nw, &grid));
+      MX_TRY(sg::plan(b, a, d.M, 6, false, &nw, &grid));
       return launch(b, "ggml_dequant_f32_mfma", [&] {
         auto go = [&](auto type) { dispatch(sg::split_gemm_kernel<GgmlSource<decltype(type)::value, 8>, 8>, grid, 512, 0, st, a); };
         switch (d.type) {

@@ -164,7 +164,7 @@ template <int WDT, int FORM, int SM, int KIND, bool XBF>
 int rg_launch(mx_backend* b, const char* name, Args& a) {
   using S8 = RgSource<WDT, FORM, SM, KIND, XBF, 8>;
   int nw = 0, grid = 0;
-  MX_TRY(plan(b, a, a.M, S8::kPA + S8::kPB, &nw, &grid));
+  MX_TRY(plan(b, a, a.M, S8::kPA + S8::kPB, XBF, &nw, &grid));
   return launch(b, name, [&] {
     if constexpr (S8::kPA + S8::kPB <= 4) {
       if (nw == 4) {

@@ -540,15 +540,19 @@ __global__ __launch_bounds__(64 * NW, 2) void split_gemm_kernel(Args a) {
 //   [4096,11008] with 86 tiles in two slices 77 us with four waves, 68 us with eight.
 //   Past that, forms whose operands have at most four parts in all run two workgroups of four waves
 //   per CU (64 KB of LDS each; [2048,4096] x [4096,11008] 603 us, 793 us with eight waves), the
-//   others one of eight waves (96 KB).  Tiles past the last whole round of resident workgroups are
-//   sliced if the slices fit one round: 258 tiles of GGML Q6_K rows (x [333,4096], N = 11008) took
-//   357 us in two rounds, 214 us with the last two tiles in 16 slices each.
-inline int plan(mx_backend* b, Args& a, int64_t M, int parts, int* nw, int* grid) {
+//   others one of eight waves (96 KB).  Up to 64 rows of f32 x have eight waves too: the GEMV, which
+//   would take them else, is 1.4e-7 to 3.2e-7 off 64 bits, four waves' single chain of sums 6.4e-7,
+//   eight waves 0.7e-7 to 1.2e-7 ([48,4096] x Int4 [4096,32768] 124 us with four waves, 125 with
+//   eight; x [4096,128256] 377 and 535; the GEMV 1005 at 32 rows there).
+//   Tiles past the last whole round of resident workgroups are sliced if the slices fit one round:
+//   258 tiles of GGML Q6_K rows (x [333,4096], N = 11008) took 357 us in two rounds, 214 us with the
+//   last two tiles in 16 slices each.
+inline int plan(mx_backend* b, Args& a, int64_t M, int parts, bool xbf, int* nw, int* grid) {
   const int64_t tiles_n = (a.N + kBN - 1) / kBN, tiles = ((M + kBM - 1) / kBM) * tiles_n;
   if (tiles >= (int64_t)1 << 28) return set_error(MX_ERR_INVALID, "FusedQuantizedDense: M=%lld too large", (long long)M);
   const int blocks = (a.K + kBK - 1) / kBK;
-  *nw = parts > 4 || tiles < 256 ? 8 : 4;
-  const int64_t round = tiles < 256 || *nw == 8 ? 256 : 512;
+  *nw = parts > 4 || tiles < 256 || (M <= 64 && !xbf) ? 8 : 4;
+  const int64_t round = *nw == 8 ? 256 : 512;
   a.whole = (int)(tiles / round * round);
   const int64_t tail = tiles - a.whole;
   int64_t S = 1;

@@ -349,3 +349,18 @@ def test_dot_general_f32_overflow(backend, transposed):
     truth = x.astype(np.float64) @ w.astype(np.float64)
     rest = np.r_[0, 3:M]
     assert np.all(np.abs(y[rest] - truth[rest]) <= (2.0 ** -22 + 3e-6) * truth[rest])
+
+
+@pytest.mark.parametrize("axis,B", [(1, 128), (0, None)])
+def test_few_rows_of_a_wide_head(backend, axis, B):
+    """256 tiles of 33 rows (a vocabulary head): as close to 64 bits as the GEMV was (1.4e-7 to 3.2e-7
+    of the result's norm), which one chain of sums over K is not."""
+    M, K, N = 33, 4096, 32768
+    p = O.make_problem(M, K, N, w_dtype=O.DT_INT8, x_dtype=F32, scale_dtype=F32, block_axis=axis, block_size=K if B is None else B,
+                       bias=False, seed=1)
+    r = QDenseRun(backend, p)
+    assert r.plan() == "qdense_refgemm_f32_mfma"
+    rows = np.array([0, 32])
+    y, truth = r.run()[rows].astype(np.float64), O.qdense_f64(p, rows)
+    err = np.linalg.norm(y - truth) / np.linalg.norm(truth)
+    assert err <= 1.6e-7, err
