@@ -25,11 +25,14 @@ namespace {
 using namespace sg;
 
 enum RgForm { kRow, kColumn, kWeight };
-// Where the weight form finds the scales (and zero points) of 4 consecutive columns of row k.
+// Where the weight form finds the scales (and zero points) of 4 consecutive columns of 4 rows.
+// kRgCols holds one scale row where the others hold four: x [2048,4096] x [4096,4096], groups of 128 with
+// zero points 546 -> 386 us (f32 x) and 348 -> 218 (bf16 x, whose four-wave kernel spilled with four).
 enum RgScales {
-  kRgCols = 0,  // one per column of a scale row: [ceil(K/B), N]
-  kRgBlk = 1,   // [K, ceil(N/B)] with B % 4 == 0: one
-  kRgAny = 2    // [K, ceil(N/B)], any B: one per column
+  kRgCols = 0,  // [ceil(K/B), N], B % 4 == 0: one per column
+  kRgBlk = 1,   // [K, ceil(N/B)], B % 4 == 0: one per row
+  kRgAny = 2,   // [K, ceil(N/B)], any other B: one each
+  kRgRows = 3   // [ceil(K/B), N], any other B: one each
 };
 
 // What the weight factor holds beside the code times the scale.
@@ -49,12 +52,14 @@ struct RgSource {
   static constexpr bool kI4 = WDT == MX_DTYPE_INT4 || WDT == MX_DTYPE_UINT4;
   static constexpr bool kSigned = WDT == MX_DTYPE_INT4 || WDT == MX_DTYPE_INT8;
   static constexpr int CT = 16 / NW;
-  static constexpr int kScales = FORM != kWeight ? 1 : SM == kRgBlk ? 1 : CT;  // per row
+  static constexpr int kScales = FORM != kWeight ? 1 : SM == kRgBlk ? 1 : CT;  // per scale row
+  static constexpr int kSRows = SM == kRgCols ? 1 : 4;                         // scale rows of 4 rows
+  static constexpr bool kAlongK = SM == kRgCols || SM == kRgRows;
 
   struct Regs {
     uint32_t w[4];
-    uint32_t s[4][kScales], z[4][kScales];  // raw words (kRgCols with bf16: pairs)
-    uint32_t ssh[4][kScales], zsh[4][kScales];
+    uint32_t s[kSRows][kScales], z[kSRows][kScales];  // raw words (kRgCols with bf16: pairs)
+    uint32_t ssh[kSRows][kScales], zsh[kSRows][kScales];
   };
   int cq, c0, j, ncl;
   uint32_t woff[4];  // from a block's first row
@@ -70,6 +75,11 @@ struct RgSource {
 #pragma unroll
     for (int e = 0; e < 4; ++e) woff[e] = ((uint32_t)(4 * j + e) * (uint32_t)a.N + (uint32_t)ncl) / (kI4 ? 2 : 1);
   }
+  // k / kB: the quotient's error, at most k 2^-23, is below the half that keeps it off the integers (K
+  // is at most 2^22).
+  static __device__ __forceinline__ int scale_row(const Args& a, int k) {
+    return (int)(((float)k + 0.5f) * (1.0f / (float)a.kB));
+  }
   // CT consecutive elements from i on: f32 CT words; bf16 CT / 2 words, repeated (one form for both).
   static __device__ __forceinline__ void words(const void* p, int64_t i, bool bf, uint32_t (&w)[kScales]) {
     const uint32_t* q = (const uint32_t*)((const char*)p + i * (bf ? 2 : 4));
@@ -78,9 +88,17 @@ struct RgSource {
   }
   __device__ __forceinline__ void load(const Args& a, Block b, Regs& R) const {
     const char* base = (const char*)a.w + (int64_t)b.k * (kI4 ? a.N / 2 : a.N);
+    const bool sbf = a.s_dt == MX_DTYPE_BFLOAT16, zbf = a.zp_dt == MX_DTYPE_BFLOAT16;
+    if constexpr (FORM == kWeight && kAlongK) {
+#pragma unroll
+      for (int r = 0; r < kSRows; ++r) {
+        const int64_t i = (int64_t)scale_row(a, b.k + 4 * j + r) * a.N + ncl;
+        words(a.scale, i, sbf, R.s[r]);
+        if constexpr (kZp) words(a.zp, i, zbf, R.z[r]);
+      }
+    }
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
-      const int k = b.k + 4 * j + e;
       const char* p = base + woff[e];
       if constexpr (kI4 && CT == 2)
         R.w[e] = *(const uint8_t*)p;
@@ -88,19 +106,13 @@ struct RgSource {
         R.w[e] = *(const uint16_t*)p;
       else
         R.w[e] = *(const uint32_t*)p;
-      if constexpr (FORM == kWeight) {
-        const bool sbf = a.s_dt == MX_DTYPE_BFLOAT16, zbf = a.zp_dt == MX_DTYPE_BFLOAT16;
-        if constexpr (SM == kRgCols) {
-          const int64_t i = (int64_t)(k / a.B) * a.N + ncl;
-          words(a.scale, i, sbf, R.s[e]);
-          if constexpr (kZp) words(a.zp, i, zbf, R.z[e]);
-        } else {
+      if constexpr (FORM == kWeight && !kAlongK) {
+        const int k = b.k + 4 * j + e;
 #pragma unroll
-          for (int c = 0; c < kScales; ++c) {
-            const int64_t i = (int64_t)k * a.nb + (ncl + c) / a.B;
-            word(a.scale, i, sbf, R.s[e][c], R.ssh[e][c]);
-            if constexpr (kZp) word(a.zp, i, zbf, R.z[e][c], R.zsh[e][c]);
-          }
+        for (int c = 0; c < kScales; ++c) {
+          const int64_t i = (int64_t)k * a.nb + (ncl + c) / a.B;
+          word(a.scale, i, sbf, R.s[e][c], R.ssh[e][c]);
+          if constexpr (kZp) word(a.zp, i, zbf, R.z[e][c], R.zsh[e][c]);
         }
       }
     }
@@ -112,7 +124,7 @@ struct RgSource {
       return kSigned ? (int)(int8_t)(w >> (8 * c)) : (int)(uint8_t)(w >> (8 * c));
   }
   static __device__ __forceinline__ float scale_of(const uint32_t (&s)[kScales], const uint32_t (&sh)[kScales], int c, bool bf) {
-    if constexpr (SM == kRgCols)
+    if constexpr (kAlongK)
       return __uint_as_float(bf ? (c & 1 ? s[c % kScales] & 0xFFFF0000u : s[c % kScales] << 16) : s[c % kScales]);
     else
       return word_f32(s[c % kScales], sh[c % kScales], bf);
@@ -129,8 +141,9 @@ struct RgSource {
         const int q = code(R.w[e], c);
         if constexpr (FORM == kWeight) {
           const float wf = KIND == kNf4 ? table[(uint32_t)q & 15u] : (float)q;
-          v[e] = mul_rn(wf, scale_of(R.s[e], R.ssh[e], c, sbf) * kLift);
-          if constexpr (kZp) v[e] = add_rn(v[e], scale_of(R.z[e], R.zsh[e], c, zbf) * kLift);
+          const int r = e % kSRows;
+          v[e] = mul_rn(wf, scale_of(R.s[r], R.ssh[r], c, sbf) * kLift);
+          if constexpr (kZp) v[e] = add_rn(v[e], scale_of(R.z[r], R.zsh[r], c, zbf) * kLift);
           if (TailT::value && 4 * j < b.skip) v[e] = 0.0f;  // x is zero there, but 0 * inf is not
         } else {
           v[e] = (float)q;
@@ -154,7 +167,7 @@ struct RgSource {
   __device__ __forceinline__ float value(const Args& a, int k, int n, const float* table) const {
     const int q = decode_weight(a.w, (int64_t)k * a.N + n, WDT);
     const float wf = KIND == kNf4 ? table[(uint32_t)q & 15u] : (float)q;
-    const int64_t i = SM == kRgCols ? (int64_t)(k / a.B) * a.N + n : (int64_t)k * a.nb + n / a.B;
+    const int64_t i = (int64_t)(k / a.kB) * a.nb + n / a.B;
     const float ws = mul_rn(wf, elem(a.scale, i, a.s_dt));
     return kZp ? add_rn(ws, elem(a.zp, i, a.zp_dt)) : ws;
   }
@@ -189,6 +202,7 @@ int rg_forms(mx_backend* b, const char* name, const QDenseDesc& d, Args& a) {
 
 template <int WDT, int KIND, bool XBF>
 int rg_scales(mx_backend* b, const char* name, const QDenseDesc& d, Args& a) {
+  if (d.block_axis == 0 && a.kB % 4 != 0) return rg_forms<WDT, kRgRows, KIND, XBF>(b, name, d, a);
   if (d.block_axis == 0) return rg_forms<WDT, kRgCols, KIND, XBF>(b, name, d, a);
   if (a.B % 4 == 0 || a.nb == 1) return rg_forms<WDT, kRgBlk, KIND, XBF>(b, name, d, a);
   return rg_forms<WDT, kRgAny, KIND, XBF>(b, name, d, a);
@@ -235,7 +249,8 @@ int qdense_refgemm_run(mx_backend* b, const QDenseDesc& d, const char* name) {
   a.zp_dt = d.zp ? d.zp_dt : MX_DTYPE_FLOAT32;
   a.b_dt = d.b_dt;
   a.act = d.act;
-  a.B = (int)std::min<int64_t>(d.block_size, d.block_axis == 0 ? d.K : d.N);
+  a.B = d.block_axis == 0 ? 1 : (int)std::min<int64_t>(d.block_size, d.N);
+  a.kB = d.block_axis == 0 ? (int)std::min<int64_t>(d.block_size, d.K) : 1;
   a.nb = (int)((d.N + a.B - 1) / a.B);
   const bool xbf = d.x_dt == MX_DTYPE_BFLOAT16;
   auto go = [&](auto wdt) {

@@ -71,8 +71,8 @@ struct Args {
   void* out;          // [M, N], x's dtype
   int M, K, N;
   int s_dt, zp_dt, b_dt, act;
-  int B;              // block size along the scale's blocked axis
-  int nb;             // scale row length of the reference layout: ceil(N / B)
+  int B, kB;          // columns and rows of weights per scale (1 along the axis that is not blocked)
+  int nb;             // scale row length: ceil(N / B)
   int64_t bpr;        // GGML: bytes per weight row
   // Work items: `whole` whole tiles (a multiple of 8), then `tail` items, the S slices of each of the
   // remaining tiles next to each other.

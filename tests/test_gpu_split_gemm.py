@@ -364,3 +364,18 @@ def test_few_rows_of_a_wide_head(backend, axis, B):
     y, truth = r.run()[rows].astype(np.float64), O.qdense_f64(p, rows)
     err = np.linalg.norm(y - truth) / np.linalg.norm(truth)
     assert err <= 1.6e-7, err
+
+
+@pytest.mark.parametrize("x_dtype,B,zp,nf4", [(F32, 6, True, False), (F32, 7, False, False), (BF16, 1, True, False), (BF16, 37, False, True),
+                                              (F32, 1043, True, False), (F32, 4, True, False)])
+@pytest.mark.parametrize("scale_dtype", [F32, BF16])
+def test_groups_of_any_number_of_rows(backend, x_dtype, B, zp, nf4, scale_dtype):
+    """Scales along K in groups that are no multiple of 4 rows (a scale row looked up for each row of
+    weights) and the smallest that is (one for every four rows)."""
+    p = O.make_problem(300, 1048, 272, w_dtype=O.DT_UINT4 if nf4 else O.DT_INT8, x_dtype=x_dtype, scale_dtype=scale_dtype, block_axis=0,
+                       block_size=B, zp=zp, scheme=O.QUANT_NF4 if nf4 else O.QUANT_LINEAR, bias=True, seed=B)
+    r = QDenseRun(backend, p)
+    assert r.plan() == "qdense_refgemm_f32_mfma"
+    y = r.run()
+    check(p, y)
+    assert np.array_equal(y, r.run())
