@@ -69,11 +69,12 @@ struct RgSource {
     cq = (t >> 1) & 31;
     c0 = NW == 8 ? 2 * ((t >> 6) & 1) : 0;
     j = (t & 1) | (t >> (NW == 8 ? 7 : 6)) << 1;
+    const int jl = min(j, a.K / 4 - 1);  // rows past K (below 32): K's last four
     // N % 16 == 0: the columns are all in range or all past N (then the first are read and the
     // outputs are not stored).
     ncl = n0 + 4 * cq < a.N ? n0 + 4 * cq + c0 : 0;
 #pragma unroll
-    for (int e = 0; e < 4; ++e) woff[e] = ((uint32_t)(4 * j + e) * (uint32_t)a.N + (uint32_t)ncl) / (kI4 ? 2 : 1);
+    for (int e = 0; e < 4; ++e) woff[e] = ((uint32_t)(4 * jl + e) * (uint32_t)a.N + (uint32_t)ncl) / (kI4 ? 2 : 1);
   }
   // k / kB: the quotient's error, at most k 2^-23, is below the half that keeps it off the integers (K
   // is at most 2^22).
@@ -92,7 +93,7 @@ struct RgSource {
     if constexpr (FORM == kWeight && kAlongK) {
 #pragma unroll
       for (int r = 0; r < kSRows; ++r) {
-        const int64_t i = (int64_t)scale_row(a, b.k + 4 * j + r) * a.N + ncl;
+        const int64_t i = (int64_t)scale_row(a, min(b.k + 4 * j + r, a.K - 1)) * a.N + ncl;
         words(a.scale, i, sbf, R.s[r]);
         if constexpr (kZp) words(a.zp, i, zbf, R.z[r]);
       }
@@ -107,7 +108,7 @@ struct RgSource {
       else
         R.w[e] = *(const uint32_t*)p;
       if constexpr (FORM == kWeight && !kAlongK) {
-        const int k = b.k + 4 * j + e;
+        const int k = min(b.k + 4 * j + e, a.K - 1);
 #pragma unroll
         for (int c = 0; c < kScales; ++c) {
           const int64_t i = (int64_t)k * a.nb + (ncl + c) / a.B;
@@ -144,7 +145,7 @@ struct RgSource {
           const int r = e % kSRows;
           v[e] = mul_rn(wf, scale_of(R.s[r], R.ssh[r], c, sbf) * kLift);
           if constexpr (kZp) v[e] = add_rn(v[e], scale_of(R.z[r], R.zsh[r], c, zbf) * kLift);
-          if (TailT::value && 4 * j < b.skip) v[e] = 0.0f;  // x is zero there, but 0 * inf is not
+          if (TailT::value && (4 * j < b.skip || 4 * j >= b.end)) v[e] = 0.0f;  // x is zero there, but 0 * inf is not
         } else {
           v[e] = (float)q;
         }
@@ -223,9 +224,10 @@ bool qdense_refgemm_fits(const QDenseDesc& d) {
   const bool xbf = d.x_dt == MX_DTYPE_BFLOAT16;
   const bool packed = dtype_is_packed(d.w_dt);
   if (!(d.scheme == MX_QUANT_LINEAR || d.scheme == MX_QUANT_NF4)) return false;
-  if (!(d.x_dt == MX_DTYPE_FLOAT32 || xbf) || d.M < 1 || d.K < kBK || d.N < 16 || d.N % 16 != 0) return false;
+  if (!(d.x_dt == MX_DTYPE_FLOAT32 || xbf) || d.M < 1 || d.K < 8 || d.N < 16 || d.N % 16 != 0) return false;
   if (d.K % (xbf ? 8 : 4) != 0 || !aligned(d.x, 16) || !aligned(d.w, packed ? 8 : 16)) return false;
-  // A tile's rows of x and a block's rows of weights are addressed by 32-bit offsets.
+  // A tile's rows of x and a block's rows of weights are addressed by 32-bit offsets; past these limits
+  // the GEMV per four rows or the reference-order kernel runs.
   if (d.M >= (int64_t)1 << 30 || d.K > (int64_t)1 << 22 || d.N > (int64_t)1 << 26) return false;
   if (d.block_axis == 0) {
     // 4 consecutive scales of a row: vector loads.

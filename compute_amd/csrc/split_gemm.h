@@ -27,7 +27,8 @@
 // bf16 (64 bytes, four 16-byte chunks XOR-swizzled by (row >> 1) & 3: every operand read and every
 // staging write covers all banks).  Block kb is multiplied while block kb + 1, in registers, is
 // split into the other LDS buffer and block kb + 2 is requested.  K past the last whole block: that
-// block starts 32 before K's end and the values the block before it holds are zeroed.
+// block starts 32 before K's end and the values the block before it holds are zeroed.  K below 32 (at
+// least 8): one block, whose loads past K read values before it and are zeroed.
 //
 // Column n of the tile lies in LDS row (n & 3) * 32 + (n >> 2): MFMA column set c of wave half wn
 // holds columns 64 wn + 4 cg + c, so a lane ends with four consecutive columns of each of its rows.
@@ -133,11 +134,11 @@ __device__ __forceinline__ float elem(const void* p, int64_t i, int dt) {
 // block, their loads, and their parts into LDS (kTail: zeros past K); P::value: the f32 weight
 // factor of one (k, n), its scale included; P::table_value: the 16 entries of the lookup table.
 // NW: waves of the workgroup, 4 (2 x 2 waves of 64 x 64) or 8 (4 x 2 waves of 32 x 64).
-// A block of K: its first row and how many of its rows the block before it holds (the last block of
-// a K that is no multiple of 32).
+// A block of K: its first row, how many of its rows the block before it holds (the last block of a K
+// that is no multiple of 32), and its rows up to K's end (fewer than 32 where K is).
 struct Block {
-  int k, skip;
-  __device__ __forceinline__ Block(int kb, int K) : k(min(kb * kBK, K - kBK)), skip(kb * kBK - k) {}
+  int k, skip, end;
+  __device__ __forceinline__ Block(int kb, int K) : k(max(0, min(kb * kBK, K - kBK))), skip(kb * kBK - k), end(K - k) {}
 };
 
 template <class P, int NW>
@@ -183,7 +184,7 @@ __global__ __launch_bounds__(64 * NW, 2) void split_gemm_kernel(Args a) {
   const char* xbase = (const char*)a.x + (int64_t)m0 * K * kXe;
   uint32_t xoff[XR];  // from the tile's first row (128 K elements stay below 2^31 bytes, checked by the host)
 #pragma unroll
-  for (int i = 0; i < XR; ++i) xoff[i] = ((uint32_t)min(xr + 64 * i, M - 1 - m0) * (uint32_t)K + 8u * xc) * kXe;
+  for (int i = 0; i < XR; ++i) xoff[i] = ((uint32_t)min(xr + 64 * i, M - 1 - m0) * (uint32_t)K + (uint32_t)min(8 * xc, K - 8)) * kXe;
   struct XRegs {
     u32x4_v v[XR][P::kXbf ? 1 : 2];
   };
@@ -195,10 +196,12 @@ __global__ __launch_bounds__(64 * NW, 2) void split_gemm_kernel(Args a) {
       if constexpr (!P::kXbf) R.v[i][1] = *(const u32x4_v*)(base + xoff[i] + 16);
     }
   };
-  // With kTail, the values that the block before holds are zero (whole runs of 8 bf16 or 4 f32).
+  // With kTail, the values that the block before holds and those past K are zero (whole runs of 8 bf16
+  // or 4 f32; the 4 before K where K is below 32 and no multiple of 8 came second).
   auto stage_x = [&](int slot, Block b, const XRegs& R, char* As, auto tail) __attribute__((always_inline)) {
     constexpr bool kTail = decltype(tail)::value;
-    const bool lo = !kTail || 8 * xc >= b.skip, hi = !kTail || (P::kXbf ? lo : 8 * xc + 4 >= b.skip);
+    const bool lo = !kTail || (8 * xc >= b.skip && 8 * xc < b.end);
+    const bool hi = !kTail || (P::kXbf ? lo : 8 * xc + 4 >= b.skip && 8 * xc + 4 < b.end);
 #pragma unroll
     for (int i = 0; i < XR; ++i) {
       char* dst = As + chunk_at(xr + 64 * i, xc);
@@ -214,6 +217,9 @@ __global__ __launch_bounds__(64 * NW, 2) void split_gemm_kernel(Args a) {
             v[e] = __uint_as_float(e & 1 ? R.v[i][0][e >> 1] & 0xFFFF0000u : R.v[i][0][e >> 1] << 16);
           else
             v[e] = __uint_as_float(R.v[i][e >> 2][e & 3]);
+          if constexpr (kTail && !P::kXbf) {
+            if (e < 4 && 8 * xc + 4 == b.end) v[e] = __uint_as_float(R.v[i][1][e & 3]);
+          }
           if constexpr (kTail) v[e] = (e < 4 ? lo : hi) ? v[e] : 0.0f;
         }
         if constexpr (P::kRow) {
@@ -243,10 +249,10 @@ __global__ __launch_bounds__(64 * NW, 2) void split_gemm_kernel(Args a) {
   // same words), into their slot two blocks ahead of their use.
   uint32_t rs = 0, rssh = 0;
   const bool sbf = a.s_dt == MX_DTYPE_BFLOAT16;
-  const int scol = P::kRow ? n0 / a.B : 0;
+  const int scol = P::kRow ? n0 / a.B : 0, srow = min(t & 31, K - 1);
   auto load_row_scale = [&](Block b) __attribute__((always_inline)) {
     if constexpr (P::kRow) {
-      const int64_t i = (int64_t)(b.k + (t & 31)) * a.nb + scol;
+      const int64_t i = (int64_t)(b.k + srow) * a.nb + scol;
       word(a.scale, i, sbf, rs, rssh);
     }
   };

@@ -366,6 +366,24 @@ def test_few_rows_of_a_wide_head(backend, axis, B):
     assert err <= 1.6e-7, err
 
 
+@pytest.mark.parametrize("form,K", [(f, K) for f in FORMS for K in (8, 12, 24, 28) if f[0] == F32 or K % 8 == 0])
+@pytest.mark.parametrize("w_dtype", [O.DT_INT8, O.DT_UINT4])
+def test_fewer_rows_of_weights_than_a_block(backend, form, K, w_dtype):
+    """K below one block of 32 (a low-rank factor), with f32 x also where 4 values of a run of 8 remain
+    (bf16 rows of K % 8 != 0 take the reference-order kernel)."""
+    x_dtype, axis, B, zp, nf4 = form
+    M, N = 2061, 1040
+    p = O.make_problem(M, K, N, w_dtype=w_dtype, x_dtype=x_dtype, scale_dtype=x_dtype, block_axis=axis,
+                       block_size=K if B is None else B, zp=zp, scheme=O.QUANT_NF4 if nf4 else O.QUANT_LINEAR, bias=True, seed=K)
+    r = QDenseRun(backend, p)
+    assert r.plan() == "qdense_refgemm_f32_mfma"
+    y = r.run()
+    check(p, y)
+    if x_dtype == F32 and not zp:
+        truth, scale = O.qdense_f64(p), O.qdense_f64(p, absolute=True)
+        assert np.all(np.abs(y - truth) <= 2.0 ** -20 * scale)
+
+
 @pytest.mark.parametrize("x_dtype,B,zp,nf4", [(F32, 6, True, False), (F32, 7, False, False), (BF16, 1, True, False), (BF16, 37, False, True),
                                               (F32, 1043, True, False), (F32, 4, True, False)])
 @pytest.mark.parametrize("scale_dtype", [F32, BF16])
