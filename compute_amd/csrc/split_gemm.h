@@ -388,19 +388,28 @@ __global__ __launch_bounds__(64 * NW, 2) void split_gemm_kernel(Args a) {
     }
   }
   auto finite = [](float v) { return fabsf(v) < __builtin_inff(); };
-  uint64_t redo = 0;  // the wave's rows that hold such sums
+  float probe = 0.0f;  // NaN after a sum that is not finite
 #pragma unroll
   for (int rb = 0; rb < RB; ++rb)
 #pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      bool bad = false;
+    for (int c = 0; c < 4; ++c)
 #pragma unroll
-      for (int c = 0; c < 4; ++c) bad |= !finite(acc[rb][c][r]);
-      const uint64_t lanes = __ballot(bad);
+      for (int r = 0; r < 4; ++r) probe = __builtin_fmaf(acc[rb][c][r], 0.0f, probe);
+  uint64_t redo = 0;  // the wave's rows that hold such sums
+  if (__any(probe != 0.0f)) {
 #pragma unroll
-      for (int q = 0; q < 4; ++q)
-        if (lanes >> (16 * q) & 0xFFFFu) redo |= (uint64_t)1 << (16 * rb + 4 * q + r);
-    }
+    for (int rb = 0; rb < RB; ++rb)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        bool bad = false;
+#pragma unroll
+        for (int c = 0; c < 4; ++c) bad |= !finite(acc[rb][c][r]);
+        const uint64_t lanes = __ballot(bad);
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+          if (lanes >> (16 * q) & 0xFFFFu) redo |= (uint64_t)1 << (16 * rb + 4 * q + r);
+      }
+  }
   // Row by row, a column per lane (0.7 ms a row of a tile at K = 4096, bound by the latency of the loads).
   const int kbeg = kb0 * kBK, kend = min(K, kb1 * kBK);
   for (; redo; redo &= redo - 1) {
