@@ -509,13 +509,15 @@ struct GgmlSource {
     const int s = (b.k % vpb) >> 5;
     float d, m = 0.0f;
     if constexpr (T == MX_GGML_Q4_K) {
-      // Scale and minimum s of the 12 packed bytes h[1..3] (scale_min_k4 on registers).
-      const int at = 8 * (s & 3);
-      const uint32_t s0 = R.h[1] >> at & 255u, s1 = R.h[2] >> at & 255u, s2 = R.h[3] >> at & 255u;
-      const uint32_t sc = s < 4 ? s0 & 63u : (s2 & 15u) | (s0 >> 6) << 4;
-      const uint32_t mn = s < 4 ? s1 & 63u : (s2 >> 4) | (s1 >> 6) << 4;
-      d = mul_rn(f16_to_f32((uint16_t)R.h[0]), (float)sc);
-      m = mul_rn(f16_to_f32((uint16_t)(R.h[0] >> 16)), (float)mn);
+      // Scale and minimum s of the 12 packed bytes h[1..3] (scale_min_k4 on registers, both at once: the
+      // scale in the low half, the minimum in the high one).  s is uniform and masks choose, since
+      // branches would keep the conversions from running under the MFMAs.
+      const uint32_t j = s & 3, low = s < 4 ? 0x003F003Fu : 0u, high = 0x003F003Fu - low;
+      const uint32_t both = __builtin_amdgcn_perm(R.h[2], R.h[1], 0x0C040C00u + 0x00010001u * j);  // bytes j of h[1], h[2]
+      const uint32_t nib = __builtin_amdgcn_ubfe(R.h[3], 8 * j, 8);
+      const uint32_t sm = (both & low) | ((((nib | nib << 12) & 0x000F000Fu) | (both >> 2 & 0x00300030u)) & high);
+      d = mul_rn(f16_to_f32((uint16_t)R.h[0]), (float)(sm & 255u));
+      m = mul_rn(f16_to_f32((uint16_t)(R.h[0] >> 16)), (float)(sm >> 16));
     } else if constexpr (T == MX_GGML_Q6_K) {
       d = mul_rn(f16_to_f32((uint16_t)R.d), (float)((int32_t)R.d >> 24));
     } else {
