@@ -40,6 +40,9 @@
 // left as they are.
 #pragma once
 
+#include <algorithm>
+#include <cmath>
+
 #include "device_common.h"
 #include "mxrt_internal.h"
 
@@ -550,9 +553,13 @@ __global__ __launch_bounds__(64 * NW, 2) void split_gemm_kernel(Args a) {
 
 // Waves per workgroup, tail slices and grid of a problem (planned for 256 CUs whatever the device
 // reports, so the summation order depends on the shape alone).
-//   Below 256 tiles every tile is sliced along K, as many slices of at least eight blocks as fill
-//   the CUs.  One workgroup per CU then has eight waves, two per SIMD: x f32 [100,4096] x Int4
-//   [4096,11008] with 86 tiles in two slices 77 us with four waves, 68 us with eight.
+//   Below 256 tiles every tile is sliced along K, as many slices as fill the CUs at most.  A slice adds
+//   0.6 us to the tile's sum at its end and a block takes 1.1 us with six products per term and 0.8
+//   with three, so S = sqrt(1.8 or 1.3 blocks) is best: Q4_K rows, x [128,512] x 512 14.6 us in four
+//   slices (19.2 in two, 14.1 in eight), [128,1024] x 1024 17.1 in eight (20.2 in four, 19.8 in 16),
+//   [128,4096] x 1024 27.0 in 16 (29.8 in 26); DotGeneral [96,115004] x 100 101 us in 80 (155 in 255).
+//   One workgroup per CU then has eight waves, two per SIMD: x f32 [100,4096] x Int4 [4096,11008] with
+//   86 tiles in two slices 77 us with four waves, 68 us with eight.
 //   Past that, forms whose operands have at most four parts in all run two workgroups of four waves
 //   per CU (64 KB of LDS each; [2048,4096] x [4096,11008] 603 us, 793 us with eight waves), the
 //   others one of eight waves (96 KB).  Up to 64 rows of f32 x have eight waves too: the GEMV, which
@@ -572,7 +579,8 @@ inline int plan(mx_backend* b, Args& a, int64_t M, int parts, bool xbf, int* nw,
   const int64_t tail = tiles - a.whole;
   int64_t S = 1;
   if (tail > 0) {
-    S = std::max<int64_t>(1, std::min<int64_t>((a.whole ? round : kMaxParts) / tail, blocks / 8));
+    const int64_t best = std::max<int64_t>(1, (int64_t)(sqrtf((parts > 4 ? 1.8f : 1.3f) * (float)blocks) + 0.5f));
+    S = std::max<int64_t>(1, std::min<int64_t>((a.whole ? round : kMaxParts) / tail, best));
     if (a.whole && b->noalloc_active && tail * S > kMaxParts) S = std::max<int64_t>(1, kMaxParts / tail);
   }
   a.kpb = (int)((blocks + S - 1) / S);
