@@ -447,7 +447,7 @@ __global__ __launch_bounds__(kChainThreads) void qdense_exact_chain_kernel(QDens
       *(f32x4_t*)(out + r) = f32x4_t{t[0], t[1], t[2], t[3]};
     }
   };
-  const int chunks = (K + kChainK - 1) / kChainK;
+  const int chunks = (int)(((int64_t)K + kChainK - 1) / kChainK);  // K is below 2^31
   const bool adds = wave == kChainWaves;
   float acc = adds && d.bias ? load_f(d.bias, nn, d.b_dt) : 0.0f;
   const int kw = kChainRows * min(wave, kChainWaves - 1);
