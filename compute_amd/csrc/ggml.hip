@@ -17,9 +17,9 @@
 //                      LDS as [m][32-value unit][36] (padded so that the 16 lanes of a 16-byte
 //                      read hit distinct banks).  Each lane takes 32-value units: their integer
 //                      codes times x are summed in f32 and the unit's scale (and min) applied
-//                      once, then the wave adds its lanes in a fixed tree.  f32 FMAs on the VALU:
-//                      x is f32 by contract, and bf16 matrix-core operands would not keep the
-//                      f32 accumulation bound.
+//                      once, then the wave adds its lanes in a fixed tree.  f32 FMAs on the VALU
+//                      (x is f32 by contract; its three bf16 parts on the matrix cores would keep
+//                      the bound too, as they do past 16 rows; not built for these).
 //   split_gemm<GgmlSource> — past 16 rows: each K block of rows dequantised as the reference forms
 //                      each value and contracted in exact bf16 parts (split_gemm.h), bias and
 //                      activation in its epilogue.

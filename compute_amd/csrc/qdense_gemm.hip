@@ -13,18 +13,21 @@
 // zero, so nothing is cleared.
 //
 // Tiling.  A workgroup (8 waves, two per SIMD) computes a 256 x 128 output tile (or, RB = 2, 128 x
-// 128 with 32 rows per wave: gemm_plan); wave w owns rows [64 wr, 64 wr + 64) x columns [64 wc, 64 wc + 64) with wr = w % 4, wc = w / 4.  K advances
-// in blocks of 64 (two 32-row steps of v_mfma_f32_16x16x32_bf16).  LDS holds
-//   - x, four buffers (three with f32 group scales): [256 rows][64 k] bf16; 16-byte k-chunks XOR-swizzled within each row by
-//     (row >> 1) & 7 so that an MFMA operand read (16 rows) hits distinct banks;
+// 128 with 32 rows per wave: gemm_plan); wave w owns rows [64 wr, 64 wr + 64) x columns [64 wc,
+// 64 wc + 64) with wr = w % 4, wc = w / 4.  K advances in blocks of 64 (two 32-row steps of
+// v_mfma_f32_16x16x32_bf16).  LDS holds
+//   - x, four buffers (three with f32 group scales off 16-byte alignment): [256 rows][64 k] bf16;
+//     16-byte k-chunks XOR-swizzled within each row by (row >> 1) & 7 so that an MFMA operand read
+//     (16 rows) hits distinct banks;
 //   - Bt, two buffers: [128 columns][64 k] bf16, the weights converted exactly to bf16 (|w| < 256
 //     has at most 8 significant bits) and transposed.  Column c is stored in row p = c ^ ((c >> 2)
 //     & 1) and its 16-byte k-chunks are XOR-swizzled by (p >> 3) & 7: the 16 lanes of a B-operand
 //     read (columns 4 apart) then cover both halves of the banks and 8 distinct chunks in each.
 // x moves straight from memory into its LDS buffer (global_load_lds_dwordx4, 1 KB = 8 rows per
 // wave instruction, the swizzle applied by choosing each lane's source chunk) three blocks ahead of
-// its use (two with f32 group scales), and takes no registers, VALU or LDS-write instructions; that leaves room for the
-// grouped kernels' second accumulator set beside a full 256 x 128 tile.  The weights travel
+// its use (two where there are three buffers), and takes no registers, VALU or LDS-write
+// instructions; that leaves room for the grouped kernels' second accumulator set beside a full
+// 256 x 128 tile.  The weights travel
 // through registers (loads of block kb + PF issued during block kb, each thread 4 rows x 4
 // columns: 4 bytes of int8, 2 of 4-bit or 8 of a half type per row; 32 threads per row segment),
 // are converted and written transposed into the Bt buffer of block kb + 1 during block kb.
@@ -60,8 +63,8 @@ template <int RB> constexpr int kBM = 64 * RB;
 template <int RB> constexpr int kABytes = kBM<RB> * kBK * 2;  // 32 or 16 KB per x buffer
 constexpr int kBtBytes = kBN * kBK * 2;  // 16 KB per Bt buffer
 // x buffers: a block's rows are requested kXBufs - 1 blocks ahead of its use.  Four (160 KB of
-// LDS with the two Bt buffers) except for f32 group scales, whose run-time group branch leaves no
-// registers for the longer wait (three: 128 KB).  Q1 360 -> 351 us, Q2 360 -> 346 us, D1 98 -> 95 us
+// LDS with the two Bt buffers) except for f32 group scales off 16-byte alignment, whose run-time
+// group branch leaves no registers for the longer wait (three: 128 KB).  Q1 360 -> 351 us, Q2 360 -> 346 us, D1 98 -> 95 us
 // per call with four; C4 unchanged.
 template <int BK, bool GRP, bool FB>
 constexpr int kXBufs = (GRP && !FB) ? 3 : 4;
@@ -402,8 +405,7 @@ __global__ __launch_bounds__(kThreads) void qdense_gemm_kernel(GemmArgs a) {
       sgw = *(const u32x2_v*)((const uint16_t*)a.scale + (size_t)(2 * g) * N + scol);
       sgw2 = *(const u32x2_v*)((const uint16_t*)a.scale + (size_t)(2 * g + 1) * N + scol);
     } else if constexpr (FB) {
-      // bf16 scales (the host takes these kernels for bf16 scales only): one 8-byte load, kept
-      // as loaded until the fold.
+      // bf16 scales: one 8-byte load, kept as loaded until the fold.
       sgw = *(const u32x2_v*)((const uint16_t*)a.scale + (size_t)g * N + scol);
     } else {
 #pragma unroll
@@ -412,8 +414,8 @@ __global__ __launch_bounds__(kThreads) void qdense_gemm_kernel(GemmArgs a) {
   };
   if constexpr (GRP) load_sg(0);
 
-  // MFMA operands of one 32-row step: x row 64*wr + 16*rb + cg, Bt column 64*wc + 4*cg + c (Bt
-  // row 64*wc + 4*cg + (c ^ (cg & 1))); with groups, Bt column 4*cg + 2*wc + c.
+  // MFMA operands of one 32-row step: x row 16*RB*wr + 16*rb + cg, Bt column 64*wc + 4*cg + c (Bt
+  // row 64*wc + 4*cg + (c ^ (cg & 1))).
   const uint32_t a_row = (uint32_t)((16 * RB * wr + cg) * (kBK * 2));
   const uint32_t b_col = (uint32_t)((64 * wc + 4 * cg) * (kBK * 2));
   const int b_par = cg & 1;

@@ -9,8 +9,10 @@
 // (fusedops/dense.go:176-205):
 //   y[m,n] = act(bias[n] + sum_k x[m,k] * (w'[k,n] * s[k,n/B] + zp[k,n/B]))
 // with w' the integer weight (Linear) or NF4LookupTable[code] (NF4, code = the low 4 bits of the
-// stored element).  The scale varies along K, so it cannot be factored out of the K sum: the
-// products are f32 FMAs on the VALU, with the per-row factor folded into x first,
+// stored element).  The scale varies along K, so it cannot be factored out of the K sum.  The
+// products are f32 FMAs on the VALU (three bf16 parts of x * s on the matrix cores, as split_gemm.h
+// has them for more rows, would also keep the bound; not built here), with the per-row factor folded
+// into x first,
 //   y = sum_k (x[k] * s[k,b]) * w'[k,n] + sum_k x[k] * zp[k,b].
 // Only the summation order and that one rounding differ from the reference loop (results are held
 // to the f32 accumulation bound); small problems keep the reference-order kernel.
