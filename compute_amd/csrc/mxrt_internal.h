@@ -282,7 +282,7 @@ const char* ggml_plan_name(const mx_backend* b, const GgmlDesc& d);
 int ggml_dense_run(mx_backend* b, const GgmlDesc& d);
 int ggml_embed_run(mx_backend* b, const GgmlEmbedDesc& e);
 
-// Prefill of the reference layout, f32 x, zero points and NF4 (qdense_refgemm.hip): the weights
+// Prefill of the reference layout, f32 x, zero points and NF4 (qdense_refgemm.h): the weights
 // dequantised per K block into LDS, f32 operands contracted in exact bf16 parts.
 bool qdense_refgemm_fits(const QDenseDesc& d);
 int qdense_refgemm_run(mx_backend* b, const QDenseDesc& d, const char* name);

@@ -18,8 +18,9 @@
 //                    with on-the-fly dequantisation.
 //   qdense_gemv (qdense_gemv.hip) — up to 16-64 rows of the reference's own layout, f32 x, zero
 //                    points, NF4: HBM-bound decode GEMV.
-//   qdense_refgemm_f32_mfma (qdense_refgemm.hip) — the same variants past the GEMV: f32
+//   qdense_refgemm_f32_mfma (qdense_refgemm.h) — the same variants past the GEMV: f32
 //                    operands in three exact bf16 parts on the bf16 matrix cores (split_gemm.h).
+//                    (A plan name is part of the interface; this one says f32 results by MFMA.)
 //   qdense_exact   — one output column per thread, k in order, each term rounded exactly as the
 //                    reference loop rounds it: bit-identical to the reference's f32 result.
 //                    Used for f32 activations and every shape/layout without a fast path.
@@ -511,7 +512,7 @@ static int exact_rows(const QDenseDesc& d) {
 
 // =============================================================================================
 // Reference layout and variants at prefill size (scale [K, ceil(N/B)] with BlockAxis = 1, f32 x,
-// zero points, NF4): the fused dequantise-and-contract kernel of qdense_refgemm.hip (f32 operands
+// zero points, NF4): the fused dequantise-and-contract kernel of qdense_refgemm.h (f32 operands
 // in exact bf16 parts, the weights dequantised per K block into LDS).  Problems of at most 2^24 multiply-adds
 // keep the exact kernel (the reference's own BenchmarkQuantizedDense shapes, up to
 // 32 x 512 x 1024, stay bit-identical to it).
@@ -528,8 +529,8 @@ static bool qdense_refgemm_plan(const QDenseDesc& d) {
 // against 66 at 64.  Narrower blocks, zero points and NF4 (6 products): int8 with zero
 // points and 64-column blocks 110 against 117 at 20 rows, 138 against 117 at 24, 366 against 117 at
 // 64.  Scales along K: int8 g64 104 against 111 at 24 rows, 138 against 111 at 32, 207 against 111 at
-// 48.  The contraction's error against 64 bits is the smaller one throughout (0.7e-7 to 1.2e-7
-// against 1.4e-7 to 3.2e-7).
+// 48.  The contraction's error against 64 bits is the smaller one (0.7e-7 to 1.2e-7 with eight waves,
+// which f32 x has up to 64 rows, against 1.4e-7 to 3.2e-7).
 static int64_t refgemm_min_rows(const QDenseDesc& d) {
   if (d.block_axis == 0) return 32;
   return d.scheme == MX_QUANT_LINEAR && !d.zp && (d.block_size % 128 == 0 || d.block_size >= d.N) ? 16 : 20;
@@ -540,12 +541,15 @@ static int64_t refgemm_min_rows(const QDenseDesc& d) {
 // =============================================================================================
 enum class QPath { kEmpty, kExact, kSkinny, kSkinnyRows, kGemv, kGemm, kRefGemm };
 
-// Past 16 rows of bf16 x: the skinny kernel once per group of 16 rows (its row limit).  Each
-// launch streams the weights once at decode rate (13-17 us per 16 rows at [4096] x 11008-14336
-// columns), while the GEMM's 256-row tiles are mostly padding at these M and its 128- or
-// 64-column tiles leave most CUs without work: one GEMM launch costs about 51 us there with
-// per-channel scales and 71-102 us with scale groups, so up to 3 (per-channel) or 4 (grouped)
-// skinny launches cost less.
+// Past 16 rows of bf16 x: the skinny kernel once per group of 16 rows (its row limit), up to 3
+// launches (per-channel scales) or 4 (scale groups).  Each launch streams the weights once at decode
+// rate; the GEMM runs one 128-row tile high for all of these rows.  x [17], [32], [33], [48] and
+// [64,4096] x [4096,14336] in row groups, and the GEMM: Int4 g128 21.9, 25.2, 34.4, 37.6, 50.3 us and
+// 29.6; int8 per channel 29.9, 32.7, 46.3, 49.2 (then the GEMM) and 28.7; int8 g128 30.9, 33.7, 47.7,
+// 50.4, 67.2 and 29.5; [4096] x 4096, Int4 g128, 18.2, 20.0, 28.4, 30.1, 40.1 and 18.3.  Up to 32 rows
+// the two are even or the row groups ahead.  From 33 rows the GEMM is, since it has 128-row tiles and K
+// slices: the limits are those of its 256-row tiles (51 us per channel, 71 to 102 with groups), and
+// the plans that callers see at these rows are held to them.
 constexpr int64_t kSkinnyRowsPerLaunch = 16;
 
 static bool skinny_rows_fit(const QDenseDesc& d) {
