@@ -605,9 +605,11 @@ static GPlan ggml_plan(const mx_backend* b, const GgmlDesc& d) {
   g4.M = 4;
   const bool gemv4 = ggml_gemv_kseg(g4) != 0;
   // The weights read once per group of four rows (22 us a group at [4096] x 11008 Q4_K rows), until
-  // the matrix-core contraction, 90 us there for any count up to 128 rows (333 rows: Q6_K 438 -> 214
-  // us, Q4_K 434 -> 204, Q8_0 443 -> 183 against an f32 copy of the weights and f32 MFMAs), costs
-  // less; both scale with the weights, so the crossover holds across shapes.
+  // the matrix-core contraction, 91 to 94 us there for any count up to 128 rows (333 rows: Q6_K 438 ->
+  // 212 us, Q4_K 434 -> 203, Q8_0 443 -> 187 against an f32 copy of the weights and f32 MFMAs), costs
+  // less; both scale with the weights, so the crossover holds across shapes.  Up to about 2^25
+  // multiply-adds the copy was faster ([128,512] x 512 rows 11.0 us, 13.5 here): few tiles, each with
+  // its six-product blocks in sequence.
   if (d.M <= 16 && gemv4) return GPlan::kGemv;
   if (d.M < (int64_t)1 << 30 && d.K <= (int64_t)1 << 22 && d.N < (int64_t)1 << 30 && (uintptr_t)d.w % 2 == 0 && (uintptr_t)d.x % 16 == 0)
     return GPlan::kSplit;

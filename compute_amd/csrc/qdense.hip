@@ -524,13 +524,14 @@ static bool qdense_refgemm_plan(const QDenseDesc& d) {
 }
 
 // Rows past which the contraction, which reads the weights once, is taken where the GEMV would read
-// them for every four rows.  Reference layout, at least 128 columns per scale block (3 products
-// per term): Int4 [4096,11008], f32 x, 79 us (GEMV) against 65 at 16 rows, 94 against 65 at 17, 314
-// against 66 at 64.  Narrower blocks, zero points and NF4 (6 products): int8 with zero
-// points and 64-column blocks 110 against 117 at 20 rows, 138 against 117 at 24, 366 against 117 at
-// 64.  Scales along K: int8 g64 104 against 111 at 24 rows, 138 against 111 at 32, 207 against 111 at
-// 48.  The contraction's error against 64 bits is the smaller one (0.7e-7 to 1.2e-7 with eight waves,
-// which f32 x has up to 64 rows, against 1.4e-7 to 3.2e-7).
+// them for every four rows (x f32, [4096,11008]).  Reference layout, at least 128 columns per scale
+// block (3 products per term): Int4 77 us (GEMV) against 67 at 16 rows, 94 against 67 at 17, 314
+// against 68 at 64.  Narrower blocks, zero points and NF4 (6 products): int8 with zero points and
+// 64-column blocks 113 against 121 at 20 rows, 138 against 121 at 24, 366 against 121 at 64.  Scales
+// along K: int8 g64 102 against 94 at 24 rows, 136 against 94 at 32, 207 against 94 at 48 (111 before
+// four rows of weights shared a scale row; the line is that time's).  The contraction's error against
+// 64 bits is the smaller one (0.7e-7 to 1.6e-7 with eight waves, which f32 x has up to 64 rows,
+// against 1.4e-7 to 3.2e-7).
 static int64_t refgemm_min_rows(const QDenseDesc& d) {
   if (d.block_axis == 0) return 32;
   return d.scheme == MX_QUANT_LINEAR && !d.zp && (d.block_size % 128 == 0 || d.block_size >= d.N) ? 16 : 20;

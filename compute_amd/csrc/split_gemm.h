@@ -13,14 +13,14 @@
 // a value at 1e-36).  x times its row's scale is lifted by 2^24: its bits below 2^-149 count, since a
 // code of up to 8 bits comes after it.  The sums are brought back once.
 //
-// What bounds it: matrix-core and VALU issue together (an MFMA keeps the VALU from about 2.5 of its
-// own issue slots; at four VALU instructions per MFMA, the conversions' share with 3 products, the
-// two run 12 ns per MFMA and SIMD where the MFMA alone takes 8).  Measured, f32 x [2048,4096] x Int4
-// [4096,11008], against an f32-MFMA kernel at 0.63 of the f32 peak: scales per row and 128 columns
-// (3 products) 1868 -> 578 us, 0.96 PFLOP/s of products; per row and 64 columns (6 products) 1868 ->
-// 1060 us; with 100 rows 363 -> 65 us (K in 2 slices).  The error against 64 bits fell from 1.1e-6
-// to 5.8e-7 (four waves) and 1.1e-7 (eight): a step sums 32 terms where the f32 MFMA summed 4, and
-// eight waves keep the sums in three levels.
+// What bounds it: matrix-core and VALU issue together (an MFMA keeps the VALU from about 2.5 of its own
+// issue slots; at four VALU instructions per MFMA, the conversions' share with 3 products, the
+// two run 12 ns per MFMA and SIMD where the MFMA alone takes 8; counters: MFMA busy 42 %, VALU 39 %).
+// Measured, f32 x [2048,4096] x Int4 [4096,11008], against an f32-MFMA kernel at 0.63 of the f32 peak:
+// scales per row and 128 columns (3 products) 1868 -> 560 us, 0.99 PFLOP/s of products; per row and 64
+// columns (6 products) 1868 -> 1069 us; with 100 rows 363 -> 68 us (K in 2 slices).  The error against
+// 64 bits fell from 1.1e-6 to 5.8e-7 (four waves) and 1.1e-7 (eight): a step sums 32 terms where the
+// f32 MFMA summed 4, and eight waves keep the sums in three levels.
 //
 // Tiling: a workgroup of 4 (or 8) waves owns a 128 x 128 output tile, 2 x 2 waves of 64 x 64 (4 x 2
 // of 32 x 64), K in blocks of 32 (one MFMA step).  An operand's part lies in LDS as 128 rows of 32
@@ -561,14 +561,14 @@ __global__ __launch_bounds__(64 * NW, 2) void split_gemm_kernel(Args a) {
 //   One workgroup per CU then has eight waves, two per SIMD: x f32 [100,4096] x Int4 [4096,11008] with
 //   86 tiles in two slices 77 us with four waves, 68 us with eight.
 //   Past that, forms whose operands have at most four parts in all run two workgroups of four waves
-//   per CU (64 KB of LDS each; [2048,4096] x [4096,11008] 603 us, 793 us with eight waves), the
+//   per CU (64 KB of LDS each; [2048,4096] x [4096,11008] 560 us, a third more with eight waves), the
 //   others one of eight waves (96 KB).  Up to 64 rows of f32 x have eight waves too: the GEMV, which
 //   would take them else, is 1.4e-7 to 3.2e-7 off 64 bits, four waves' single chain of sums 6.4e-7,
 //   eight waves 0.7e-7 to 1.2e-7 ([48,4096] x Int4 [4096,32768] 124 us with four waves, 125 with
 //   eight; x [4096,128256] 377 and 535; the GEMV 1005 at 32 rows there).
 //   Tiles past the last whole round of resident workgroups are sliced if the slices fit one round:
-//   258 tiles of GGML Q6_K rows (x [333,4096], N = 11008) took 357 us in two rounds, 214 us with the
-//   last two tiles in 16 slices each.
+//   258 tiles of GGML Q6_K rows (x [333,4096], N = 11008) took 357 us in two rounds, 212 us with the
+//   last two tiles in slices.
 inline int plan(mx_backend* b, Args& a, int64_t M, int parts, bool xbf, int* nw, int* grid) {
   const int64_t tiles_n = (a.N + kBN - 1) / kBN, tiles = ((M + kBM - 1) / kBM) * tiles_n;
   if (tiles >= (int64_t)1 << 28) return set_error(MX_ERR_INVALID, "FusedQuantizedDense: M=%lld too large", (long long)M);
