@@ -1,13 +1,13 @@
 #!/usr/bin/env python3
 """Benchmark of the MI355X backend's FusedQuantizedDense hot path.
 
-Headline workload (the config the metric is quoted on): decode GEMV,
+Headline workload (C2, the one the metric is quoted on): decode GEMV,
 x bf16 [1,4096], Int4 weights [4096,11008] (reference packing), group-128 bf16 scales along K,
 no bias.  A step is one Execute of the compiled graph over one batch, with every input already
 resident in HBM.  Weight sets are rotated (> 512 MB of distinct copies) so each step reads its
 weights from HBM rather than the 256 MB Infinity Cache.
 
-The JSON line also reports, under "extra", the other BASELINE configurations measured the same
+The JSON line also reports, under "extra", the other workloads measured the same
 way: C3 batched decode (HBM roofline), C4 prefill (bf16 MFMA roofline) and C5, the quantized MLP
 graph built through the Builder API (microseconds per Execute, 100 resident calls); G1 / G2,
 the GGML block-format decode GEMV (Q4_0 / Q4_K rows, f32 x [1,4096], 11008 rows; HBM roofline);

@@ -1,4 +1,4 @@
-"""Synthetic workloads of the benchmark: the BASELINE.json configurations of FusedQuantizedDense.
+"""Synthetic workloads of the benchmark: FusedQuantizedDense at decode and prefill, and the quantized MLP.
 
 Each workload builds seeded host data in the storage dtypes the backend takes (bf16 as uint16
 bits, Int4 packed two per byte in the reference packing) and compiles the graph the reference's
@@ -75,7 +75,7 @@ class QDWorkload:
 
 @dataclass
 class MLPWorkload:
-    """the quantized MLP built through the Builder API, batch 8 x seq 1:
+    """C5, the quantized MLP built through the Builder API, batch 8 x seq 1:
     RMSNorm (eps 1e-6, no gamma) over bf16 x [8,4096]; gate and up FusedQuantizedDense Int4 g128
     [4096 -> 14336] (SiLU fused into gate's epilogue); SiLU(gate) * up; down FusedQuantizedDense
     Int4 g128 [14336 -> 4096]; residual add.  RMSNorm runs in f32 (ConvertDType around it)."""
@@ -138,7 +138,7 @@ class MLPWorkload:
 
 @dataclass
 class GGMLWorkload:
-    """FusedQuantizedDense over GGML block rows (not a BASELINE config; the reference's GGML
+    """FusedQuantizedDense over GGML block rows (the reference's GGML
     scheme, quantizeddense_ggml.go): f32 x [M, K], weights [N, bytesPerRow] Uint8 in one of the
     supported block formats."""
 
@@ -311,7 +311,7 @@ def _rngs(seed: int, n: int):
 
 
 def make(name: str, seed: int = 0) -> QDWorkload:
-    """C1 .. C5."""
+    """The workload of a name: C1 .. C5, Q1, Q2, D1, R1 .. R3."""
     rx, rw, rs, rb = _rngs(seed, 4)
     if name == "C1":  # int8 per-channel, x f32 [4,512] U(-1,1), bias f32, no activation
         M, K, N = 4, 512, 512

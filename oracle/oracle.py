@@ -4,7 +4,7 @@ Only tests/, __graft_entry__.smoke() and bench.py's cpu_baseline leg may import 
 and only as the checker (or the timed CPU baseline), never as a product path.
 
 It loads oracle/_build/liboracle.so (a plain-C restatement of the reference's arithmetic,
-qdense_ref.c and ggml_ref.c) and provides numpy helpers: seeded generators for the BASELINE configurations, the
+qdense_ref.c and ggml_ref.c) and provides numpy helpers: seeded generators for the benchmark workloads, the
 reference packing of 4-bit weights, bf16 rounding, and brute-force numpy restatements of the
 DotGeneral output layout (shapeinference/dotgeneral.go:16-152) for small cases.
 """
@@ -222,7 +222,7 @@ def expected_output(p: QDenseProblem, rows=None, threads: int = 1) -> np.ndarray
 
 
 # ---------------------------------------------------------------------------------------------
-# Seeded generators for BASELINE.json configs (and smaller variants of the same form).
+# Seeded generators for the benchmark workloads (and smaller variants of the same form).
 # ---------------------------------------------------------------------------------------------
 def _bf16(rng_vals) -> np.ndarray:
     return bf16_round(np.asarray(rng_vals, dtype=np.float32))
@@ -271,7 +271,7 @@ def make_problem(M, K, N, *, w_dtype=DT_INT8, x_dtype=DT_BFLOAT16, scale_dtype=D
 
 
 def baseline_config(i: int, seed: int = 0) -> QDenseProblem:
-    """BASELINE.json configs[i] as a QDenseProblem (i = 0..3; config 4 is the MLP graph)."""
+    """Benchmark workload C1 .. C4 (i = 0 .. 3) as a QDenseProblem (C5 is the MLP graph)."""
     if i == 0:
         return make_problem(4, 512, 512, w_dtype=DT_INT8, x_dtype=DT_FLOAT32, scale_dtype=DT_FLOAT32, block_axis=0,
                             block_size=512, per_channel_1d=True, bias=True, bias_dtype=DT_FLOAT32,

@@ -52,7 +52,7 @@ def test_gemm_activations(backend, act):
 
 
 def test_gemm_c4_config_full_size(backend):
-    """x bf16 [2048,4096], int8 [4096,4096] per-channel f32 scales, bias,
+    """Workload C4: x bf16 [2048,4096], int8 [4096,4096] per-channel f32 scales, bias,
     exact GELU.  128 seeded rows are checked against the oracle; two calls must agree bitwise."""
     p = O.baseline_config(3)
     r = QDenseRun(backend, p)
@@ -113,7 +113,7 @@ def test_gemm_grouped_activations(backend, act):
 @pytest.mark.parametrize("w_dtype,G", [(O.DT_INT4, 128), (O.DT_INT8, 64), (O.DT_INT4, 32)])
 def test_gemm_grouped_prefill_full_size(backend, w_dtype, G):
     """x bf16 [2048,4096] x Int4 [4096,14336] g128 (the MLP's gate/up weights at prefill) and the
-    int8 g64 layout of BASELINE configs[2] at the same size: 128 seeded rows against the oracle,
+    int8 g64 layout of workload C3 at the same size: 128 seeded rows against the oracle,
     two calls bit-equal."""
     p = O.make_problem(2048, 4096, 14336, w_dtype=w_dtype, block_axis=0, block_size=G, bias=False,
                        scale_range=(0.002, 0.02), seed=G)

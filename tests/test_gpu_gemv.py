@@ -5,7 +5,7 @@ The reference's FusedQuantizedDense takes f32 x and scales in its own layout, sc
 dequantisation.  Small problems keep the reference-order kernel (bit-identical); at decode sizes
 (K*N >= 2^20, M <= 64, four rows per launch) the GEMV kernel runs, whose results differ from the reference loop only by
 summation order and the folding of the scale into x:
-  - f32 outputs: within 1e-5 of sum|terms| of the f64 value (the north star's fp32 bar);
+  - f32 outputs: within 1e-5 of sum|terms| of the f64 value (the fp32 bar);
   - bf16 outputs: within rel 1e-2 / abs 1e-3 of the oracle's f32 result, and the same
     accumulation bound plus half a bf16 ulp.
 """

@@ -1,11 +1,11 @@
-"""The quantized MLP built through the Builder API and executed on the
+"""The quantized MLP (workload C5) built through the Builder API and executed on the
 GPU, checked op by op against the CPU oracle on the GPU's own intermediate values:
   - h = bf16(RMSNorm(x)) computed in f32: within one bf16 ulp of the oracle's restatement of the
     reference graph (sequential f32 ReduceSum, Rsqrt through f64; oracle.rmsnorm_chain, pinned by
     closed forms in test_oracle).  The GPU adds each row's squares in another order (strided
     partial sums and an LDS tree), so the f32 mean square may differ in its last bits;
   - gate = SiLU(FusedQuantizedDense(h)), up and down = FusedQuantizedDense(...): within the
-    north star's rel 1e-2 / abs 1e-3 of the reference loop (the oracle) on the same inputs;
+    rel 1e-2 / abs 1e-3 of the reference loop (the oracle) on the same inputs;
   - gate*up and the residual add: bit-exact bf16 products / sums of the GPU's operands.
 Checked op by op because the composition rounds to bf16 six times: an intermediate that rounds
 to the neighbouring bf16 value (another summation order) carries that ulp on, so an end-to-end

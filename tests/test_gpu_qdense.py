@@ -1,6 +1,6 @@
 """FusedQuantizedDense on the GPU vs the CPU oracle (the reference's arithmetic restated).
 
-Bars (from the task's north star):
+Bars:
   - f32 activations: the exact kernel reproduces the reference loop order, so results must be
     bit-identical to the oracle's f32 result;
   - bf16 activations through the exact kernel: bit-identical to RNE(oracle f32);
@@ -25,7 +25,7 @@ FAST_DECODE = "qdense_skinny_mfma"
 # Exact kernel: bit-exact vs the reference loop.
 # ---------------------------------------------------------------------------------------------
 def test_c1_config_bit_exact(backend):
-    """int8 per-channel, x f32 [4,512], bias, no activation."""
+    """Workload C1: int8 per-channel, x f32 [4,512], bias, no activation."""
     p = O.baseline_config(0)
     r = QDenseRun(backend, p)
     assert r.plan() == "qdense_exact"
@@ -136,7 +136,7 @@ def test_gemv_activations_and_per_channel(backend, act):
 
 
 def test_gemv_c2_config_full_size(backend):
-    """x bf16 [1,4096], Int4 [4096,11008] g128, bf16 scales, no bias."""
+    """Workload C2: x bf16 [1,4096], Int4 [4096,11008] g128, bf16 scales, no bias."""
     p = O.baseline_config(1)
     r = QDenseRun(backend, p)
     assert r.plan().startswith(FAST_DECODE) and r.plan().endswith("_i4")

@@ -83,7 +83,7 @@ def test_skinny_per_channel(backend, w_dtype):
 
 
 def test_skinny_c3_config_full_size(backend):
-    """x bf16 [16,4096], int8 [4096,14336] g64 bf16 scales, bias, SiLU."""
+    """Workload C3: x bf16 [16,4096], int8 [4096,14336] g64 bf16 scales, bias, SiLU."""
     p = O.baseline_config(2)
     r = QDenseRun(backend, p)
     assert r.plan() == "qdense_skinny_mfma_i8"
