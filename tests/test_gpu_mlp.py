@@ -4,7 +4,7 @@ GPU, checked op by op against the CPU oracle on the GPU's own intermediate value
     reference graph (sequential f32 ReduceSum, Rsqrt through f64; oracle.rmsnorm_chain, pinned by
     closed forms in test_oracle).  The GPU adds each row's squares in another order (strided
     partial sums and an LDS tree), so the f32 mean square may differ in its last bits;
-  - gate = SiLU(FusedQuantizedDense(h)), up and down = FusedQuantizedDense(...): within the
+  - gate = SiLU(FusedQuantizedDense(h)), up and down = FusedQuantizedDense(...): within
     rel 1e-2 / abs 1e-3 of the reference loop (the oracle) on the same inputs;
   - gate*up and the residual add: bit-exact bf16 products / sums of the GPU's operands.
 Checked op by op because the composition rounds to bf16 six times: an intermediate that rounds
