@@ -416,7 +416,8 @@ __global__ __launch_bounds__(64 * NW, 2) void split_gemm_kernel(Args a) {
   // Row by row, a column per lane (0.7 ms a row of a tile at K = 4096, bound by the latency of the loads).
   const int kbeg = kb0 * kBK, kend = min(K, kb1 * kBK);
   for (; redo; redo &= redo - 1) {
-    const int i = __builtin_ctzll(redo), m = min(m0 + row0 + i, M - 1);
+    const int i = __builtin_ctzll(redo), m = m0 + row0 + i;
+    if (m >= M) break;  // rows of padding, not stored
     auto xat = [&](int k) { return elem(a.x, (int64_t)m * K + k, P::kXbf ? MX_DTYPE_BFLOAT16 : MX_DTYPE_FLOAT32); };
     bool nan = false;  // a NaN in the row of x: the sums are NaN, as they should be
     for (int k = kbeg; k < kend && !nan; k += 256) {

@@ -397,3 +397,26 @@ def test_groups_of_any_number_of_rows(backend, x_dtype, B, zp, nf4, scale_dtype)
     y = r.run()
     check(p, y)
     assert np.array_equal(y, r.run())
+
+
+@pytest.mark.parametrize("M,B,K", [(260, 64, 1024), (97, 128, 4100), (97, 64, 9000)])
+def test_nan_and_infinite_scales(backend, M, B, K):
+    """Columns with a NaN scale stay NaN and those with an infinite one infinite in every row, beside
+    rows of x with an infinity (the last row of x among them) and sums past f32's range."""
+    p = O.make_problem(M, K, 272, w_dtype=O.DT_UINT8, x_dtype=F32, scale_dtype=F32, block_axis=1, block_size=B, bias=True,
+                       scale_range=(0.001, 0.0039), seed=M + K)
+    w, x, s = np.maximum(p.w, 1), np.abs(p.x) + np.float32(0.1), p.scale.copy()
+    s[K // 2, 1], s[K - 1, 2] = np.nan, np.inf
+    x[M - 1, 5], x[8, K - 1] = np.inf, -np.inf
+    x[9, :] = 3e38
+    p = dataclasses.replace(p, w=w, x=x, scale=s)
+    y = QDenseRun(backend, p).run().astype(np.float64)
+    with np.errstate(invalid="ignore", over="ignore"):
+        truth, scale = O.qdense_f64(p), O.qdense_f64(p, absolute=True)
+        truth = np.where(np.abs(truth) > 3.4028235e38, np.copysign(np.inf, truth), truth)
+    assert np.array_equal(np.isnan(y), np.isnan(truth)) and np.isnan(truth[:, B:2 * B]).all()
+    inf = np.isinf(truth)
+    assert inf[:, 2 * B:].any() and inf[M - 1].any() and inf[8].any() and inf[9].any() and np.array_equal(y[inf], truth[inf])
+    fin = np.isfinite(truth)
+    assert fin.any() and np.all(np.abs(y[fin] - truth[fin]) <= 2.0 ** -22 * np.abs(truth[fin]) + 1e-5 * scale[fin])
+
